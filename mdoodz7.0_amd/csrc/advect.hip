@@ -9,20 +9,50 @@
 // marker. The arithmetic is the reference's, in the same order, built
 // without contraction, so positions and velocities match the CPU
 // restatement bit for bit.
+//
+// Bound: FP64 issue. Each stage divides twelve times by a cell width; those
+// divisions are xdiv_core's product and four fused multiply-adds (the same
+// bits), and one test per stage, over the marker's coordinates and the four
+// products of a velocity, says whether every one of them is in range (the
+// coordinate tables are tested once, on the host); a marker that fails it
+// repeats the stage with divisions. The reference's substitutions for air
+// nodes (tag 30) are left out: mdg_set_bc accepts no such tag on velocity
+// nodes, and reading the tags took 8 more gathers per stage.
+// Measured with 37.7M markers on 2047^2, conservative interpolation:
+// k_advect_rk4 3.26 ms with divisions and tags, 1.63 ms with exact_div tested
+// division by division, 1.48 ms with one test per stage (about 1500 VALU
+// instructions per marker, at the issue rate; 1.66 GB of marker streams would
+// take 0.36 ms).
+#include "exact_div.h"
 #include "mdg_internal.h"
 
 namespace {
 
 struct v2p_grid {
     int Nx, Nz;                       // vertices
-    double dx, dz;
+    exact_div dx, dz;
     const double *xg, *zg, *xvz, *zvx;
-    const signed char *tu, *tv;       // BCu / BCv tags (30: air)
     double xmin, xmax, zmin, zmax;    // box of isoutPart
+    int tables_ok;                    // every coordinate passes v2p_coord_ok
 };
 
-__device__ inline int v2p_cell(double d, double h, int n) {
-    int j = (int)ceil(d / h) - 1;
+// The divisions of a stage: by exact_div's steps, collecting whether any
+// numerator is out of their range, or by the division itself.
+struct div_steps {
+    bool bad;
+    __device__ __forceinline__ double dist(double a, const exact_div &h) const { return xdiv_core(a, h); }
+    __device__ __forceinline__ double prod(double a, const exact_div &h) {
+        bad |= !xdiv_takes(a, h);
+        return xdiv_core(a, h);
+    }
+};
+struct div_plain {
+    __device__ __forceinline__ double dist(double a, const exact_div &h) const { return a / h.b; }
+    __device__ __forceinline__ double prod(double a, const exact_div &h) const { return a / h.b; }
+};
+
+__device__ __forceinline__ int v2p_cell(double q, int n) {
+    int j = (int)ceil(q) - 1;
     if (j < 0) j = 0;
     if (j > n - 2) j = n - 2;
     return j;
@@ -34,84 +64,60 @@ __device__ inline double v2p_corr(double t) {
     return 0.5 * (y * y);
 }
 
+// One velocity component at a marker: F on an n1 x n2 node grid (stride s1
+// along the component's own axis, s2 across it), cell (c1, c2), distances d1,
+// t1 = d1 / h1 along it and t2 across it.  The correction of the second
+// difference reads one node beyond the cell on the side the marker is on.
+template <bool CONSERV, typename D>
+__device__ __forceinline__ double v2p_comp(D &div, const double *__restrict__ F, int at, int s1, int s2, int c1, int n1,
+                                           double d1, double t1, double t2, const exact_div &h1) {
+    const double A0 = F[at], A1 = F[at + s1], B0 = F[at + s2], B1 = F[at + s1 + s2];
+    double a = A0 * (1.0 - t1) + div.prod(A1 * d1, h1);
+    double b = B0 * (1.0 - t1) + div.prod(B1 * d1, h1);
+    if (CONSERV) {
+        const bool up = t1 >= 0.5, on = up ? c1 < n1 - 2 : c1 > 0;
+        const int far = at + (on ? (up ? 2 * s1 : -s1) : 0);
+        const double Af = F[far], Bf = F[far + s2], w = v2p_corr(t1);
+        const double ac = a + w * ((up ? A0 : Af) - 2.0 * (up ? A1 : A0) + (up ? Af : A1));
+        const double bc = b + w * ((up ? B0 : Bf) - 2.0 * (up ? B1 : B0) + (up ? Bf : B1));
+        a = on ? ac : a;
+        b = on ? bc : b;
+    }
+    return (1.0 - t2) * a + t2 * b;
+}
+
 // V2P of one active marker (ParticleRoutines.c:76-252)
-__device__ void v2p_one(const v2p_grid &g, const double *__restrict__ u, const double *__restrict__ v,
-                        int conserv, double x, double z, double *vxm, double *vzm) {
-    const double dx = g.dx, dz = g.dz;
+template <bool CONSERV, typename D>
+__device__ __forceinline__ void v2p_with(D &div, const v2p_grid &g, const double *__restrict__ u,
+                                         const double *__restrict__ v, double x, double z, double *vxm, double *vzm) {
     {
-        const signed char *t = g.tu;
         const int Nx = g.Nx, Nz = g.Nz + 1;
-        const int j = v2p_cell(x - g.xg[0], dx, Nx), i = v2p_cell(z - g.zvx[0], dz, Nz);
+        const int j = v2p_cell(div.dist(x - g.xg[0], g.dx), Nx), i = v2p_cell(div.dist(z - g.zvx[0], g.dz), Nz);
         const double dxm = fabs(x - g.xg[j]), dzm = fabs(z - g.zvx[i]);
-        const int iSW = j + i * Nx, iSE = iSW + 1, iNW = j + (i + 1) * Nx, iNE = iNW + 1;
-        double VNW = u[iNW], VNE = u[iNE], VSW = u[iSW], VSE = u[iSE];
-        const bool aSW = t[iSW] == 30, aSE = t[iSE] == 30, aNW = t[iNW] == 30, aNE = t[iNE] == 30;
-        if (aSW) VSW = u[iNW];
-        if (aSE) VSE = u[iNE];
-        if (aNW) VNW = u[iSW];
-        if (aNE) VNE = u[iSE];
-        if (aNE && aSE) { VNE = VSW; VSE = VSW; }
-        if (aNW && aSW) { VNW = VSE; VSW = VSE; }
-        double v13 = VSW * (1.0 - dxm / dx) + VSE * dxm / dx;
-        double v24 = VNW * (1.0 - dxm / dx) + VNE * dxm / dx;
-        if (conserv == 1) {
-            if (dxm / dx >= 0.5) {
-                if (j < Nx - 2) {
-                    const int iSEE = iSE + 1, iNEE = iNE + 1;
-                    double VSEE = u[iSEE], VNEE = u[iNEE];
-                    if (t[iSEE] == 30) VSEE = u[iSW];
-                    if (t[iNEE] == 30) VNEE = u[iNW];
-                    v13 = v13 + v2p_corr(dxm / dx) * (VSW - 2.0 * VSE + VSEE);
-                    v24 = v24 + v2p_corr(dxm / dx) * (VNW - 2.0 * VNE + VNEE);
-                }
-            } else if (j > 0) {
-                const int iSWW = iSW - 1, iNWW = iNW - 1;
-                double VSWW = u[iSWW], VNWW = u[iNWW];
-                if (t[iSWW] == 30) VSWW = u[iSE];
-                if (t[iNWW] == 30) VNWW = u[iNE];
-                v13 = v13 + v2p_corr(dxm / dx) * (VSWW - 2.0 * VSW + VSE);
-                v24 = v24 + v2p_corr(dxm / dx) * (VNWW - 2.0 * VNW + VNE);
-            }
-        }
-        *vxm = (1.0 - dzm / dz) * v13 + (dzm / dz) * v24;
+        *vxm = v2p_comp<CONSERV>(div, u, j + i * Nx, 1, Nx, j, Nx, dxm, div.dist(dxm, g.dx), div.dist(dzm, g.dz), g.dx);
     }
     {
-        const signed char *t = g.tv;
         const int Nx = g.Nx + 1, Nz = g.Nz;
-        const int j = v2p_cell(x - g.xvz[0], dx, Nx), i = v2p_cell(z - g.zg[0], dz, Nz);
+        const int j = v2p_cell(div.dist(x - g.xvz[0], g.dx), Nx), i = v2p_cell(div.dist(z - g.zg[0], g.dz), Nz);
         const double dxm = fabs(x - g.xvz[j]), dzm = fabs(z - g.zg[i]);
-        const int iSW = j + i * Nx, iSE = iSW + 1, iNW = j + (i + 1) * Nx, iNE = iNW + 1;
-        double VSE = v[iSE], VSW = v[iSW], VNE = v[iNE], VNW = v[iNW];
-        const bool aSW = t[iSW] == 30, aSE = t[iSE] == 30, aNW = t[iNW] == 30, aNE = t[iNE] == 30;
-        // the reference replaces an air SW value by NE (ParticleRoutines.c:207)
-        if (aSW) VSW = v[iNE];
-        if (aSE) VSE = v[iNE];
-        if (aNW) VNW = v[iSW];
-        if (aNE) VNE = v[iSE];
-        if (aNE && aSE) { VNE = VSW; VSE = VSW; }
-        if (aNW && aSW) { VNW = VSE; VSW = VSE; }
-        double v12 = VSW * (1.0 - dzm / dz) + VNW * dzm / dz;
-        double v34 = VSE * (1.0 - dzm / dz) + VNE * dzm / dz;
-        if (conserv == 1) {
-            if (dzm / dz >= 0.5) {
-                if (i < Nz - 2) {
-                    const int iNNW = j + (i + 2) * Nx, iNNE = iNNW + 1;
-                    double VNNW = v[iNNW], VNNE = v[iNNE];
-                    if (t[iNNW] == 30) VNNW = v[iSW];
-                    if (t[iNNE] == 30) VNNE = v[iSE];
-                    v12 = v12 + v2p_corr(dzm / dz) * (VSW - 2.0 * VNW + VNNW);
-                    v34 = v34 + v2p_corr(dzm / dz) * (VSE - 2.0 * VNE + VNNE);
-                }
-            } else if (i > 0) {
-                const int iSSW = j + (i - 1) * Nx, iSSE = iSSW + 1;
-                double VSSW = v[iSSW], VSSE = v[iSSE];
-                if (t[iSSW] == 30) VSSW = v[iNW];
-                if (t[iSSE] == 30) VSSE = v[iNE];
-                v12 = v12 + v2p_corr(dzm / dz) * (VSSW - 2.0 * VSW + VNW);
-                v34 = v34 + v2p_corr(dzm / dz) * (VSSE - 2.0 * VSE + VNE);
-            }
-        }
-        *vzm = (1.0 - dxm / dx) * v12 + (dxm / dx) * v34;
+        *vzm = v2p_comp<CONSERV>(div, v, j + i * Nx, Nx, 1, i, Nz, dzm, div.dist(dzm, g.dz), div.dist(dxm, g.dx), g.dz);
+    }
+}
+
+// A coordinate whose distances to the table's entries are zero or in
+// exact_div's range: zero, or of a size in [2^-400, 2^400).
+__host__ __device__ inline bool v2p_coord_ok(double x) {
+    return (xdiv_hi(x) & 0x7fffffffu) - ((uint32_t)(1023 - 400) << 20) < ((uint32_t)800 << 20) || x == 0.0;
+}
+
+template <bool CONSERV>
+__device__ __forceinline__ void v2p_one(const v2p_grid &g, const double *__restrict__ u, const double *__restrict__ v,
+                                        double x, double z, double *vxm, double *vzm) {
+    div_steps steps{!(v2p_coord_ok(x) && v2p_coord_ok(z)) || !g.tables_ok};
+    v2p_with<CONSERV>(steps, g, u, v, x, z, vxm, vzm);
+    if (__builtin_expect(steps.bad, 0)) {
+        div_plain plain;
+        v2p_with<CONSERV>(plain, g, u, v, x, z, vxm, vzm);
     }
 }
 
@@ -119,49 +125,47 @@ __device__ inline void isout(const v2p_grid &g, double x, double z, int *ph) {
     if (x < g.xmin || x > g.xmax || z < g.zmin || z > g.zmax) *ph = -1;
 }
 
-__global__ void k_v2p(v2p_grid g, const double *__restrict__ u, const double *__restrict__ v, int conserv, int n,
+template <bool CONSERV>
+__global__ void k_v2p(v2p_grid g, const double *__restrict__ u, const double *__restrict__ v, int n,
                       const double *__restrict__ x, const double *__restrict__ z, const int *__restrict__ phase,
                       double *__restrict__ vx, double *__restrict__ vz) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     double a = 0.0, b = 0.0;
-    if (phase[k] != -1) v2p_one(g, u, v, conserv, x[k], z[k], &a, &b);
+    if (phase[k] != -1) v2p_one<CONSERV>(g, u, v, x[k], z[k], &a, &b);
     vx[k] = a;
     vz[k] = b;
 }
 
 // RogerGuntherII's loop body (AdvectionRoutines.c:372-405)
+template <bool CONSERV>
 __global__ void k_advect_rk4(v2p_grid g, const double *__restrict__ u, const double *__restrict__ v, double dt,
-                             int conserv, int n, double *__restrict__ x, double *__restrict__ z,
+                             int n, double *__restrict__ x, double *__restrict__ z,
                              int *__restrict__ phase, double *__restrict__ vxo, double *__restrict__ vzo) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     const double xA = x[k], zA = z[k];
-    double xk = xA, zk = zA;
+    double xk = xA, zk = zA, sx = 0.0, sz = 0.0;
     int ph = phase[k];
-    double VxA = 0.0, VzA = 0.0, VxB = 0.0, VzB = 0.0, VxC = 0.0, VzC = 0.0, VxD = 0.0, VzD = 0.0;
-    if (ph != -1) v2p_one(g, u, v, conserv, xk, zk, &VxA, &VzA);
-    if (ph != -1) {
-        xk = xA + 0.5 * dt * VxA;
-        zk = zA + 0.5 * dt * VzA;
+    // stages A, B, C, D: the sums VxA + 2 VxB + 2 VxC + VxD grow in order
+#pragma unroll 1
+    for (int s = 0; s < 4; s++) {
+        if (ph != -1) {
+            double a, b;
+            v2p_one<CONSERV>(g, u, v, xk, zk, &a, &b);
+            const double w = (s == 1 || s == 2) ? 2.0 : 1.0;
+            sx = (s == 0) ? a : sx + w * a;
+            sz = (s == 0) ? b : sz + w * b;
+            if (s < 3) {
+                const double h = (s == 2) ? 1.0 * dt : 0.5 * dt;
+                xk = xA + h * a;
+                zk = zA + h * b;
+            }
+        }
+        if (s < 3) isout(g, xk, zk, &ph);
     }
-    isout(g, xk, zk, &ph);
-    if (ph != -1) v2p_one(g, u, v, conserv, xk, zk, &VxB, &VzB);
     if (ph != -1) {
-        xk = xA + 0.5 * dt * VxB;
-        zk = zA + 0.5 * dt * VzB;
-    }
-    isout(g, xk, zk, &ph);
-    if (ph != -1) v2p_one(g, u, v, conserv, xk, zk, &VxC, &VzC);
-    if (ph != -1) {
-        xk = xA + 1.0 * dt * VxC;
-        zk = zA + 1.0 * dt * VzC;
-    }
-    isout(g, xk, zk, &ph);
-    if (ph != -1) v2p_one(g, u, v, conserv, xk, zk, &VxD, &VzD);
-    VxA = (1.0 / 6.0) * (VxA + 2.0 * VxB + 2.0 * VxC + VxD);
-    VzA = (1.0 / 6.0) * (VzA + 2.0 * VzB + 2.0 * VzC + VzD);
-    if (ph != -1) {
+        const double VxA = (1.0 / 6.0) * sx, VzA = (1.0 / 6.0) * sz;
         xk = xA + dt * VxA;
         zk = zA + dt * VzA;
         if (vxo) vxo[k] = VxA;
@@ -173,9 +177,15 @@ __global__ void k_advect_rk4(v2p_grid g, const double *__restrict__ u, const dou
     phase[k] = ph;
 }
 
+bool tables_ok(const mdg_ctx *c) {
+    for (const std::vector<double> *t : {&c->h_xg, &c->h_zg, &c->h_xvz, &c->h_zvx})
+        if (!std::all_of(t->begin(), t->end(), v2p_coord_ok)) return false;
+    return true;
+}
+
 v2p_grid make_grid(const mdg_ctx *c) {
-    return v2p_grid{c->Nx, c->Nz, c->dx, c->dz, c->xg.p, c->zg.p, c->xvz.p, c->zvx.p,
-                    c->BCu_t.p, c->BCv_t.p, c->xmin, c->xmax, c->zmin, c->zmax};
+    return v2p_grid{c->Nx, c->Nz, make_exact_div(c->dx), make_exact_div(c->dz), c->xg.p, c->zg.p, c->xvz.p, c->zvx.p,
+                    c->xmin, c->xmax, c->zmin, c->zmax, tables_ok(c) ? 1 : 0};
 }
 
 // A caller's array as a device pointer: itself, or a device copy (copied in
@@ -233,8 +243,8 @@ extern "C" int mdg_v2p(mdg_ctx *c, const double *u, const double *v, int conserv
         (rc = dev_view(c, vz, (size_t)n, s.vz, false, &dvz)))
         return rc;
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    hipLaunchKernelGGL(k_v2p, dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, make_grid(c), du, dv, conserv_interp, n,
-                       dx_, dz_, dph, dvx, dvz);
+    hipLaunchKernelGGL(conserv_interp == 1 ? k_v2p<true> : k_v2p<false>, dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream,
+                       make_grid(c), du, dv, n, dx_, dz_, dph, dvx, dvz);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     if ((rc = copy_back(c, vx, (const double *)dvx, (size_t)n)) || (rc = copy_back(c, vz, (const double *)dvz, (size_t)n)))
@@ -263,8 +273,8 @@ extern "C" int mdg_advect_rk4(mdg_ctx *c, const double *u, const double *v, doub
         (rc = dev_view(c, vz, (size_t)n, s.vz, true, &dvz)))
         return rc;
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    hipLaunchKernelGGL(k_advect_rk4, dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, make_grid(c), du, dv, dt,
-                       conserv_interp, n, dx_, dz_, dph, dvx, dvz);
+    hipLaunchKernelGGL(conserv_interp == 1 ? k_advect_rk4<true> : k_advect_rk4<false>, dim3(mdg_grid1d(n, 256)), dim3(256),
+                       0, c->stream, make_grid(c), du, dv, dt, n, dx_, dz_, dph, dvx, dvz);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     if ((rc = copy_back(c, x, (const double *)dx_, (size_t)n)) || (rc = copy_back(c, z, (const double *)dz_, (size_t)n)) ||

@@ -153,6 +153,9 @@ extern "C" int mdg_set_bc(mdg_ctx *c, const signed char *BCu_t, const double *BC
     HIPCHK(c, hipMemcpy(hv.data(), c->BCv_t.p, nv, hipMemcpyDeviceToHost));
     HIPCHK(c, hipMemcpy(hp.data(), c->BCp_t.p, np, hipMemcpyDeviceToHost));
     HIPCHK(c, hipMemcpy(hg.data(), c->BCg_t.p, ng, hipMemcpyDeviceToHost));
+    // the tags are on the device from here on, also if they are refused below
+    auto air = [](signed char t) { return t == 30 || t == 31; };
+    c->air_nodes = std::any_of(hp.begin(), hp.end(), air) || std::any_of(hg.begin(), hg.end(), air);
     for (size_t i = 0; i < np; i++)
         if (hp[i] != -1) return mdg_fail(c, MDG_ERR_UNSUPPORTED, "BCp_t must be -1 (no air cells)");
     for (size_t i = 0; i < ng; i++)

@@ -4,104 +4,131 @@
 // four centres around it (the centre field stays in L2); the marker streams
 // x, z, phase in and the field (or P read-modify-write) out. Same arithmetic
 // and order as the reference, built without contraction: bit-exact.
+//
+// Bound: the marker streams once the FP64 divisions by the cell widths are
+// exact_div's (the same bits at a fifth of the instructions) and the cell
+// index and weights are computed once for all fields of a node set. The
+// node tags are gathered only where the box has air nodes (AIR).
+// Measured with 37.7M markers on 2047^2: k_add_stress 0.96 -> 0.63 ms (2.56
+// GB of marker streams, 4.1 TB/s), k_add_g2p 0.39 -> 0.32 ms (1.36 GB).
+#include "exact_div.h"
 #include "mdg_internal.h"
 
 namespace {
 
 struct cgrid {
     int Nx, Nz;               // centres per row / column
-    double dx, dz;
+    exact_div dx, dz;
     const double *X, *Z;      // xvz, zvx (centre coordinates with one ghost each side)
     const signed char *tag;   // BCp
 };
 
-__device__ double g2p_cent_one(const cgrid &g, const double *__restrict__ F, double x, double z) {
-    const int Nx = g.Nx, Nz = g.Nz;
-    const double dx = g.dx, dz = g.dz;
-    const int j = (int)ceil((x - g.X[0]) / dx) - 1;
-    const int i = (int)ceil((z - g.Z[0]) / dz) - 1;
-    int iSW = 0, iSE = 0, iNW = 0, iNE = 0;
-    if (j > 0 && j < Nx && i > 0 && i < Nz) {
-        iSW = (j - 1) + (i - 1) * Nx; iSE = iSW + 1; iNW = (j - 1) + i * Nx; iNE = iNW + 1;
-    } else if (j == 0 && i > 0 && i < Nz) {          // west edge: copy along it
-        iSW = iSE = (i - 1) * Nx; iNW = iNE = i * Nx;
-    } else if (j == Nx && i > 0 && i < Nz) {         // east edge
-        iSW = iSE = (j - 1) + (i - 1) * Nx; iNW = iNE = (j - 1) + i * Nx;
-    } else if (i == 0 && j > 0 && j < Nx) {          // south edge
-        iSW = iNW = j - 1; iSE = iNE = j;
-    } else if (i == Nz && j > 0 && j < Nx) {         // north edge
-        iSW = iNW = (j - 1) + (i - 1) * Nx; iSE = iNE = iSW + 1;
-    } else if (i == 0 && j == 0) {
-        iSW = iSE = iNW = iNE = 0;
-    } else if (i == 0 && j == Nx) {
-        iSW = iSE = iNW = iNE = j - 1;
-    } else if (i == Nz && j == 0) {
-        iSW = iSE = iNW = iNE = (i - 1) * Nx;
-    } else if (i == Nz && j == Nx) {
-        iSW = iSE = iNW = iNE = (j - 1) + (i - 1) * Nx;
+// The four centres around a marker and their weights, shared by every field.
+struct cstencil {
+    int sw, se, nw, ne;
+    double wsw, wse, wnw, wne, sum;
+    template <typename F>
+    __device__ __forceinline__ double at(F f) const {
+        double val = 0.0;
+        val += wsw * f(sw);
+        val += wse * f(se);
+        val += wnw * f(nw);
+        val += wne * f(ne);
+        if (sum > 1e-13) val /= sum;
+        return val;
     }
-    // markers of the box always land in one of the cases above; clamp the
-    // coordinate index for any other input so every read stays in range
+};
+
+template <bool AIR>
+__device__ __forceinline__ cstencil g2p_cent(const cgrid &g, double x, double z) {
+    const int Nx = g.Nx, Nz = g.Nz;
+    const int j = (int)ceil(xdiv(x - g.X[0], g.dx)) - 1;
+    const int i = (int)ceil(xdiv(z - g.Z[0], g.dz)) - 1;
+    // The reference's nine cases (inside, four edges, four corners: copies
+    // along the edges) are the clamped columns and rows of the interior one;
+    // a marker outside them all (outside the box by half a cell) reads cell 0.
+    int iSW = 0, iSE = 0, iNW = 0, iNE = 0;
+    if (j >= 0 && j <= Nx && i >= 0 && i <= Nz) {
+        const int jw = max(j - 1, 0), je = min(j, Nx - 1), is = max(i - 1, 0) * Nx, in = min(i, Nz - 1) * Nx;
+        iSW = jw + is; iSE = je + is; iNW = jw + in; iNE = je + in;
+    }
+    // clamp the coordinate index for any other input so every read stays in range
     const int jj = j < 0 ? 0 : (j > Nx ? Nx : j), ii = i < 0 ? 0 : (i > Nz ? Nz : i);
-    const double dxm = x - g.X[jj], dzm = z - g.Z[ii];
-    const signed char *t = g.tag;
-    const bool aSW = t[iSW] == 30 || t[iSW] == 31, aSE = t[iSE] == 30 || t[iSE] == 31;
-    const bool aNW = t[iNW] == 30 || t[iNW] == 31, aNE = t[iNE] == 30 || t[iNE] == 31;
-    double val = 0.0, sumW = 0.0;
-    val += (1.0 - dxm / dx) * (1.0 - dzm / dz) * F[aSW ? iNW : iSW];
-    sumW += (1.0 - dxm / dx) * (1.0 - dzm / dz);
-    val += (dxm / dx) * (1.0 - dzm / dz) * F[aSE ? iNE : iSE];
-    sumW += (dxm / dx) * (1.0 - dzm / dz);
-    val += (1.0 - dxm / dx) * (dzm / dz) * F[aNW ? iSW : iNW];
-    sumW += (1.0 - dxm / dx) * (dzm / dz);
-    val += (dxm / dx) * (dzm / dz) * F[aNE ? iSE : iNE];
-    sumW += (dxm / dx) * (dzm / dz);
-    if (sumW > 1e-13) val /= sumW;
-    return val;
+    const double tx = xdiv(x - g.X[jj], g.dx), tz = xdiv(z - g.Z[ii], g.dz);
+    cstencil c;
+    c.sw = iSW; c.se = iSE; c.nw = iNW; c.ne = iNE;
+    if (AIR) {
+        const signed char *t = g.tag;
+        const bool aSW = t[iSW] == 30 || t[iSW] == 31, aSE = t[iSE] == 30 || t[iSE] == 31;
+        const bool aNW = t[iNW] == 30 || t[iNW] == 31, aNE = t[iNE] == 30 || t[iNE] == 31;
+        if (aSW) c.sw = iNW;
+        if (aSE) c.se = iNE;
+        if (aNW) c.nw = iSW;
+        if (aNE) c.ne = iSE;
+    }
+    c.wsw = (1.0 - tx) * (1.0 - tz);
+    c.wse = tx * (1.0 - tz);
+    c.wnw = (1.0 - tx) * tz;
+    c.wne = tx * tz;
+    c.sum = 0.0;
+    c.sum += c.wsw;
+    c.sum += c.wse;
+    c.sum += c.wnw;
+    c.sum += c.wne;
+    return c;
 }
 
+template <bool AIR>
 __global__ void k_g2p_centroids(cgrid g, const double *__restrict__ F, int n, const double *__restrict__ x,
                                 const double *__restrict__ z, const int *__restrict__ phase,
                                 double *__restrict__ out) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    out[k] = (phase[k] != -1) ? g2p_cent_one(g, F, x[k], z[k]) : 0.0;
+    out[k] = (phase[k] != -1) ? g2p_cent<AIR>(g, x[k], z[k]).at([&](int c) { return F[c]; }) : 0.0;
 }
 
 // Interp_Grid2P (ParticleRoutines.c:1223-1325) on the vertices
 struct vgrid {
     int Nx, Nz;
-    double dx, dz;
+    exact_div dx, dz;
     const double *X, *Z;      // xg, zg
     const signed char *tag;   // BCg
 };
-__device__ double g2p_vert_one(const vgrid &g, const double *__restrict__ F, double xk, double zk) {
-    const double dx = g.dx, dz = g.dz;
-    int j = (int)ceil((xk - g.X[0]) / dx) - 1;
+template <bool AIR>
+__device__ __forceinline__ double g2p_vert_one(const vgrid &g, const double *__restrict__ F, double xk, double zk) {
+    int j = (int)ceil(xdiv(xk - g.X[0], g.dx)) - 1;
     if (j < 0) j = 0;
     if (j > g.Nx - 2) j = g.Nx - 2;
-    int i = (int)ceil((zk - g.Z[0]) / dz) - 1;
+    int i = (int)ceil(xdiv(zk - g.Z[0], g.dz)) - 1;
     if (i < 0) i = 0;
     if (i > g.Nz - 2) i = g.Nz - 2;
-    const double dxm = fabs(xk - g.X[j]), dzm = fabs(zk - g.Z[i]);
+    const double tx = xdiv(fabs(xk - g.X[j]), g.dx), tz = xdiv(fabs(zk - g.Z[i]), g.dz);
     const int iSW = j + i * g.Nx, iSE = iSW + 1, iNW = j + (i + 1) * g.Nx, iNE = iNW + 1;
-    const signed char *t = g.tag;
-    const bool aSW = t[iSW] == 30 || t[iSW] == 31, aSE = t[iSE] == 30 || t[iSE] == 31;
-    const bool aNW = t[iNW] == 30 || t[iNW] == 31, aNE = t[iNE] == 30 || t[iNE] == 31;
+    int sw = iSW, se = iSE, nw = iNW, ne = iNE;
+    if (AIR) {
+        const signed char *t = g.tag;
+        const bool aSW = t[iSW] == 30 || t[iSW] == 31, aSE = t[iSE] == 30 || t[iSE] == 31;
+        const bool aNW = t[iNW] == 30 || t[iNW] == 31, aNE = t[iNE] == 30 || t[iNE] == 31;
+        if (aSW) sw = iNW;
+        if (aSE) se = iNE;
+        if (aNW) nw = iSW;
+        if (aNE) ne = iSE;
+    }
     double val = 0.0;
-    val += (1.0 - dxm / dx) * (1.0 - dzm / dz) * F[aSW ? iNW : iSW];
-    val += (dxm / dx) * (1.0 - dzm / dz) * F[aSE ? iNE : iSE];
-    val += (1.0 - dxm / dx) * (dzm / dz) * F[aNW ? iSW : iNW];
-    val += (dxm / dx) * (dzm / dz) * F[aNE ? iSE : iNE];
+    val += (1.0 - tx) * (1.0 - tz) * F[sw];
+    val += tx * (1.0 - tz) * F[se];
+    val += (1.0 - tx) * tz * F[nw];
+    val += tx * tz * F[ne];
     return val;
 }
 
+template <bool AIR>
 __global__ void k_g2p_vertices(vgrid g, const double *__restrict__ F, int n, const double *__restrict__ x,
                                const double *__restrict__ z, const int *__restrict__ phase,
                                double *__restrict__ out) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    out[k] = (phase[k] != -1) ? g2p_vert_one(g, F, x[k], z[k]) : 0.0;
+    out[k] = (phase[k] != -1) ? g2p_vert_one<AIR>(g, F, x[k], z[k]) : 0.0;
 }
 
 // grid stress increments of UpdateParticleStress (RheologyParticles.c:1929-1939)
@@ -121,17 +148,25 @@ __global__ void k_stress_increments(int nc, int nv, const signed char *__restric
         dxz[j] = (tg[j] != 30) ? sxz[j] - sxz0[j] : 0.0;
     }
 }
+template <bool AIR>
 __global__ void k_add_stress(cgrid gc, vgrid gv, const double *__restrict__ dxx, const double *__restrict__ dzz,
                              const double *__restrict__ dxz, int n, const double *__restrict__ x,
                              const double *__restrict__ z, const int *__restrict__ phase, double *__restrict__ mxx,
                              double *__restrict__ mzz, double *__restrict__ mxz) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    const bool on = phase[k] != -1;
-    const double xk = x[k], zk = z[k];
-    mxx[k] = mxx[k] + (on ? g2p_cent_one(gc, dxx, xk, zk) : 0.0);
-    mzz[k] = mzz[k] + (on ? g2p_cent_one(gc, dzz, xk, zk) : 0.0);
-    mxz[k] = mxz[k] + (on ? g2p_vert_one(gv, dxz, xk, zk) : 0.0);
+    const double xx = mxx[k], zz = mzz[k], xz = mxz[k];
+    double a = 0.0, b = 0.0, c = 0.0;
+    if (phase[k] != -1) {
+        const double xk = x[k], zk = z[k];
+        const cstencil s = g2p_cent<AIR>(gc, xk, zk);
+        a = s.at([&](int q) { return dxx[q]; });
+        b = s.at([&](int q) { return dzz[q]; });
+        c = g2p_vert_one<AIR>(gv, dxz, xk, zk);
+    }
+    mxx[k] = xx + a;
+    mzz[k] = zz + b;
+    mxz[k] = xz + c;
 }
 
 __global__ void k_pressure_increment(int nc, const signed char *__restrict__ tag, const double *__restrict__ p_in,
@@ -140,12 +175,14 @@ __global__ void k_pressure_increment(int nc, const signed char *__restrict__ tag
     if (c < nc) dp[c] = (tag[c] != 30) ? (p_in[c] - p0[c]) : 0.0;
 }
 
+template <bool AIR>
 __global__ void k_add_g2p(cgrid g, const double *__restrict__ F, int n, const double *__restrict__ x,
                           const double *__restrict__ z, const int *__restrict__ phase, double *__restrict__ P) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    const double inc = (phase[k] != -1) ? g2p_cent_one(g, F, x[k], z[k]) : 0.0;
-    P[k] = P[k] + inc;
+    const double p = P[k];
+    const double inc = (phase[k] != -1) ? g2p_cent<AIR>(g, x[k], z[k]).at([&](int c) { return F[c]; }) : 0.0;
+    P[k] = p + inc;
 }
 
 // AccumulatedStrainII (RheologyParticles.c:346-649): per-centre increments
@@ -181,7 +218,7 @@ __global__ void k_strain_increments(int nc, double dt, strain_rates7 r, double *
 struct strain_out8 {
     double *s[8];            // strain, el, pl, pl_vol, pwl, exp, lin, gbs
 };
-__global__ void k_accumulate_strain(int Ncx, int Ncz, double dx, double dz, const double *__restrict__ xc,
+__global__ void k_accumulate_strain(int Ncx, int Ncz, exact_div dx, exact_div dz, const double *__restrict__ xc,
                                     const double *__restrict__ zc, const signed char *__restrict__ tag,
                                     const double *__restrict__ inc, int n, const double *__restrict__ x,
                                     const double *__restrict__ z, const int *__restrict__ phase, strain_out8 out) {
@@ -191,14 +228,13 @@ __global__ void k_accumulate_strain(int Ncx, int Ncz, double dx, double dz, cons
     double dE[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (phase[k] != -1) {
         const double xk = x[k], zk = z[k];
-        int j = (int)ceil((xk - xc[0]) / dx) - 1;
+        int j = (int)ceil(xdiv(xk - xc[0], dx)) - 1;
         j = j < 0 ? 0 : (j > Ncx - 2 ? Ncx - 2 : j);
-        int i = (int)ceil((zk - zc[0]) / dz) - 1;
+        int i = (int)ceil(xdiv(zk - zc[0], dz)) - 1;
         i = i < 0 ? 0 : (i > Ncz - 2 ? Ncz - 2 : i);
-        const double dxm = xk - xc[j], dzm = zk - zc[i];
+        const double tx = xdiv(xk - xc[j], dx), tz = xdiv(zk - zc[i], dz);
         const int nd[4] = {j + i * Ncx, j + i * Ncx + 1, j + (i + 1) * Ncx, j + (i + 1) * Ncx + 1};
-        const double w[4] = {(1.0 - dxm / dx) * (1.0 - dzm / dz), (dxm / dx) * (1.0 - dzm / dz),
-                             (1.0 - dxm / dx) * (dzm / dz), (dxm / dx) * (dzm / dz)};
+        const double w[4] = {(1.0 - tx) * (1.0 - tz), tx * (1.0 - tz), (1.0 - tx) * tz, tx * tz};
         double sumW = 0.0;
         for (int q = 0; q < 4; q++) {
             const signed char t = tag[nd[q]];
@@ -232,8 +268,13 @@ __global__ void k_rotate_stress(int mode, double dt, int n, const int *__restric
 }
 
 cgrid make_cgrid(const mdg_ctx *c) {
-    return cgrid{c->Nx - 1, c->Nz - 1, c->dx, c->dz, c->xvz.p, c->zvx.p, c->BCp_t.p};
+    return cgrid{c->Nx - 1, c->Nz - 1, make_exact_div(c->dx), make_exact_div(c->dz), c->xvz.p, c->zvx.p, c->BCp_t.p};
 }
+vgrid make_vgrid(const mdg_ctx *c) {
+    return vgrid{c->Nx, c->Nz, make_exact_div(c->dx), make_exact_div(c->dz), c->xg.p, c->zg.p, c->BCg_t.p};
+}
+// instantiation of a marker kernel for a box with or without air nodes
+#define G2P_AIR(c, K) ((c)->air_nodes ? K<true> : K<false>)
 
 // Subgrid relaxation of UpdateParticleStress / UpdateParticlePressure
 // (RheologyParticles.c:1845-1850, :1660-1666): on active markers
@@ -344,7 +385,7 @@ extern "C" int mdg_g2p_centroids(mdg_ctx *c, const double *F, int n, const doubl
         dout = s.out.p;
     }
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    hipLaunchKernelGGL(k_g2p_centroids, dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, make_cgrid(c), dF, n, dx_,
+    hipLaunchKernelGGL(G2P_AIR(c, k_g2p_centroids), dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, make_cgrid(c), dF, n, dx_,
                        dz_, dph, dout);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
@@ -369,9 +410,9 @@ extern "C" int mdg_g2p_vertices(mdg_ctx *c, const double *F, int n, const double
         HIPCHK(c, s.out.reserve((size_t)n));
         dout = s.out.p;
     }
-    const vgrid g = {c->Nx, c->Nz, c->dx, c->dz, c->xg.p, c->zg.p, c->BCg_t.p};
+    const vgrid g = make_vgrid(c);
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    hipLaunchKernelGGL(k_g2p_vertices, dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, g, dF, n, dx_, dz_, dph, dout);
+    hipLaunchKernelGGL(G2P_AIR(c, k_g2p_vertices), dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, g, dF, n, dx_, dz_, dph, dout);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     if (dout != out) HIPCHK(c, hipMemcpyAsync(out, dout, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
@@ -406,7 +447,7 @@ extern "C" int mdg_update_particle_pressure(mdg_ctx *c, const double *p_in, cons
     hipLaunchKernelGGL(k_pressure_increment, dim3(mdg_grid1d(nc, 256)), dim3(256), 0, c->stream, nc,
                        (const signed char *)c->BCp_t.p, dpin, dp0, ddp);
     if (n > 0)
-        hipLaunchKernelGGL(k_add_g2p, dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, make_cgrid(c), (const double *)ddp,
+        hipLaunchKernelGGL(G2P_AIR(c, k_add_g2p), dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, make_cgrid(c), (const double *)ddp,
                            n, dx_, dz_, dph, dP);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
@@ -448,12 +489,12 @@ extern "C" int mdg_update_particle_stress(mdg_ctx *c, const double *sxxd, const 
             dm[q] = s.m[q].p;
         }
     }
-    const vgrid gv = {c->Nx, c->Nz, c->dx, c->dz, c->xg.p, c->zg.p, c->BCg_t.p};
+    const vgrid gv = make_vgrid(c);
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     hipLaunchKernelGGL(k_stress_increments, dim3(mdg_grid1d(nc + nv, 256)), dim3(256), 0, c->stream, nc, nv,
                        (const signed char *)c->BCp_t.p, (const signed char *)c->BCg_t.p, d[0], d[1], d[2], d[3], d[4],
                        d[5], dxx, dzz, dxz);
-    hipLaunchKernelGGL(k_add_stress, dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, make_cgrid(c), gv,
+    hipLaunchKernelGGL(G2P_AIR(c, k_add_stress), dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, make_cgrid(c), gv,
                        (const double *)dxx, (const double *)dzz, (const double *)dxz, n, dx_, dz_, dph, dm[0], dm[1],
                        dm[2]);
     HIPCHK(c, hipGetLastError());
@@ -499,7 +540,8 @@ extern "C" int mdg_accumulated_strain(mdg_ctx *c, double dt, const double *const
     if (h_bad != 0x7f7f7f7f)
         return mdg_fail(c, MDG_ERR_ARG, "negative strain increment at cell %d (AccumulatedStrainII exits there)", h_bad - 1);
     if (n > 0)
-        hipLaunchKernelGGL(k_accumulate_strain, dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, Ncx, Ncz, c->dx, c->dz,
+        hipLaunchKernelGGL(k_accumulate_strain, dim3(mdg_grid1d(n, 256)), dim3(256), 0, c->stream, Ncx, Ncz, make_exact_div(c->dx),
+                           make_exact_div(c->dz),
                            (const double *)c->xc.p, (const double *)c->zc.p, (const signed char *)c->BCp_t.p,
                            (const double *)s.inc.p, n, dx_, dz_, dph, out);
     HIPCHK(c, hipGetLastError());
@@ -601,17 +643,17 @@ extern "C" int mdg_update_particle_stress_subgrid(mdg_ctx *c, double dt, const d
     HIPCHK(c, s.inc.reserve((size_t)nv));
     double *gs[3] = {s.gsub[0].p, s.gsub[1].p, s.gsub[2].p}, *gr[3] = {s.gsub[3].p, s.gsub[4].p, s.inc.p};
     const cgrid gc = make_cgrid(c);
-    const vgrid gv = {c->Nx, c->Nz, c->dx, c->dz, c->xg.p, c->zg.p, c->BCg_t.p};
+    const vgrid gv = make_vgrid(c);
     local_timer t;
     HIPCHK(c, hipEventCreate(&t.a));
     HIPCHK(c, hipEventCreate(&t.b));
     HIPCHK(c, hipEventRecord(t.a, c->stream));
     const dim3 gm(mdg_grid1d(n, 256)), bk(256);
     // old stresses and the vertex viscosity at the markers
-    hipLaunchKernelGGL(k_g2p_centroids, gm, bk, 0, c->stream, gc, d[3], n, dx_, dz_, dph, m0[0]);
-    hipLaunchKernelGGL(k_g2p_centroids, gm, bk, 0, c->stream, gc, d[4], n, dx_, dz_, dph, m0[1]);
-    hipLaunchKernelGGL(k_g2p_vertices, gm, bk, 0, c->stream, gv, d[5], n, dx_, dz_, dph, m0[2]);
-    hipLaunchKernelGGL(k_g2p_vertices, gm, bk, 0, c->stream, gv, d[6], n, dx_, dz_, dph, etam);
+    hipLaunchKernelGGL(G2P_AIR(c, k_g2p_centroids), gm, bk, 0, c->stream, gc, d[3], n, dx_, dz_, dph, m0[0]);
+    hipLaunchKernelGGL(G2P_AIR(c, k_g2p_centroids), gm, bk, 0, c->stream, gc, d[4], n, dx_, dz_, dph, m0[1]);
+    hipLaunchKernelGGL(G2P_AIR(c, k_g2p_vertices), gm, bk, 0, c->stream, gv, d[5], n, dx_, dz_, dph, m0[2]);
+    hipLaunchKernelGGL(G2P_AIR(c, k_g2p_vertices), gm, bk, 0, c->stream, gv, d[6], n, dx_, dz_, dph, etam);
     relax3 ra{{dm[0], dm[1], dm[2]}, {m0[0], m0[1], m0[2]}, {ms[0], ms[1], ms[2]}};
     hipLaunchKernelGGL(k_subgrid_relax, gm, bk, 0, c->stream, n, 3, dt, dG, dph, (const double *)etam, ra);
     HIPCHK(c, hipGetLastError());
@@ -625,9 +667,9 @@ extern "C" int mdg_update_particle_stress_subgrid(mdg_ctx *c, double dt, const d
     hipLaunchKernelGGL(k_stress_remaining, dim3(mdg_grid1d(nc + nv, 256)), bk, 0, c->stream, nc, nv,
                        (const signed char *)c->BCp_t.p, (const signed char *)c->BCg_t.p, d[0], d[1], d[2], d[3], d[4],
                        d[5], (const double *)gs[0], (const double *)gs[1], (const double *)gs[2], gr[0], gr[1], gr[2]);
-    hipLaunchKernelGGL(k_g2p_centroids, gm, bk, 0, c->stream, gc, (const double *)gr[0], n, dx_, dz_, dph, mr[0]);
-    hipLaunchKernelGGL(k_g2p_centroids, gm, bk, 0, c->stream, gc, (const double *)gr[1], n, dx_, dz_, dph, mr[1]);
-    hipLaunchKernelGGL(k_g2p_vertices, gm, bk, 0, c->stream, gv, (const double *)gr[2], n, dx_, dz_, dph, mr[2]);
+    hipLaunchKernelGGL(G2P_AIR(c, k_g2p_centroids), gm, bk, 0, c->stream, gc, (const double *)gr[0], n, dx_, dz_, dph, mr[0]);
+    hipLaunchKernelGGL(G2P_AIR(c, k_g2p_centroids), gm, bk, 0, c->stream, gc, (const double *)gr[1], n, dx_, dz_, dph, mr[1]);
+    hipLaunchKernelGGL(G2P_AIR(c, k_g2p_vertices), gm, bk, 0, c->stream, gv, (const double *)gr[2], n, dx_, dz_, dph, mr[2]);
     for (int q = 0; q < 3; q++)
         hipLaunchKernelGGL(k_add_two, gm, bk, 0, c->stream, n, dph, (const double *)ms[q], (const double *)mr[q], dm[q]);
     HIPCHK(c, hipGetLastError());
@@ -681,16 +723,16 @@ extern "C" int mdg_update_particle_pressure_subgrid(mdg_ctx *c, double dt, const
     const signed char *tag = c->BCp_t.p;
     hipLaunchKernelGGL(k_pressure_increment, gcl, bk, 0, c->stream, nc, tag, dpin, dp0, ddp);
     if (n > 0) {
-        hipLaunchKernelGGL(k_g2p_centroids, gm, bk, 0, c->stream, gc, deta, n, dx_, dz_, dph, etam);
+        hipLaunchKernelGGL(G2P_AIR(c, k_g2p_centroids), gm, bk, 0, c->stream, gc, deta, n, dx_, dz_, dph, etam);
         hipLaunchKernelGGL(k_masked, gcl, bk, 0, c->stream, nc, tag, dp0, (const double *)nullptr, Pg0);
-        hipLaunchKernelGGL(k_g2p_centroids, gm, bk, 0, c->stream, gc, (const double *)Pg0, n, dx_, dz_, dph, Pm0);
+        hipLaunchKernelGGL(G2P_AIR(c, k_g2p_centroids), gm, bk, 0, c->stream, gc, (const double *)Pg0, n, dx_, dz_, dph, Pm0);
         relax3 ra{{dP[0], nullptr, nullptr}, {Pm0, nullptr, nullptr}, {dPms, nullptr, nullptr}};
         hipLaunchKernelGGL(k_subgrid_relax, gm, bk, 0, c->stream, n, 1, dt, dB, dph, (const double *)etam, ra);
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipMemsetAsync(dPgs, 0, (size_t)nc * 8, c->stream));
         if ((rc = mdg_p2mastah(c, dPms, n, dPgs, tag, 1, 0, 0, 1, 1, 0, nullptr))) return rc;
         hipLaunchKernelGGL(k_masked, gcl, bk, 0, c->stream, nc, tag, (const double *)ddp, (const double *)dPgs, dPgr);
-        hipLaunchKernelGGL(k_g2p_centroids, gm, bk, 0, c->stream, gc, (const double *)dPgr, n, dx_, dz_, dph, dPmr);
+        hipLaunchKernelGGL(G2P_AIR(c, k_g2p_centroids), gm, bk, 0, c->stream, gc, (const double *)dPgr, n, dx_, dz_, dph, dPmr);
         hipLaunchKernelGGL(k_add_two, gm, bk, 0, c->stream, n, dph, (const double *)dPms, (const double *)dPmr, dP[0]);
     }
     HIPCHK(c, hipGetLastError());

@@ -51,6 +51,7 @@ struct mdg_ctx {
     dbuf<signed char> BCu_t, BCv_t, BCp_t, BCg_t;
     dbuf<double>      BCu_v, BCv_v;
     bool              have_bc = false;
+    bool              air_nodes = false;   // a centre or vertex tag is 30 or 31
     // markers, sorted by (cell, quarter cell)
     int               n_markers = 0;
     dbuf<double>      mx, mz;        // sorted coordinates
