@@ -4,27 +4,40 @@
 // Jacobi-preconditioned CG of SolveThermalPCG (ThermalSolver.c:338-480)
 // started from the current temperature.
 //
-// Per iteration four launches on the context's stream:
-//   apply  : p = z + beta p_old on the cell and its four neighbours (the
-//            previous iteration's direction update, folded in here), q = A p,
+// Per iteration two launches on the context's stream:
+//   apply  : the previous iteration's ||r|| / ||r0|| test, breakdown -3,
+//            iteration limit and beta; p = z + beta p_old on the cell and its
+//            four neighbours (the direction update, folded in here), q = A p,
 //            block partials of p.q;
-//   fin1   : alpha = rz / p.q (breakdown -2);
-//   update : x += alpha p, r -= alpha q, z = M^-1 r, block partials of r.r
-//            and r.z;
-//   fin2   : ||r|| / ||r0|| test, breakdown -3, beta, iteration limit.
-// The control block lives in device memory; once it says "done" every later
-// launch returns at once, so the host queues iterations in batches and
-// reads the control block between batches only.  Products and sums within a
-// cell follow the reference's CSR row order (south, west, centre, east,
-// north), so only the dot-product reductions round differently.
+//   update : alpha = rz / p.q (breakdown -2); x += alpha p, r -= alpha q,
+//            z = M^-1 r, block partials of r.r and r.z.
+// Every block sums the previous kernel's partials itself, in one fixed order
+// (at most TH_BLOCKS of them, read from L2), and takes the same decision;
+// block 0 writes it down for the next kernel.  One-block kernels for those
+// sums over 16k partials took 46 of an iteration's 144 us at 2047^2, and two
+// launches of the four on small grids.  Once the control block says "done"
+// every later launch returns at once, so the host queues iterations in
+// batches and reads the control block between batches only.  Products and
+// sums within a cell follow the reference's CSR row order (south, west,
+// centre, east, north), so only the dot-product reductions round differently.
+//
+// Bound: memory.  apply streams 7 arrays of a cell (z, p_old, kx, kz, diag
+// read, p, q written), update 8 (p, q, r, x, minv read, x, r, z written).
+// Measured at 2047^2: apply 66 us, update 44 us (3.6 and 6.1 TB/s, the second
+// helped by the last-level cache), against 57 + 16 + 38 + 30 us for the four
+// kernels.  2048 blocks, or two or four cells of a thread loaded before any is
+// stored, measured 70-77 and 47-49 us: the blocks then spread over more rows.
+#include <cmath>
+
 #include "mdg_internal.h"
 
 namespace {
 
-constexpr int TB = 256;
+constexpr int TB = 512;
 
+// State between kernels: [0] written by update (and the set-up), [1] by apply.
 struct th_ctl {
-    double rz, r0, alpha, beta, rel_tol;
+    double rz, r0, rel_tol, alpha, beta;
     int done, its, it, max_its;
 };
 
@@ -33,22 +46,52 @@ struct th_geom {
     double idx2, idz2, dx;
 };
 
-// Block b of nb takes a contiguous share of the cell range per XCD (blocks
-// are dispatched round-robin over the 8 XCDs), so the rows above and below a
-// block's cells are in the same L2 as the neighbouring blocks that read them.
-__device__ inline int xcd_block(int b, int nb) {
-    const int xcd = b & 7, per = nb >> 3, rem = nb & 7;
-    return xcd * per + min(xcd, rem) + (b >> 3);
+// At most this many blocks (4 per CU, all resident).  Blocks are dispatched
+// round-robin over the 8 XCDs; each XCD takes a contiguous band of the cells
+// and its blocks walk it side by side in steps of TB, so that the rows above
+// and below a block's cells are in the same L2 as the blocks that read them.
+constexpr int TH_BLOCKS = 1024;
+struct th_share {
+    int lo, hi, step;      // cells lo + threadIdx.x, + step, ... below hi
+};
+__device__ inline th_share th_cells(int n) {
+    const int nb = gridDim.x, xcd = blockIdx.x & 7, per = nb >> 3, rem = nb & 7;
+    const int first = xcd * per + min(xcd, rem), mine = per + (xcd < rem ? 1 : 0);   // the XCD's blocks
+    const long steps = (n + TB - 1) / TB;
+    const int lo = (int)(steps * first / nb), hi = (int)(steps * (first + mine) / nb);
+    return th_share{(lo + (int)(blockIdx.x >> 3)) * TB, min(n, hi * TB), mine * TB};
 }
 
-__device__ inline double block_sum(double v, double *s) {
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int w = TB / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-        __syncthreads();
+// Sums of a and b over the block, in every thread.
+struct sum2 {
+    double a, b;
+};
+__device__ inline sum2 block_sum2(double a, double b, double (*s)[2]) {
+    for (int w = 32; w > 0; w >>= 1) {
+        a += __shfl_xor(a, w);
+        b += __shfl_xor(b, w);
     }
-    return s[0];
+    if ((threadIdx.x & 63) == 0) {
+        s[threadIdx.x >> 6][0] = a;
+        s[threadIdx.x >> 6][1] = b;
+    }
+    __syncthreads();
+    sum2 t{0.0, 0.0};
+    for (int w = 0; w < TB / 64; w++) {
+        t.a += s[w][0];
+        t.b += s[w][1];
+    }
+    __syncthreads();
+    return t;
+}
+// Totals of nb <= TH_BLOCKS partials, the same in every block and thread.
+__device__ inline sum2 part_sum2(int nb, const double *__restrict__ pa, const double *__restrict__ pb, double (*s)[2]) {
+    double a = 0.0, b = 0.0;
+    for (int i = threadIdx.x; i < nb; i += TB) {
+        a += pa[i];
+        if (pb) b += pb[i];
+    }
+    return block_sum2(a, b, s);
 }
 
 // Diagonal and boundary right-hand side of cell (k, l), in the order of the
@@ -84,17 +127,22 @@ __device__ inline void th_diag(const th_geom &g, double rhoCp_dt, const double *
     *bbc = b;
 }
 
-// Row c2 = (k, l) of A times v, with P(j) giving v at cell j.
+// Row c2 = (k, l) of A times v, with P(j) giving v at cell j.  At a wall the
+// neighbour is the cell itself with a zero coefficient: its product adds a
+// zero, and the loads of all five cells stay free of branches.
 template <typename F>
 __device__ inline double th_row(const th_geom &g, const double *__restrict__ kx, const double *__restrict__ kz,
                                 double d, int k, int l, int c2, F P) {
     const int c1 = k + (l + 1) * g.nx, c3 = k + l * g.nxvz + 1;
+    const bool S = l > 0, W = k > 0, E = k < g.ncx - 1, N = l < g.ncz - 1;
+    const double aS = S ? -kz[c3] * g.idz2 : 0.0, aW = W ? -kx[c1] * g.idx2 : 0.0;
+    const double aE = E ? -kx[c1 + 1] * g.idx2 : 0.0, aN = N ? -kz[c3 + g.nxvz] * g.idz2 : 0.0;
     double s = 0.0;
-    if (l > 0) s += -kz[c3] * g.idz2 * P(c2 - g.ncx);
-    if (k > 0) s += -kx[c1] * g.idx2 * P(c2 - 1);
+    s += aS * P(S ? c2 - g.ncx : c2);
+    s += aW * P(W ? c2 - 1 : c2);
     s += d * P(c2);
-    if (k < g.ncx - 1) s += -kx[c1 + 1] * g.idx2 * P(c2 + 1);
-    if (l < g.ncz - 1) s += -kz[c3 + g.nxvz] * g.idz2 * P(c2 + g.ncx);
+    s += aE * P(E ? c2 + 1 : c2);
+    s += aN * P(N ? c2 + g.ncx : c2);
     return s;
 }
 
@@ -103,17 +151,17 @@ struct th_in {
     const signed char *BT;
 };
 
-// b, diag, M^-1, r = b - A x, z = M^-1 r, p = z; partials of r.z and r.r.
+// b, diag, M^-1, r = b - A x, z = M^-1 r, p = z; partials of r.r and r.z.
 __global__ void __launch_bounds__(TB) k_th_setup(th_geom g, double dt, th_in in, const double *__restrict__ x,
                                                  double *__restrict__ diag, double *__restrict__ minv,
                                                  double *__restrict__ r, double *__restrict__ z,
-                                                 double *__restrict__ p, double *__restrict__ part_rz,
-                                                 double *__restrict__ part_rr) {
-    __shared__ double s[TB];
-    const int n = g.ncx * g.ncz, blk = xcd_block(blockIdx.x, gridDim.x);
-    const int c2 = blk * TB + threadIdx.x;
+                                                 double *__restrict__ p, double *__restrict__ part_rr,
+                                                 double *__restrict__ part_rz) {
+    __shared__ double s[TB / 64][2];
+    const int n = g.ncx * g.ncz;
+    const th_share c = th_cells(n);
     double rz = 0.0, rr = 0.0;
-    if (c2 < n) {
+    for (int c2 = c.lo + threadIdx.x; c2 < c.hi; c2 += c.step) {
         const int k = c2 % g.ncx, l = c2 / g.ncx;
         const double rhoCp = in.rho[c2] * in.Cp[c2];
         double d, bbc;
@@ -131,129 +179,147 @@ __global__ void __launch_bounds__(TB) k_th_setup(th_geom g, double dt, th_in in,
         const double zi = mi * ri;
         z[c2] = zi;
         p[c2] = zi;
-        rz = ri * zi;
-        rr = ri * ri;
+        rz += ri * zi;
+        rr += ri * ri;
     }
-    const double a = block_sum(rz, s);
-    __syncthreads();
-    const double b2 = block_sum(rr, s);
+    const sum2 t = block_sum2(rr, rz, s);
     if (threadIdx.x == 0) {
-        part_rz[blk] = a;
-        part_rr[blk] = b2;
+        part_rr[blockIdx.x] = t.a;
+        part_rz[blockIdx.x] = t.b;
     }
 }
 
-__device__ inline double sum_parts(int nb, const double *__restrict__ part, double *s) {
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < nb; i += TB) acc += part[i];
-    return block_sum(acc, s);
-}
-
-__global__ void __launch_bounds__(TB) k_th_fin0(int nb, const double *__restrict__ part_rz,
-                                                const double *__restrict__ part_rr, th_ctl *ctl) {
-    __shared__ double s[TB];
-    const double rz = sum_parts(nb, part_rz, s);
-    __syncthreads();
-    const double rr = sum_parts(nb, part_rr, s);
+__global__ void __launch_bounds__(TB) k_th_start(int nb, const double *__restrict__ part_rr,
+                                                 const double *__restrict__ part_rz, th_ctl *ctl) {
+    __shared__ double s[TB / 64][2];
+    const sum2 t = part_sum2(nb, part_rr, part_rz, s);
     if (threadIdx.x == 0) {
-        const double r0 = sqrt(rr);
-        ctl->rz = rz;
-        ctl->r0 = r0;
-        ctl->beta = 0.0;
-        ctl->it = 0;
-        ctl->done = (r0 < 1e-30) ? 1 : 0;
-        ctl->its = (r0 < 1e-30) ? 0 : -1;
+        const double r0 = sqrt(t.a);
+        th_ctl c = ctl[0];
+        c.rz = t.b;
+        c.r0 = r0;
+        c.it = 0;
+        c.done = (r0 < 1e-30) ? 1 : 0;
+        c.its = (r0 < 1e-30) ? 0 : -1;
+        ctl[0] = c;
+        ctl[1] = c;
     }
 }
 
+// FIRST: p = z (the set-up's), nothing to test.
+template <bool FIRST>
 __global__ void __launch_bounds__(TB) k_th_apply(th_geom g, const double *__restrict__ kx,
                                                  const double *__restrict__ kz, const double *__restrict__ diag,
                                                  const double *__restrict__ z, const double *__restrict__ pold,
-                                                 double *__restrict__ pnew, double *__restrict__ q,
-                                                 double *__restrict__ part, const th_ctl *__restrict__ ctl) {
-    if (ctl->done) return;
-    __shared__ double s[TB];
-    const double beta = ctl->beta;
-    const int n = g.ncx * g.ncz, blk = xcd_block(blockIdx.x, gridDim.x);
-    const int c2 = blk * TB + threadIdx.x;
+                                                 double *__restrict__ pnew, double *__restrict__ q, int nb,
+                                                 const double *__restrict__ part_rr, const double *__restrict__ part_rz,
+                                                 double *__restrict__ part_pq, th_ctl *ctl) {
+    __shared__ double s[TB / 64][2];
+    sum2 t{0.0, 0.0};
+    if (!FIRST) t = part_sum2(nb, part_rr, part_rz, s);   // before the test: one round of loads
+    th_ctl c = ctl[0];
+    if (c.done) return;
+    if (!FIRST) {
+        c.it++;
+        if (sqrt(t.a) / c.r0 < c.rel_tol) {
+            c.its = c.it;
+            c.done = 1;
+        } else if (fabs(c.rz) < 1e-30) {
+            c.its = -3;
+            c.done = 1;
+        } else {
+            c.beta = t.b / c.rz;
+            c.rz = t.b;
+            if (c.it >= c.max_its) c.done = 1;   // its stays -1
+        }
+    } else {
+        c.beta = 0.0;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl[1] = c;
+    if (c.done) return;
+    const int n = g.ncx * g.ncz;
+    const th_share sh = th_cells(n);
+    const double beta = c.beta;
     double pq = 0.0;
-    if (c2 < n) {
-        const int k = c2 % g.ncx, l = c2 / g.ncx;
+    int c2 = sh.lo + threadIdx.x, l = c2 / g.ncx, k = c2 - l * g.ncx;
+    const int dl = sh.step / g.ncx, dk = sh.step - dl * g.ncx;
+    for (; c2 < sh.hi; c2 += sh.step) {
         auto P = [&](int j) { return z[j] + beta * pold[j]; };
         const double qi = th_row(g, kx, kz, diag[c2], k, l, c2, P);
         const double pi = P(c2);
         pnew[c2] = pi;
         q[c2] = qi;
-        pq = pi * qi;
-    }
-    const double t = block_sum(pq, s);
-    if (threadIdx.x == 0) part[blk] = t;
-}
-
-__global__ void __launch_bounds__(TB) k_th_fin1(int nb, const double *__restrict__ part, th_ctl *ctl) {
-    if (ctl->done) return;
-    __shared__ double s[TB];
-    const double pq = sum_parts(nb, part, s);
-    if (threadIdx.x == 0) {
-        if (fabs(pq) < 1e-30) {
-            ctl->its = -2;
-            ctl->done = 1;
-        } else {
-            ctl->alpha = ctl->rz / pq;
+        pq += pi * qi;
+        k += dk;
+        l += dl;
+        if (k >= g.ncx) {
+            k -= g.ncx;
+            l++;
         }
     }
+    t = block_sum2(pq, 0.0, s);
+    if (threadIdx.x == 0) part_pq[blockIdx.x] = t.a;
 }
 
 __global__ void __launch_bounds__(TB) k_th_update(int n, const double *__restrict__ p, const double *__restrict__ q,
                                                   const double *__restrict__ minv, double *__restrict__ x,
-                                                  double *__restrict__ r, double *__restrict__ z,
-                                                  double *__restrict__ part_rr, double *__restrict__ part_rz,
-                                                  const th_ctl *__restrict__ ctl) {
-    if (ctl->done) return;
-    __shared__ double s[TB];
-    const double alpha = ctl->alpha;
-    const int blk = xcd_block(blockIdx.x, gridDim.x);
-    const int i = blk * TB + threadIdx.x;
+                                                  double *__restrict__ r, double *__restrict__ z, int nb,
+                                                  const double *__restrict__ part_pq, double *__restrict__ part_rr,
+                                                  double *__restrict__ part_rz, th_ctl *ctl) {
+    __shared__ double s[TB / 64][2];
+    const double pq = part_sum2(nb, part_pq, nullptr, s).a;
+    th_ctl c = ctl[1];
+    if (!c.done) {
+        if (fabs(pq) < 1e-30) {
+            c.its = -2;
+            c.done = 1;
+        } else {
+            c.alpha = c.rz / pq;
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl[0] = c;
+    if (c.done) return;
+    const th_share sh = th_cells(n);
+    const double alpha = c.alpha;
     double rr = 0.0, rz = 0.0;
-    if (i < n) {
+    for (int i = sh.lo + threadIdx.x; i < sh.hi; i += sh.step) {
         x[i] += alpha * p[i];
         const double ri = r[i] - alpha * q[i];
         r[i] = ri;
         const double zi = minv[i] * ri;
         z[i] = zi;
-        rr = ri * ri;
-        rz = ri * zi;
+        rr += ri * ri;
+        rz += ri * zi;
     }
-    const double a = block_sum(rr, s);
-    __syncthreads();
-    const double b = block_sum(rz, s);
+    const sum2 t = block_sum2(rr, rz, s);
     if (threadIdx.x == 0) {
-        part_rr[blk] = a;
-        part_rz[blk] = b;
+        part_rr[blockIdx.x] = t.a;
+        part_rz[blockIdx.x] = t.b;
     }
 }
 
-__global__ void __launch_bounds__(TB) k_th_fin2(int nb, const double *__restrict__ part_rr,
-                                                const double *__restrict__ part_rz, th_ctl *ctl) {
-    if (ctl->done) return;
-    __shared__ double s[TB];
-    const double rr = sum_parts(nb, part_rr, s);
-    __syncthreads();
-    const double rzn = sum_parts(nb, part_rz, s);
+// What the next apply would decide, for the host: the state with that test
+// taken, the ratio ||r|| / ||r0|| in beta.
+__global__ void __launch_bounds__(TB) k_th_test(int nb, const double *__restrict__ part_rr, const th_ctl *__restrict__ ctl,
+                                                th_ctl *__restrict__ out) {
+    __shared__ double s[TB / 64][2];
+    th_ctl c = ctl[0];
+    const double rr = part_sum2(nb, part_rr, nullptr, s).a;
     if (threadIdx.x == 0) {
-        const int it = ctl->it + 1;
-        ctl->it = it;
-        if (sqrt(rr) / ctl->r0 < ctl->rel_tol) {
-            ctl->its = it;
-            ctl->done = 1;
-        } else if (fabs(ctl->rz) < 1e-30) {
-            ctl->its = -3;
-            ctl->done = 1;
-        } else {
-            ctl->beta = rzn / ctl->rz;
-            ctl->rz = rzn;
-            if (it >= ctl->max_its) ctl->done = 1;   // its stays -1
+        if (!c.done) {
+            c.it++;
+            c.beta = sqrt(rr) / c.r0;
+            if (c.beta < c.rel_tol) {
+                c.its = c.it;
+                c.done = 1;
+            } else if (fabs(c.rz) < 1e-30) {
+                c.its = -3;
+                c.done = 1;
+            } else if (c.it >= c.max_its) {
+                c.done = 1;
+            }
         }
+        *out = c;
     }
 }
 
@@ -262,7 +328,7 @@ __global__ void __launch_bounds__(TB) k_th_fin2(int nb, const double *__restrict
 struct thermal_scratch {
     dbuf<double> in[8];   // staged inputs: rho, Cp, Qr, Wdiss, Ha, kx, kz, BCT_v
     dbuf<signed char> bt;
-    dbuf<double> x, diag, minv, r, z, p[2], q, part[2];
+    dbuf<double> x, diag, minv, r, z, p[2], q, part[3];
     dbuf<th_ctl> ctl;
 };
 
@@ -271,7 +337,7 @@ void mdg_thermal_release(mdg_ctx *c) {
     thermal_scratch *s = c->thermal;
     for (auto &b : s->in) b.release();
     s->bt.release(); s->x.release(); s->diag.release(); s->minv.release(); s->r.release(); s->z.release();
-    s->p[0].release(); s->p[1].release(); s->q.release(); s->part[0].release(); s->part[1].release();
+    s->p[0].release(); s->p[1].release(); s->q.release(); s->part[0].release(); s->part[1].release(); s->part[2].release();
     s->ctl.release();
     delete s;
     c->thermal = nullptr;
@@ -306,11 +372,12 @@ extern "C" int mdg_energy_step(mdg_ctx *c, double dt, const double *rho_n, const
         HIPCHK(c, hipMemcpyAsync(s.x.p, T, (size_t)n * 8, hipMemcpyHostToDevice, c->stream));
         x = s.x.p;
     }
-    const int nb = mdg_grid1d(n, TB);
+    const int nb = std::min(TH_BLOCKS, mdg_grid1d(n, TB));
     HIPCHK(c, s.diag.reserve(n)); HIPCHK(c, s.minv.reserve(n)); HIPCHK(c, s.r.reserve(n));
     HIPCHK(c, s.z.reserve(n)); HIPCHK(c, s.p[0].reserve(n)); HIPCHK(c, s.p[1].reserve(n));
-    HIPCHK(c, s.q.reserve(n)); HIPCHK(c, s.part[0].reserve(nb)); HIPCHK(c, s.part[1].reserve(nb));
-    HIPCHK(c, s.ctl.reserve(1));
+    HIPCHK(c, s.q.reserve(n));
+    for (auto &p : s.part) HIPCHK(c, p.reserve(nb));
+    HIPCHK(c, s.ctl.reserve(3));
     th_ctl h{};
     h.rel_tol = rel_tol;
     h.max_its = max_its;
@@ -318,11 +385,11 @@ extern "C" int mdg_energy_step(mdg_ctx *c, double dt, const double *rho_n, const
     h.its = -1;
     HIPCHK(c, hipMemcpyAsync(s.ctl.p, &h, sizeof h, hipMemcpyHostToDevice, c->stream));
     const th_geom g{ncx, ncz, c->Nx, c->Nx + 1, 1.0 / (c->dx * c->dx), 1.0 / (c->dz * c->dz), c->dx};
+    double *rr = s.part[0].p, *rz = s.part[1].p, *pq = s.part[2].p;
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     hipLaunchKernelGGL(k_th_setup, dim3(nb), dim3(TB), 0, c->stream, g, dt, in, (const double *)x, s.diag.p,
-                       s.minv.p, s.r.p, s.z.p, s.p[0].p, s.part[0].p, s.part[1].p);
-    hipLaunchKernelGGL(k_th_fin0, dim3(1), dim3(TB), 0, c->stream, nb, (const double *)s.part[0].p,
-                       (const double *)s.part[1].p, s.ctl.p);
+                       s.minv.p, s.r.p, s.z.p, s.p[0].p, rr, rz);
+    hipLaunchKernelGGL(k_th_start, dim3(1), dim3(TB), 0, c->stream, nb, (const double *)rr, (const double *)rz, s.ctl.p);
     HIPCHK(c, hipGetLastError());
     // With max_its = 0 the reference's loop does not run: its = -1 unless
     // the start already has a zero residual.
@@ -334,24 +401,26 @@ extern "C" int mdg_energy_step(mdg_ctx *c, double dt, const double *rho_n, const
     while (launched < max_its) {
         const int m = std::min(batch, max_its - launched);
         for (int i = 0; i < m; i++) {
-            hipLaunchKernelGGL(k_th_apply, dim3(nb), dim3(TB), 0, c->stream, g, in.kx, in.kz,
+            const bool first = launched + i == 0;
+            hipLaunchKernelGGL(first ? k_th_apply<true> : k_th_apply<false>, dim3(nb), dim3(TB), 0, c->stream, g, in.kx, in.kz,
                                (const double *)s.diag.p, (const double *)s.z.p, (const double *)s.p[cur].p,
-                               s.p[cur ^ 1].p, s.q.p, s.part[0].p, (const th_ctl *)s.ctl.p);
-            hipLaunchKernelGGL(k_th_fin1, dim3(1), dim3(TB), 0, c->stream, nb, (const double *)s.part[0].p,
-                               s.ctl.p);
+                               s.p[cur ^ 1].p, s.q.p, nb, (const double *)rr, (const double *)rz, pq, s.ctl.p);
             hipLaunchKernelGGL(k_th_update, dim3(nb), dim3(TB), 0, c->stream, n, (const double *)s.p[cur ^ 1].p,
-                               (const double *)s.q.p, (const double *)s.minv.p, x, s.r.p, s.z.p, s.part[0].p,
-                               s.part[1].p, (const th_ctl *)s.ctl.p);
-            hipLaunchKernelGGL(k_th_fin2, dim3(1), dim3(TB), 0, c->stream, nb, (const double *)s.part[0].p,
-                               (const double *)s.part[1].p, s.ctl.p);
+                               (const double *)s.q.p, (const double *)s.minv.p, x, s.r.p, s.z.p, nb, (const double *)pq, rr, rz,
+                               s.ctl.p);
             cur ^= 1;
         }
+        hipLaunchKernelGGL(k_th_test, dim3(1), dim3(TB), 0, c->stream, nb, (const double *)rr, (const th_ctl *)s.ctl.p,
+                           s.ctl.p + 2);
         HIPCHK(c, hipGetLastError());
         launched += m;
-        HIPCHK(c, hipMemcpyAsync(&h, s.ctl.p, sizeof h, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipMemcpyAsync(&h, s.ctl.p + 2, sizeof h, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         if (h.done) break;
-        batch = std::min(batch * 2, 128);
+        // the next batch: as many as the mean rate so far still needs (an
+        // iteration too many costs two empty launches, one too few a round trip)
+        const double left = h.beta < 1.0 ? launched * (std::log(rel_tol) / std::log(h.beta) - 1.0) : batch;
+        batch = (int)std::min(128.0, std::max(8.0, 1.02 * left + 1.0));
     }
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     if (x != T) HIPCHK(c, hipMemcpyAsync(T, x, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
