@@ -16,14 +16,26 @@
 // is one 8-byte load.
 //
 // Convolution as implicit GEMM: a wavefront owns 64 consecutive pixels of a
-// row (M, four 16-pixel tiles) and all output channels (N = 16*NT); K =
-// 9*Cin runs in chunks of 32, each lane reading two groups of 4 consecutive
-// channels (8 bytes each, NHWC, from the workgroup's LDS tile; each group of
-// one tap, as Cin is a multiple of 4).  Lane l holds
-// A[l%16][8(l/16)..+7], B[8(l/16)..+7][l%16] and receives
+// row (M, four 16-pixel tiles) and 16*NT output channels (N); K = 9*Cin runs
+// in chunks of 32, each lane reading 8 consecutive channels of one tap (4 of
+// two taps for the 4-channel layers) from the workgroup's LDS tile.  Lane l
+// holds A[l%16][8(l/16)..+7], B[8(l/16)..+7][l%16] and receives
 // D[4(l/16)+i][l%16].  The weight gradient is the GEMM over pixels
-// dW[k][co] = sum_p X[p + off(k)][ci(k)] dZ[p][co], split over pixel chunks
+// dW[k][co] = sum_p X[p + off(k)][ci(k)] dZ[p][co], split over pixel tiles
 // whose partial sums are added in a fixed order (no atomics).
+//
+// Bound: latency.  A 256 x 256 gradient is 3.6 GFLOP (3 us of the matrix
+// cores) in about 40 dependent launches of a few microseconds, so every
+// kernel keeps its chain of memory round trips short: the channel count is a
+// template parameter and the K loop unrolled, weights are fetched CT_PF
+// chunks ahead, the small levels spread their output channels over blocks,
+// and the weight gradient stages its operands pixel-major in LDS.
+// Measured, 256 x 256 gradient: 1.46 -> 0.40 ms per call. k_conv_wgrad
+// 91 -> 9-20 us per layer (it read single channels at pixel stride),
+// k_conv3x3 13-22 -> 7-11 us, the bias gradients' two launches folded into
+// those of the weights, the loss normaliser summed on the device.
+#include <type_traits>
+
 #include "mdg_internal.h"
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
@@ -37,7 +49,6 @@ constexpr int NL = 7;
 constexpr int L_CIN[NL] = {4, 32, 32, 64, 64, 32, 32};
 constexpr int L_COUT[NL] = {32, 32, 64, 64, 32, 32, 3};
 constexpr int L_LEVEL[NL] = {0, 1, 2, 3, 2, 1, 0};
-constexpr int WG_CHUNK = 1024;   // pixels per weight-gradient partial
 
 __host__ __device__ inline int rup(int a, int m) { return (a + m - 1) / m * m; }
 
@@ -54,79 +65,107 @@ __device__ __forceinline__ bf16x8 pack8(bf16x4 lo, bf16x4 hi) {
     return __builtin_bit_cast(bf16x8, v);
 }
 
-// y = conv3x3(x) + bias (optional ReLU).  x: H*W*Cs_in (bf16 or fp32),
-// Wt: (16*NT) x Kp bf16, out: H*W*Cs_out (bf16 or fp32), channels < Cout.
-// A workgroup owns CT_H rows of CT_W pixels: it stages the rows and columns
-// the 3 x 3 taps reach (one pixel of halo, zero outside the image), all
-// input channels, once into LDS as bf16 (pixel stride Cs_in + 4 elements,
-// so the 16 pixels of an MFMA fragment fall on distinct banks); each wave
-// then computes one row as 4 M tiles of 16 pixels, every B fragment (one
-// 16-byte load per lane) feeding 4 MFMAs.
+// y = conv3x3(x) + bias (optional ReLU).  x: H*W*CS (bf16 or fp32),
+// Wt: (16*NT*gridDim.z) x Kp bf16, out: H*W*Cs_out (bf16 or fp32), channels
+// < Cout.  A workgroup owns CT_H rows of CT_W pixels and the 16*NT output
+// channels of its blockIdx.z: it stages the rows and columns the 3 x 3 taps
+// reach (one pixel of halo, zero outside the image), all input channels, once
+// into LDS as bf16 (pixel stride CS + 8 elements: 16-byte reads of the 16
+// pixels of an MFMA fragment fall on distinct banks); each wave then computes
+// one row as 4 M tiles of 16 pixels, every B fragment (one 16-byte load per
+// lane, CT_PF chunks ahead) feeding 4 MFMAs.
 #define CT_H 4
 #define CT_W 64
-template <int NT, bool IN_F32, bool RELU, bool OUT_F32>
+#define CT_PF 4
+#define CT_LD 8
+template <int CS, int NT, bool IN_F32, bool RELU, bool OUT_F32>
 __global__ void __launch_bounds__(256)
-k_conv3x3(int H, int W, int Cs_in, int Kp, int Cout, int Cs_out, const void *__restrict__ in,
-          const bf16_t *__restrict__ Wt, const float *__restrict__ bias, void *__restrict__ out) {
-    extern __shared__ bf16_t tile[];
-    const int CS = Cs_in + 4, TW = CT_W + 2;
+k_conv3x3(int H, int W, int Cout, int Cs_out, const void *__restrict__ in, const bf16_t *__restrict__ Wt,
+          const float *__restrict__ bias, void *__restrict__ out) {
+    constexpr int K = 9 * CS, Kp = (K + 31) / 32 * 32, NK = Kp / 32;
+    constexpr int LS = CS >= 8 ? CS + 8 : CS, TW = CT_W + 2, CQ = CS / 4;
+    __shared__ __align__(16) bf16_t tile[(CT_H + 2) * TW * LS];
     const int x0 = blockIdx.x * CT_W, y0 = blockIdx.y * CT_H;
-    const int t = threadIdx.x;
-    const int cq = Cs_in >> 2;                          // 4-channel groups per pixel
-    const int nel = (CT_H + 2) * TW * cq;
-    for (int e = t; e < nel; e += 256) {
-        const int q = e % cq, pix = e / cq, lx = pix % TW, ly = pix / TW;
-        const int gx = x0 + lx - 1, gy = y0 + ly - 1;
-        bf16x4 v = {0, 0, 0, 0};
-        if (gx >= 0 && gx < W && gy >= 0 && gy < H) {
-            const long off = ((long)gy * W + gx) * Cs_in + 4 * q;
-            if (IN_F32) {
-                const float4 f = *(const float4 *)((const float *)in + off);
-                v = bf16x4{(short)f2bf(f.x), (short)f2bf(f.y), (short)f2bf(f.z), (short)f2bf(f.w)};
-            } else {
-                v = *(const bf16x4 *)((const bf16_t *)in + off);
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, m = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.z * 16 * NT;
+    const bf16_t *wp = Wt + (long)(n0 + m) * Kp + 8 * g;
+    bf16x8 bw[CT_PF][NT];
+#pragma unroll
+    for (int q = 0; q < CT_PF && q < NK; q++)
+#pragma unroll
+        for (int n = 0; n < NT; n++) bw[q][n] = *(const bf16x8 *)(wp + (long)n * 16 * Kp + 32 * q);
+    // the tile, CT_LD loads of a thread in flight at a time
+    constexpr int NIT = ((CT_H + 2) * TW * CQ + 255) / 256;
+#pragma unroll
+    for (int i0 = 0; i0 < NIT; i0 += CT_LD) {
+        typename std::conditional<IN_F32, float4, bf16x4>::type v[CT_LD];
+#pragma unroll
+        for (int i = 0; i < CT_LD; i++) {
+            const int e = t + (i0 + i) * 256, q = e % CQ, pix = e / CQ, lx = pix % TW, ly = pix / TW;
+            const int gx = x0 + lx - 1, gy = y0 + ly - 1;
+            v[i] = {};
+            if (i0 + i < NIT && ly < CT_H + 2 && gx >= 0 && gx < W && gy >= 0 && gy < H) {
+                const long off = ((long)gy * W + gx) * CS + 4 * q;
+                if constexpr (IN_F32) v[i] = *(const float4 *)((const float *)in + off);
+                else v[i] = *(const bf16x4 *)((const bf16_t *)in + off);
             }
         }
-        *(bf16x4 *)(tile + (ly * TW + lx) * CS + 4 * q) = v;
+#pragma unroll
+        for (int i = 0; i < CT_LD; i++) {
+            const int e = t + (i0 + i) * 256, q = e % CQ, pix = e / CQ;
+            if (i0 + i >= NIT || pix >= (CT_H + 2) * TW) continue;
+            bf16x4 o;
+            if constexpr (IN_F32) o = bf16x4{(short)f2bf(v[i].x), (short)f2bf(v[i].y), (short)f2bf(v[i].z), (short)f2bf(v[i].w)};
+            else o = v[i];
+            *(bf16x4 *)(tile + pix * LS + 4 * q) = o;
+        }
     }
     __syncthreads();
-    const int lane = t & 63, wave = t >> 6, m = lane & 15, g = lane >> 4;
-    const int K = 9 * Cs_in;
     f32x4 acc[4][NT];
 #pragma unroll
     for (int mt = 0; mt < 4; mt++)
 #pragma unroll
         for (int n = 0; n < NT; n++) acc[mt][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int kc = 0; kc < Kp; kc += 32) {
-        bf16x8 bw[NT];
 #pragma unroll
-        for (int n = 0; n < NT; n++) bw[n] = *(const bf16x8 *)(Wt + (long)(n * 16 + m) * Kp + kc + 8 * g);
-        int base[2];
-        bool kv[2];
+    for (int kq = 0; kq < NK; kq++) {
+        bf16x8 a[4];
+        if (CS >= 8) {
+            // chunks of 32 lie within one tap
+            const int tap = 32 * kq / CS, ci = 32 * kq % CS;
+            const bf16_t *src = tile + ((wave + tap / 3) * TW + m + tap % 3) * LS + ci + 8 * g;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int k = kc + 8 * g + 4 * h;
-            kv[h] = k < K;
-            const int tap = kv[h] ? k / Cs_in : 0, ci = kv[h] ? k - tap * Cs_in : 0;
-            // tap (dy, dx) of the wave's row and of fragment pixel m, tile coordinates
-            base[h] = ((wave + tap / 3) * TW + m + tap % 3) * CS + ci;
+            for (int mt = 0; mt < 4; mt++) a[mt] = *(const bf16x8 *)(src + 16 * mt * LS);
+        } else {
+            int base[2];
+            bool kv[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int tap = 8 * kq + 2 * g + h;
+                kv[h] = tap < 9;
+                base[h] = kv[h] ? ((wave + tap / 3) * TW + m + tap % 3) * LS : 0;
+            }
+#pragma unroll
+            for (int mt = 0; mt < 4; mt++) {
+                bf16x4 ah[2];
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    ah[h] = kv[h] ? *(const bf16x4 *)(tile + base[h] + 16 * mt * LS) : bf16x4{0, 0, 0, 0};
+                a[mt] = pack8(ah[0], ah[1]);
+            }
         }
 #pragma unroll
-        for (int mt = 0; mt < 4; mt++) {
-            bf16x4 ah[2];
+        for (int n = 0; n < NT; n++) {
+            const bf16x8 w = bw[kq % CT_PF][n];
+            if (kq + CT_PF < NK) bw[kq % CT_PF][n] = *(const bf16x8 *)(wp + (long)n * 16 * Kp + 32 * (kq + CT_PF));
 #pragma unroll
-            for (int h = 0; h < 2; h++)
-                ah[h] = kv[h] ? *(const bf16x4 *)(tile + base[h] + 16 * mt * CS) : bf16x4{0, 0, 0, 0};
-            const bf16x8 a = pack8(ah[0], ah[1]);
-#pragma unroll
-            for (int n = 0; n < NT; n++) acc[mt][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bw[n], acc[mt][n], 0, 0, 0);
+            for (int mt = 0; mt < 4; mt++) acc[mt][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], w, acc[mt][n], 0, 0, 0);
         }
     }
     const int y = y0 + wave;
     if (y >= H) return;
 #pragma unroll
     for (int n = 0; n < NT; n++) {
-        const int co = n * 16 + m;
+        const int co = n0 + n * 16 + m;
         if (co >= Cout) continue;
         const float bn = bias ? bias[co] : 0.f;
 #pragma unroll
@@ -144,193 +183,287 @@ k_conv3x3(int H, int W, int Cs_in, int Kp, int Cout, int Cs_out, const void *__r
     }
 }
 
-// Partial weight gradients of one pixel chunk: part[chunk][k][co16]
-// (k < Kp, co16 < 16*NTn) for one (k tile, n tile) per wavefront.
-__global__ void __launch_bounds__(64)
-k_conv_wgrad(int H, int W, int Cs_in, int Kp, int Cout, int Cs_g, int NTn,
-             const bf16_t *__restrict__ X, const float *__restrict__ G, float *__restrict__ part) {
-    const int lane = threadIdx.x, m = lane & 15, g = lane >> 4;
-    const int kt = blockIdx.y / NTn, nt = blockIdx.y - kt * NTn;
-    const long npix = (long)H * W;
-    const long q0 = (long)blockIdx.x * WG_CHUNK;
-    const long q1 = (q0 + WG_CHUNK < npix) ? q0 + WG_CHUNK : npix;
-    const int k = kt * 16 + m, K = 9 * Cs_in;
-    const bool kv = k < K;
-    const int tap = kv ? k / Cs_in : 0, ci = kv ? k - tap * Cs_in : 0;
-    const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-    const int n = nt * 16 + m;
-    const bool nv = n < Cout;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    // the lane's 8 consecutive pixels of each 32-pixel step start at
-    // qb + 8g; their (y, x) advance by 32 pixels a step (one division at
-    // the start, wrap-arounds after)
-    long qs = q0 + 8 * g;
-    int ys = (int)(qs / W), xs = (int)(qs - (long)ys * W);
-    for (long qb = q0; qb < q1; qb += 32) {
-        bf16x4 a4[2], b4[2];
-        int y = ys, x = xs;
+// Weight and bias gradients of the pixel tiles blockIdx.x, + gridDim.x, ...
+// for the taps of row dy = blockIdx.y - 1: part[block][k][co] (k = tap*CS +
+// ci, 16*NT columns) and, from the dy = 0 blocks, bpart[block][co].
+// A tile is WG_PIX pixels, TW = 2^ltw wide.  Both operands of the GEMM over
+// pixels want 8 consecutive pixels of one channel per lane, so the tile is
+// turned in LDS: dZ as [co][pixel], X (the image row dy below or above) as
+// [dx][ci][pixel], one copy per dx shift so that every fragment is one aligned
+// 16-byte read (row stride WG_PIX + 8 elements: the 16 rows of a fragment fall
+// on distinct banks).  The 3*CS rows (dx, ci) are dealt to the four waves in
+// tiles of 16.  The bias sums the unrounded gradient values.
+#define WG_PIX 128
+#define WG_BLOCKS 512   // pixel blocks (partials) at most
+template <int CS, int NT>
+__global__ void __launch_bounds__(256)
+k_conv_wgrad(int H, int W, int ltw, int ntx, int ntiles, int Cout, int Cs_g, const bf16_t *__restrict__ X,
+             const float *__restrict__ G, float *__restrict__ part, float *__restrict__ bpart) {
+    constexpr int PS = WG_PIX + 8, ROWS = 3 * CS, NA = (ROWS + 15) / 16, AW = (NA + 3) / 4;
+    constexpr int XV = CS >= 8 ? 8 : 4, XQ = CS / XV;
+    __shared__ __align__(16) bf16_t xs[NA * 16 * PS];
+    __shared__ __align__(16) bf16_t gs[NT * 16 * PS];
+    __shared__ float bs[256][4];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, m = lane & 15, g = lane >> 4;
+    const int dy = (int)blockIdx.y - 1, TW = 1 << ltw, R = WG_PIX >> ltw;
+    const int gq = Cs_g >> 2;                 // 4-channel groups of dZ (1, 8 or 16)
+    // rows that no load below fills stay zero
+    for (int e = t; e < NA * 16 * PS; e += 256) xs[e] = 0;
+    for (int e = t; e < NT * 16 * PS; e += 256) gs[e] = 0;
+    f32x4 acc[AW][NT];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const long q = qb + 8 * g + j;
-            bf16_t av = 0, bv = 0;
-            if (q < q1) {
-                if (kv) {
-                    const int yy = y + dy, xx = x + dx;
-                    if (yy >= 0 && yy < H && xx >= 0 && xx < W) av = X[((long)yy * W + xx) * Cs_in + ci];
-                }
-                if (nv) bv = f2bf(G[q * Cs_g + n]);
+    for (int a = 0; a < AW; a++)
+#pragma unroll
+        for (int n = 0; n < NT; n++) acc[a][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float b4[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int ty = tile / ntx, x0 = (tile - ty * ntx) * TW, y0 = ty * R;
+        __syncthreads();                      // zeros written, previous tile consumed
+        // dZ: thread t keeps the channel group t % gq; 4 loads in flight
+        for (int e0 = t; e0 < WG_PIX * gq; e0 += 4 * 256) {
+            float4 f[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int e = e0 + 256 * i, q = e & (gq - 1), p = e / gq, x = x0 + (p & (TW - 1)), y = y0 + (p >> ltw);
+                f[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (p < WG_PIX && x < W && y < H) f[i] = *(const float4 *)(G + ((long)y * W + x) * Cs_g + 4 * q);
             }
-            a4[j >> 2][j & 3] = (short)av;
-            b4[j >> 2][j & 3] = (short)bv;
-            if (++x == W) { x = 0; y++; }
-        }
-        xs += 32;
-        while (xs >= W) { xs -= W; ys++; }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pack8(a4[0], a4[1]), pack8(b4[0], b4[1]), acc, 0, 0, 0);
-    }
-    const int ld = 16 * NTn;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int kk = kt * 16 + 4 * g + i;
-        part[((long)blockIdx.x * Kp + kk) * ld + n] = acc[i];
+            for (int i = 0; i < 4; i++) {
+                const int e = e0 + 256 * i, q = e & (gq - 1), p = e / gq;
+                if (p >= WG_PIX) continue;
+                b4[0] += f[i].x; b4[1] += f[i].y; b4[2] += f[i].z; b4[3] += f[i].w;
+                bf16_t *o = gs + 4 * q * PS + p;
+                o[0] = f2bf(f[i].x); o[PS] = f2bf(f[i].y); o[2 * PS] = f2bf(f[i].z); o[3 * PS] = f2bf(f[i].w);
+            }
+        }
+        // X: source columns -1 .. TW of the tile's rows shifted by dy
+        const int npx = R * (TW + 2);
+        for (int e0 = t; e0 < npx * XQ; e0 += 4 * 256) {
+            __align__(16) bf16_t v[4][XV];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int e = e0 + 256 * i, q = e / npx, pix = e - q * npx, ly = pix / (TW + 2), sx = pix - ly * (TW + 2) - 1;
+                const int x = x0 + sx, y = y0 + ly + dy;
+#pragma unroll
+                for (int j = 0; j < XV; j++) v[i][j] = 0;
+                if (q < XQ && x >= 0 && x < W && y >= 0 && y < H) {
+                    const bf16_t *src = X + ((long)y * W + x) * CS + XV * q;
+#pragma unroll
+                    for (int j = 0; j < XV; j += 4) *(bf16x4 *)(v[i] + j) = *(const bf16x4 *)(src + j);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int e = e0 + 256 * i, q = e / npx, pix = e - q * npx, ly = pix / (TW + 2), sx = pix - ly * (TW + 2) - 1;
+                if (q >= XQ) continue;
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    const int lx = sx + 1 - d;    // pixel whose tap dx = d - 1 reads this column
+                    if (lx < 0 || lx >= TW) continue;
+                    bf16_t *o = xs + (d * CS + XV * q) * PS + (ly << ltw) + lx;
+#pragma unroll
+                    for (int j = 0; j < XV; j++) o[j * PS] = v[i][j];
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int kk = 0; kk < WG_PIX / 32; kk++) {
+            bf16x8 b[NT];
+#pragma unroll
+            for (int n = 0; n < NT; n++) b[n] = *(const bf16x8 *)(gs + (n * 16 + m) * PS + 32 * kk + 8 * g);
+#pragma unroll
+            for (int a = 0; a < AW; a++) {
+                if (wave + 4 * a >= NA) continue;
+                const bf16x8 x = *(const bf16x8 *)(xs + ((wave + 4 * a) * 16 + m) * PS + 32 * kk + 8 * g);
+#pragma unroll
+                for (int n = 0; n < NT; n++) acc[a][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, b[n], acc[a][n], 0, 0, 0);
+            }
+        }
+    }
+    float *po = part + ((long)blockIdx.x * 9 * CS + blockIdx.y * ROWS) * (16 * NT);
+#pragma unroll
+    for (int a = 0; a < AW; a++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = (wave + 4 * a) * 16 + 4 * g + i;
+            if (r >= ROWS) continue;
+#pragma unroll
+            for (int n = 0; n < NT; n++) po[(long)r * (16 * NT) + n * 16 + m] = acc[a][n][i];
+        }
+    if (dy != 0) return;
+#pragma unroll
+    for (int j = 0; j < 4; j++) bs[t][j] = b4[j];
+    __syncthreads();
+    if (t < Cout) {
+        float r = 0.f;
+        for (int q = t >> 2; q < 256; q += gq) r += bs[q][t & 3];
+        bpart[(long)blockIdx.x * 64 + t] = r;
     }
 }
 
-// dW[tap][ci][co] (+)= sum over chunks.  A 256-thread block owns 16
-// consecutive weights; 16 threads per weight sum every 16th chunk and the
-// 16 partial sums are combined in LDS in a fixed order.
+// dW[tap][ci][co] (+)= sum over blocks, db[co] likewise (the last block).  A
+// 256-thread block owns 16 consecutive weights; 16 threads per weight sum
+// every 16th partial and the 16 sums are combined in LDS in a fixed order.
 __global__ void __launch_bounds__(256) k_wgrad_reduce(int nchunk, int Kp, int ld, int Cin, int Cs_in, int Cout,
-                                                      const float *__restrict__ part, float *__restrict__ dW,
-                                                      int accumulate) {
-    __shared__ float sh[16][17];
+                                                      const float *__restrict__ part, const float *__restrict__ bpart,
+                                                      float *__restrict__ dW, float *__restrict__ db, int accumulate) {
+    __shared__ float sh[256];
+    if (blockIdx.x == gridDim.x - 1) {
+        const int t = threadIdx.x, ng = 256 / Cout, co = t % Cout, pg = t / Cout;
+        float s = 0.f;
+        if (pg < ng)
+            for (int c = pg; c < nchunk; c += ng) s += bpart[(long)c * 64 + co];
+        sh[t] = s;
+        __syncthreads();
+        if (t < Cout) {
+            float r = 0.f;
+            for (int k = 0; k < ng; k++) r += sh[k * Cout + t];
+            db[t] = accumulate ? db[t] + r : r;
+        }
+        return;
+    }
     const int w = threadIdx.x & 15, j = threadIdx.x >> 4;
     const int i = blockIdx.x * 16 + w, nw = 9 * Cin * Cout;
     float s = 0.f;
     if (i < nw) {
         const int co = i % Cout, ci = (i / Cout) % Cin, tap = i / (Cout * Cin);
-        const int k = tap * Cs_in + ci;
-        for (int c = j; c < nchunk; c += 16) s += part[((long)c * Kp + k) * ld + co];
+        const float *p = part + (long)(tap * Cs_in + ci) * ld + co;
+#pragma unroll 8
+        for (int c = j; c < nchunk; c += 16) s += p[(long)c * Kp * ld];
     }
-    sh[j][w] = s;
+    sh[16 * j + w] = s;
     __syncthreads();
     if (j == 0 && i < nw) {
         float r = 0.f;
-        for (int q = 0; q < 16; q++) r += sh[q][w];
+        for (int q = 0; q < 16; q++) r += sh[16 * q + w];
         dW[i] = accumulate ? dW[i] + r : r;
     }
 }
-// Bias gradient: per-chunk channel sums, then the sum over chunks.  A
-// 256-thread block splits its pixels (or chunks) over 256 / Cout groups of
-// Cout channel threads and combines the groups in LDS in a fixed order.
-__global__ void __launch_bounds__(256) k_bias_part(long npix, int Cout, int Cs_g, const float *__restrict__ G,
-                                                   float *__restrict__ part) {
-    __shared__ float sh[256];
-    const int t = threadIdx.x, ng = 256 / Cout, co = t % Cout, pg = t / Cout;
-    const long q0 = (long)blockIdx.x * WG_CHUNK;
-    const long q1 = (q0 + WG_CHUNK < npix) ? q0 + WG_CHUNK : npix;
-    float s = 0.f;
-    if (pg < ng)
-        for (long q = q0 + pg; q < q1; q += ng) s += G[q * Cs_g + co];
-    sh[t] = s;
-    __syncthreads();
-    if (t < Cout) {
-        float r = 0.f;
-        for (int k = 0; k < ng; k++) r += sh[k * Cout + t];
-        part[(long)blockIdx.x * 64 + t] = r;
-    }
+
+// The kernels between the convolutions work on 4 consecutive channels a
+// thread (channel counts are multiples of 4; n4 = pixels * channels / 4).
+struct px4 {
+    int c4, y, x;      // channel group, row, column of element i on a W-wide image
+};
+__device__ __forceinline__ px4 px4_of(long i, int W, int C4) {
+    const long p = i / C4;
+    const int y = (int)(p / W);
+    return px4{(int)(i - p * C4), y, (int)(p - (long)y * W)};
 }
-__global__ void __launch_bounds__(256) k_bias_reduce(int nchunk, int Cout, const float *__restrict__ part,
-                                                     float *__restrict__ db, int accumulate) {
-    __shared__ float sh[256];
-    const int t = threadIdx.x, ng = 256 / Cout, co = t % Cout, pg = t / Cout;
-    float s = 0.f;
-    if (pg < ng)
-        for (int c = pg; c < nchunk; c += ng) s += part[(long)c * 64 + co];
-    sh[t] = s;
-    __syncthreads();
-    if (t < Cout) {
-        float r = 0.f;
-        for (int k = 0; k < ng; k++) r += sh[k * Cout + t];
-        db[t] = accumulate ? db[t] + r : r;
-    }
+__device__ __forceinline__ float4 ldbf4(const bf16_t *p) {
+    const bf16x4 v = *(const bf16x4 *)p;
+    return make_float4(bf2f((bf16_t)v[0]), bf2f((bf16_t)v[1]), bf2f((bf16_t)v[2]), bf2f((bf16_t)v[3]));
+}
+__device__ __forceinline__ void stbf4(bf16_t *p, float4 v) {
+    *(bf16x4 *)p = bf16x4{(short)f2bf(v.x), (short)f2bf(v.y), (short)f2bf(v.z), (short)f2bf(v.w)};
+}
+template <typename F>
+__device__ __forceinline__ float4 map4(F f, float4 a, float4 b, float4 c, float4 d) {
+    return make_float4(f(a.x, b.x, c.x, d.x), f(a.y, b.y, c.y, d.y), f(a.z, b.z, c.z, d.z), f(a.w, b.w, c.w, d.w));
 }
 
 // 2x2 mean pool (fine H x W -> H/2 x W/2), bf16 in/out, fp32 arithmetic.
-__global__ void k_pool(int Hc, int Wc, int C, int Cs, const bf16_t *__restrict__ in, bf16_t *__restrict__ out) {
+__global__ void k_pool(long n4, int Wc, int C4, const bf16_t *__restrict__ in, bf16_t *__restrict__ out) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)Hc * Wc * C) return;
-    const int c = (int)(i % C);
-    const long pc = i / C;
-    const int y = (int)(pc / Wc), x = (int)(pc - (long)y * Wc);
-    const int W = 2 * Wc;
-    const long f = ((long)(2 * y) * W + 2 * x) * Cs + c;
-    const float s = (bf2f(in[f]) + bf2f(in[f + Cs])) + (bf2f(in[f + (long)W * Cs]) + bf2f(in[f + (long)W * Cs + Cs]));
-    out[pc * Cs + c] = f2bf(s * 0.25f);
+    if (i >= n4) return;
+    const px4 e = px4_of(i, Wc, C4);
+    const long W = 2 * Wc, f = 4 * (((long)(2 * e.y) * W + 2 * e.x) * C4 + e.c4), row = 4 * W * C4;
+    stbf4(out + 4 * i, map4([](float a, float b, float c, float d) { return ((a + b) + (c + d)) * 0.25f; }, ldbf4(in + f),
+                            ldbf4(in + f + 4 * C4), ldbf4(in + f + row), ldbf4(in + f + row + 4 * C4)));
 }
 // s = bf16(fine + up(coarse)) on the fine grid.
-__global__ void k_up_add(int H, int W, int C, int Cs, const bf16_t *__restrict__ fine,
-                         const bf16_t *__restrict__ coarse, bf16_t *__restrict__ out) {
+__global__ void k_up_add(long n4, int W, int C4, const bf16_t *__restrict__ fine, const bf16_t *__restrict__ coarse,
+                         bf16_t *__restrict__ out) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)H * W * C) return;
-    const int c = (int)(i % C);
-    const long p = i / C;
-    const int y = (int)(p / W), x = (int)(p - (long)y * W);
-    const long pc = (long)(y >> 1) * (W >> 1) + (x >> 1);
-    out[p * Cs + c] = f2bf(bf2f(fine[p * Cs + c]) + bf2f(coarse[pc * Cs + c]));
+    if (i >= n4) return;
+    const px4 e = px4_of(i, W, C4);
+    const float4 a = ldbf4(fine + 4 * i);
+    const float4 b = ldbf4(coarse + 4 * (((long)(e.y >> 1) * (W >> 1) + (e.x >> 1)) * C4 + e.c4));
+    stbf4(out + 4 * i, make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w));
 }
 // out(coarse) = (sum of the 4 fine gradients) * (act > 0)
-__global__ void k_up_bwd_mask(int Hc, int Wc, int C, int Cs, const float *__restrict__ g,
-                              const bf16_t *__restrict__ act, float *__restrict__ out) {
+__global__ void k_up_bwd_mask(long n4, int Wc, int C4, const float *__restrict__ g, const bf16_t *__restrict__ act,
+                              float *__restrict__ out) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)Hc * Wc * C) return;
-    const int c = (int)(i % C);
-    const long pc = i / C;
-    const int y = (int)(pc / Wc), x = (int)(pc - (long)y * Wc);
-    const int W = 2 * Wc;
-    const long f = ((long)(2 * y) * W + 2 * x) * Cs + c;
-    const float s = (g[f] + g[f + Cs]) + (g[f + (long)W * Cs] + g[f + (long)W * Cs + Cs]);
-    out[pc * Cs + c] = bf2f(act[pc * Cs + c]) > 0.f ? s : 0.f;
+    if (i >= n4) return;
+    const px4 e = px4_of(i, Wc, C4);
+    const long W = 2 * Wc, f = 4 * (((long)(2 * e.y) * W + 2 * e.x) * C4 + e.c4), row = 4 * W * C4;
+    const float4 s = map4([](float a, float b, float c, float d) { return (a + b) + (c + d); }, *(const float4 *)(g + f),
+                          *(const float4 *)(g + f + 4 * C4), *(const float4 *)(g + f + row),
+                          *(const float4 *)(g + f + row + 4 * C4));
+    const float4 a = ldbf4(act + 4 * i);
+    *(float4 *)(out + 4 * i) = make_float4(a.x > 0.f ? s.x : 0.f, a.y > 0.f ? s.y : 0.f, a.z > 0.f ? s.z : 0.f,
+                                           a.w > 0.f ? s.w : 0.f);
 }
-// fine += coarse / 4 replicated (pool backward)
-__global__ void k_pool_bwd_acc(int H, int W, int C, int Cs, const float *__restrict__ coarse, float *__restrict__ fine) {
+// fine = (fine + coarse / 4 replicated) * (act > 0): pool and ReLU backward
+__global__ void k_pool_bwd_mask(long n4, int W, int C4, const float *__restrict__ coarse, const bf16_t *__restrict__ act,
+                                float *__restrict__ fine) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)H * W * C) return;
-    const int c = (int)(i % C);
-    const long p = i / C;
-    const int y = (int)(p / W), x = (int)(p - (long)y * W);
-    const long pc = (long)(y >> 1) * (W >> 1) + (x >> 1);
-    fine[p * Cs + c] += coarse[pc * Cs + c] * 0.25f;
+    if (i >= n4) return;
+    const px4 e = px4_of(i, W, C4);
+    const float4 c = *(const float4 *)(coarse + 4 * (((long)(e.y >> 1) * (W >> 1) + (e.x >> 1)) * C4 + e.c4));
+    const float4 f = *(const float4 *)(fine + 4 * i), a = ldbf4(act + 4 * i);
+    *(float4 *)(fine + 4 * i) =
+        make_float4(a.x > 0.f ? f.x + c.x * 0.25f : 0.f, a.y > 0.f ? f.y + c.y * 0.25f : 0.f,
+                    a.z > 0.f ? f.z + c.z * 0.25f : 0.f, a.w > 0.f ? f.w + c.w * 0.25f : 0.f);
 }
-__global__ void k_mask_mul(long n, int C, int Cs, float *__restrict__ g, const bf16_t *__restrict__ act) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n * C) return;
-    const long o = (i / C) * Cs + i % C;
-    if (!(bf2f(act[o]) > 0.f)) g[o] = 0.f;
-}
-// 0.5 * sum(mask (y - t)^2) / sum(mask) partials; dy = mask (y - t) / sum(mask)
-__global__ void __launch_bounds__(256)
-k_loss(long n4, const float *__restrict__ y, const float *__restrict__ t, const float *__restrict__ mask,
-       float inv_cnt, float *__restrict__ dy, double *__restrict__ part) {
-    __shared__ double s[256];
-    double acc = 0.0;
-    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n4; i += (long)gridDim.x * 256) {
-        const float d = (i % 4 < 3) ? mask[i] * (y[i] - t[i]) : 0.f;
-        dy[i] = d * inv_cnt;
-        acc += 0.5 * (double)d * (double)d;
-    }
-    s[threadIdx.x] = acc;
+
+// Four floats of a caller's image, aligned to a float only.
+struct __attribute__((packed, aligned(4))) f4u {
+    float x, y, z, w;
+};
+__device__ __forceinline__ f4u ldu4(const float *p) { return *(const f4u *)p; }
+
+// Sum over the 256 threads of a block, in every thread.
+__device__ inline double block_sum256(double v, double *s) {
+    s[threadIdx.x] = v;
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
         if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = s[0];
+    const double r = s[0];
+    __syncthreads();
+    return r;
 }
-__global__ void k_sum_partials(int n, const double *__restrict__ part, double scale, double *__restrict__ out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double s = 0.0;
-    for (int i = 0; i < n; i++) s += part[i];
-    *out = s * scale;
+#define LOSS_BLOCKS 256
+__device__ inline double at_least_one(double n) { return n < 1.0 ? 1.0 : n; }
+// Partial sums of the mask over channels 0..2 (the loss normaliser).
+__global__ void __launch_bounds__(256) k_mask_count(long npix, const float *__restrict__ mask, double *__restrict__ cpart) {
+    __shared__ double s[256];
+    double acc = 0.0;
+    for (long p = (long)blockIdx.x * 256 + threadIdx.x; p < npix; p += (long)gridDim.x * 256) {
+        const f4u v = ldu4(mask + 4 * p);
+        acc += (double)v.x + (double)v.y + (double)v.z;
+    }
+    const double r = block_sum256(acc, s);
+    if (threadIdx.x == 0) cpart[blockIdx.x] = r;
+}
+// 0.5 * sum(mask (y - t)^2) partials; dy = mask (y - t) / sum(mask).  Every
+// block sums the LOSS_BLOCKS mask partials itself, in one fixed order.
+__global__ void __launch_bounds__(256)
+k_loss(long npix, const float *__restrict__ y, const float *__restrict__ t, const float *__restrict__ mask,
+       const double *__restrict__ cpart, float *__restrict__ dy, double *__restrict__ part) {
+    __shared__ double s[256];
+    const float inv_cnt = (float)(1.0 / at_least_one(block_sum256(cpart[threadIdx.x], s)));
+    double acc = 0.0;
+    for (long p = (long)blockIdx.x * 256 + threadIdx.x; p < npix; p += (long)gridDim.x * 256) {
+        const float4 a = *(const float4 *)(y + 4 * p);
+        const f4u b = ldu4(t + 4 * p), k = ldu4(mask + 4 * p);
+        const float d0 = k.x * (a.x - b.x), d1 = k.y * (a.y - b.y), d2 = k.z * (a.z - b.z);
+        *(float4 *)(dy + 4 * p) = make_float4(d0 * inv_cnt, d1 * inv_cnt, d2 * inv_cnt, 0.f);
+        acc += 0.5 * (double)d0 * (double)d0 + 0.5 * (double)d1 * (double)d1 + 0.5 * (double)d2 * (double)d2;
+    }
+    const double r = block_sum256(acc, s);
+    if (threadIdx.x == 0) part[blockIdx.x] = r;
+}
+__global__ void __launch_bounds__(256) k_loss_sum(const double *__restrict__ part, const double *__restrict__ cpart,
+                                                  double *__restrict__ out) {
+    __shared__ double s[256];
+    const double l = block_sum256(part[threadIdx.x], s), n = at_least_one(block_sum256(cpart[threadIdx.x], s));
+    if (threadIdx.x == 0) *out = l * (1.0 / n);
 }
 
 // Adam on one layer's FP32 weights and bias, then repack the BF16 copies.
@@ -452,6 +585,17 @@ struct tdesc { int lev, C; };
 const tdesc ADESC[13] = {{0, 4}, {0, 32}, {1, 32}, {1, 32}, {2, 32}, {2, 64}, {3, 64}, {3, 64},
                          {2, 64}, {2, 32}, {1, 32}, {1, 32}, {0, 32}};
 
+// Pixel tiles of the weight gradient: as wide as the image allows up to 64
+// (a level narrower than 64 would leave most of a wider tile empty).
+struct wg_tiles {
+    int ltw, ntx, n, blocks;
+};
+wg_tiles wgrad_tiles(int H, int W) {
+    const int ltw = W > 32 ? 6 : (W > 16 ? 5 : 4), R = WG_PIX >> ltw;
+    const int ntx = (W + (1 << ltw) - 1) >> ltw, n = ntx * ((H + R - 1) / R);
+    return wg_tiles{ltw, ntx, n, std::min(n, WG_BLOCKS)};
+}
+
 int ensure_buffers(mdg_ctx *c, pcnet_state *s, int H, int W) {
     if (H == s->H && W == s->W) return MDG_OK;
     long off = 0;
@@ -480,11 +624,8 @@ int ensure_buffers(mdg_ctx *c, pcnet_state *s, int H, int W) {
     long maxpart = 0;
     for (int k = 0; k < NL; k++) {
         const pc_layer &l = s->L[k];
-        const long np = (long)(H >> l.level) * (W >> l.level);
-        const long nch = (np + WG_CHUNK - 1) / WG_CHUNK;
-        const long need = nch * l.kpf * 16 * l.ntf;
-        if (need > maxpart) maxpart = need;
-        if (nch * 64 > maxpart) maxpart = nch * 64;
+        const wg_tiles w = wgrad_tiles(H >> l.level, W >> l.level);
+        maxpart = std::max(maxpart, (long)w.blocks * (9L * l.csi * 16 * l.ntf + 64));
     }
     HIPCHK(c, s->part.reserve(maxpart));
     HIPCHK(c, s->lpart.reserve(1024));
@@ -497,13 +638,27 @@ int ensure_buffers(mdg_ctx *c, pcnet_state *s, int H, int W) {
 bf16_t *A(pcnet_state *s, int a) { return s->act.p + s->aoff[a]; }
 float *Gb(pcnet_state *s, int i) { return s->gbuf.p + s->goff[i]; }
 
-template <int NT, bool IN_F32, bool RELU, bool OUT_F32>
-void conv_launch(mdg_ctx *c, int H, int W, int Cs_in, int Kp, int Cout, int Cs_out, const void *in,
-                 const bf16_t *Wt, const float *bias, void *out) {
+// NTOT 16-channel output tiles: all in one block where the image alone gives
+// CONV_BLOCKS of them (one per CU), else as few per block as it takes (a
+// 64-channel layer on 32 x 32 pixels is 8 blocks whole, 32 split).
+#define CONV_BLOCKS 256
+template <int CS, int NTOT, bool IN_F32, bool RELU, bool OUT_F32>
+void conv_launch(mdg_ctx *c, int H, int W, int Cout, int Cs_out, const void *in, const bf16_t *Wt, const float *bias,
+                 void *out) {
     const dim3 grid((W + CT_W - 1) / CT_W, (H + CT_H - 1) / CT_H);
-    const size_t lds = (size_t)(CT_H + 2) * (CT_W + 2) * (Cs_in + 4) * sizeof(bf16_t);
-    hipLaunchKernelGGL((k_conv3x3<NT, IN_F32, RELU, OUT_F32>), grid, dim3(256), lds, c->stream, H, W,
-                       Cs_in, Kp, Cout, Cs_out, in, Wt, bias, out);
+    const long nb = (long)grid.x * grid.y;
+    auto go = [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
+        hipLaunchKernelGGL((k_conv3x3<CS, NT, IN_F32, RELU, OUT_F32>), dim3(grid.x, grid.y, NTOT / NT), dim3(256), 0, c->stream,
+                           H, W, Cout, Cs_out, in, Wt, bias, out);
+    };
+    if constexpr (NTOT == 4) {
+        if (nb >= CONV_BLOCKS) return go(std::integral_constant<int, 4>());
+    }
+    if constexpr (NTOT >= 2) {
+        if (nb * (NTOT / 2) >= CONV_BLOCKS) return go(std::integral_constant<int, 2>());
+    }
+    go(std::integral_constant<int, 1>());
 }
 
 // forward convolution of layer k: bf16 input, bf16 (ReLU) or fp32 output
@@ -512,10 +667,13 @@ void conv_fwd(mdg_ctx *c, pcnet_state *s, int k, const bf16_t *in, void *out) {
     const int H = s->H >> l.level, W = s->W >> l.level;
     const bf16_t *Wt = s->Wf.p + s->wf_off[k];
     const float *b = s->P.p + l.boff;
-    if (k == NL - 1) { conv_launch<1, false, false, true>(c, H, W, l.csi, l.kpf, l.cout, l.cso, in, Wt, b, out); return; }
-    switch (l.ntf) {
-    case 2: conv_launch<2, false, true, false>(c, H, W, l.csi, l.kpf, l.cout, l.cso, in, Wt, b, out); break;
-    default: conv_launch<4, false, true, false>(c, H, W, l.csi, l.kpf, l.cout, l.cso, in, Wt, b, out); break;
+    switch (k) {
+    case 0: conv_launch<4, 2, false, true, false>(c, H, W, l.cout, l.cso, in, Wt, b, out); break;
+    case 2: conv_launch<32, 4, false, true, false>(c, H, W, l.cout, l.cso, in, Wt, b, out); break;
+    case 3: conv_launch<64, 4, false, true, false>(c, H, W, l.cout, l.cso, in, Wt, b, out); break;
+    case 4: conv_launch<64, 2, false, true, false>(c, H, W, l.cout, l.cso, in, Wt, b, out); break;
+    case 6: conv_launch<32, 1, false, false, true>(c, H, W, l.cout, l.cso, in, Wt, b, out); break;
+    default: conv_launch<32, 2, false, true, false>(c, H, W, l.cout, l.cso, in, Wt, b, out); break;   // 1, 5
     }
 }
 
@@ -524,34 +682,53 @@ void conv_bwd_data(mdg_ctx *c, pcnet_state *s, int k, const float *dz, float *dx
     const pc_layer &l = s->L[k];
     const int H = s->H >> l.level, W = s->W >> l.level;
     const bf16_t *Wt = s->Wb.p + s->wb_off[k];
-    switch (l.ntb) {
-    case 1: conv_launch<1, true, false, true>(c, H, W, l.cso, l.kpb, l.cin, l.csi, dz, Wt, nullptr, dx); break;
-    case 2: conv_launch<2, true, false, true>(c, H, W, l.cso, l.kpb, l.cin, l.csi, dz, Wt, nullptr, dx); break;
-    default: conv_launch<4, true, false, true>(c, H, W, l.cso, l.kpb, l.cin, l.csi, dz, Wt, nullptr, dx); break;
+    switch (k) {
+    case 2: conv_launch<64, 2, true, false, true>(c, H, W, l.cin, l.csi, dz, Wt, nullptr, dx); break;
+    case 3: conv_launch<64, 4, true, false, true>(c, H, W, l.cin, l.csi, dz, Wt, nullptr, dx); break;
+    case 4: conv_launch<32, 4, true, false, true>(c, H, W, l.cin, l.csi, dz, Wt, nullptr, dx); break;
+    case 6: conv_launch<4, 2, true, false, true>(c, H, W, l.cin, l.csi, dz, Wt, nullptr, dx); break;
+    default: conv_launch<32, 2, true, false, true>(c, H, W, l.cin, l.csi, dz, Wt, nullptr, dx); break;   // 1, 5
     }
 }
 
 void conv_bwd_weights(mdg_ctx *c, pcnet_state *s, int k, const bf16_t *x, const float *dz, int accumulate) {
     const pc_layer &l = s->L[k];
     const int H = s->H >> l.level, W = s->W >> l.level;
-    const long npix = (long)H * W;
-    const int nch = (int)((npix + WG_CHUNK - 1) / WG_CHUNK);
-    hipLaunchKernelGGL(k_conv_wgrad, dim3(nch, (l.kpf / 16) * l.ntf), dim3(64), 0, c->stream, H, W, l.csi,
-                       l.kpf, l.cout, l.cso, l.ntf, x, dz, s->part.p);
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3((int)((9L * l.cin * l.cout + 15) / 16)), dim3(256), 0, c->stream, nch,
-                       l.kpf, 16 * l.ntf, l.cin, l.csi, l.cout, (const float *)s->part.p,
-                       s->G.p + l.woff, accumulate);
-    hipLaunchKernelGGL(k_bias_part, dim3(nch), dim3(256), 0, c->stream, npix, l.cout, l.cso, dz, s->part.p);
-    hipLaunchKernelGGL(k_bias_reduce, dim3(1), dim3(256), 0, c->stream, nch, l.cout, (const float *)s->part.p,
+    const wg_tiles w = wgrad_tiles(H, W);
+    const int ld = 16 * l.ntf;
+    float *part = s->part.p, *bpart = part + (long)w.blocks * 9 * l.csi * ld;
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(w.blocks, 3), dim3(256), 0, c->stream, H, W, w.ltw, w.ntx, w.n, l.cout, l.cso, x, dz, part,
+                           bpart);
+    };
+    switch (k) {
+    case 0: go(k_conv_wgrad<4, 2>); break;
+    case 2: go(k_conv_wgrad<32, 4>); break;
+    case 3: go(k_conv_wgrad<64, 4>); break;
+    case 4: go(k_conv_wgrad<64, 2>); break;
+    case 6: go(k_conv_wgrad<32, 1>); break;
+    default: go(k_conv_wgrad<32, 2>); break;   // 1, 5
+    }
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3((int)((9L * l.cin * l.cout + 15) / 16) + 1), dim3(256), 0, c->stream, w.blocks,
+                       9 * l.csi, ld, l.cin, l.csi, l.cout, (const float *)part, (const float *)bpart, s->G.p + l.woff,
                        s->G.p + l.boff, accumulate);
 }
 
 void pool_launch(mdg_ctx *c, int Hf, int Wf, int C, const bf16_t *in, bf16_t *out) {
-    const int Hc = Hf / 2, Wc = Wf / 2;
-    hipLaunchKernelGGL(k_pool, dim3(nblk256((long)Hc * Wc * C)), dim3(256), 0, c->stream, Hc, Wc, C, rup(C, 4), in, out);
+    const long n4 = (long)(Hf / 2) * (Wf / 2) * (C / 4);
+    hipLaunchKernelGGL(k_pool, dim3(nblk256(n4)), dim3(256), 0, c->stream, n4, Wf / 2, C / 4, in, out);
 }
 void up_add_launch(mdg_ctx *c, int H, int W, int C, const bf16_t *fine, const bf16_t *coarse, bf16_t *out) {
-    hipLaunchKernelGGL(k_up_add, dim3(nblk256((long)H * W * C)), dim3(256), 0, c->stream, H, W, C, rup(C, 4), fine, coarse, out);
+    const long n4 = (long)H * W * (C / 4);
+    hipLaunchKernelGGL(k_up_add, dim3(nblk256(n4)), dim3(256), 0, c->stream, n4, W, C / 4, fine, coarse, out);
+}
+void up_bwd_launch(mdg_ctx *c, int Hc, int Wc, int C, const float *g, const bf16_t *act, float *out) {
+    const long n4 = (long)Hc * Wc * (C / 4);
+    hipLaunchKernelGGL(k_up_bwd_mask, dim3(nblk256(n4)), dim3(256), 0, c->stream, n4, Wc, C / 4, g, act, out);
+}
+void pool_bwd_launch(mdg_ctx *c, int H, int W, int C, const float *coarse, const bf16_t *act, float *fine) {
+    const long n4 = (long)H * W * (C / 4);
+    hipLaunchKernelGGL(k_pool_bwd_mask, dim3(nblk256(n4)), dim3(256), 0, c->stream, n4, W, C / 4, coarse, act, fine);
 }
 
 int forward(mdg_ctx *c, pcnet_state *s) {
@@ -575,38 +752,34 @@ int forward(mdg_ctx *c, pcnet_state *s) {
 
 int backward(mdg_ctx *c, pcnet_state *s, int accumulate) {
     const int H = s->H, W = s->W;
-    float *dy = Gb(s, 0), *de0 = Gb(s, 1), *dz0 = Gb(s, 2), *de1 = Gb(s, 3), *dz1 = Gb(s, 4);
+    float *dy = Gb(s, 0), *de0 = Gb(s, 1), *de1 = Gb(s, 3), *dz1 = Gb(s, 4);
     float *de2 = Gb(s, 5), *dz2 = Gb(s, 6), *dz3 = Gb(s, 7), *dp = Gb(s, 8);
     // layer 6 (level 0): ds0 -> de0
     conv_bwd_weights(c, s, 6, A(s, A_S0), dy, accumulate);
     conv_bwd_data(c, s, 6, dy, de0);
     // layer 5 (level 1): dz5 = up_bwd(ds0) * (d1 > 0)
-    hipLaunchKernelGGL(k_up_bwd_mask, dim3(nblk256((long)(H / 2) * (W / 2) * 32)), dim3(256), 0, c->stream, H / 2, W / 2, 32, 32, (const float *)de0, (const bf16_t *)A(s, A_D1), dz1);
+    up_bwd_launch(c, H / 2, W / 2, 32, de0, A(s, A_D1), dz1);
     conv_bwd_weights(c, s, 5, A(s, A_S1), dz1, accumulate);
     conv_bwd_data(c, s, 5, dz1, de1);                      // ds1 -> de1
     // layer 4 (level 2)
-    hipLaunchKernelGGL(k_up_bwd_mask, dim3(nblk256((long)(H / 4) * (W / 4) * 32)), dim3(256), 0, c->stream, H / 4, W / 4, 32, 32, (const float *)de1, (const bf16_t *)A(s, A_D2), dz2);
+    up_bwd_launch(c, H / 4, W / 4, 32, de1, A(s, A_D2), dz2);
     conv_bwd_weights(c, s, 4, A(s, A_S2), dz2, accumulate);
     conv_bwd_data(c, s, 4, dz2, de2);                      // ds2 -> de2
     // layer 3 (level 3)
-    hipLaunchKernelGGL(k_up_bwd_mask, dim3(nblk256((long)(H / 8) * (W / 8) * 64)), dim3(256), 0, c->stream, H / 8, W / 8, 64, 64, (const float *)de2, (const bf16_t *)A(s, A_E3), dz3);
+    up_bwd_launch(c, H / 8, W / 8, 64, de2, A(s, A_E3), dz3);
     conv_bwd_weights(c, s, 3, A(s, A_P2), dz3, accumulate);
     conv_bwd_data(c, s, 3, dz3, dp);                       // dp2 (level 3, 64)
-    hipLaunchKernelGGL(k_pool_bwd_acc, dim3(nblk256((long)(H / 4) * (W / 4) * 64)), dim3(256), 0, c->stream, H / 4, W / 4, 64, 64, (const float *)dp, de2);
     // layer 2 (level 2)
-    hipLaunchKernelGGL(k_mask_mul, dim3(nblk256((long)(H / 4) * (W / 4) * 64)), dim3(256), 0, c->stream, (long)(H / 4) * (W / 4), 64, 64, de2, (const bf16_t *)A(s, A_E2));
+    pool_bwd_launch(c, H / 4, W / 4, 64, dp, A(s, A_E2), de2);
     conv_bwd_weights(c, s, 2, A(s, A_P1), de2, accumulate);
     conv_bwd_data(c, s, 2, de2, dp);                       // dp1 (level 2, 32)
-    hipLaunchKernelGGL(k_pool_bwd_acc, dim3(nblk256((long)(H / 2) * (W / 2) * 32)), dim3(256), 0, c->stream, H / 2, W / 2, 32, 32, (const float *)dp, de1);
     // layer 1 (level 1)
-    hipLaunchKernelGGL(k_mask_mul, dim3(nblk256((long)(H / 2) * (W / 2) * 32)), dim3(256), 0, c->stream, (long)(H / 2) * (W / 2), 32, 32, de1, (const bf16_t *)A(s, A_E1));
+    pool_bwd_launch(c, H / 2, W / 2, 32, dp, A(s, A_E1), de1);
     conv_bwd_weights(c, s, 1, A(s, A_P0), de1, accumulate);
     conv_bwd_data(c, s, 1, de1, dp);                       // dp0 (level 1, 32)
-    hipLaunchKernelGGL(k_pool_bwd_acc, dim3(nblk256((long)H * W * 32)), dim3(256), 0, c->stream, H, W, 32, 32, (const float *)dp, de0);
     // layer 0 (level 0)
-    hipLaunchKernelGGL(k_mask_mul, dim3(nblk256((long)H * W * 32)), dim3(256), 0, c->stream, (long)H * W, 32, 32, de0, (const bf16_t *)A(s, A_E0));
+    pool_bwd_launch(c, H, W, 32, dp, A(s, A_E0), de0);
     conv_bwd_weights(c, s, 0, A(s, A_X), de0, accumulate);
-    (void)dz0;
     HIPCHK(c, hipGetLastError());
     return MDG_OK;
 }
@@ -755,18 +928,11 @@ extern "C" int mdg_pcnet_grad(mdg_ctx *c, int H, int W, const float *x, const fl
         HIPCHK(c, hipMemcpyAsync(s->mbuf.p, mask, n4 * sizeof(float), hipMemcpyHostToDevice, c->stream));
         md = s->mbuf.p;
     }
-    // the loss normaliser (number of unmasked output values) is counted on the host side copy
-    std::vector<float> hm(n4);
-    HIPCHK(c, hipMemcpyAsync(hm.data(), md, n4 * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    double cnt = 0.0;
-    for (long i = 0; i < n4; i++)
-        if (i % 4 < 3) cnt += hm[i];
-    if (cnt < 1.0) cnt = 1.0;
-    const int nb = 256;
-    hipLaunchKernelGGL(k_loss, dim3(nb), dim3(256), 0, c->stream, n4, (const float *)s->y.p, td, md,
-                       (float)(1.0 / cnt), Gb(s, 0), s->lpart.p);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1), 0, c->stream, nb, (const double *)s->lpart.p, 1.0 / cnt, s->loss.p);
+    double *lp = s->lpart.p, *cp = lp + LOSS_BLOCKS;
+    hipLaunchKernelGGL(k_mask_count, dim3(LOSS_BLOCKS), dim3(256), 0, c->stream, n4 / 4, md, cp);
+    hipLaunchKernelGGL(k_loss, dim3(LOSS_BLOCKS), dim3(256), 0, c->stream, n4 / 4, (const float *)s->y.p, td, md,
+                       (const double *)cp, Gb(s, 0), lp);
+    hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(256), 0, c->stream, (const double *)lp, (const double *)cp, s->loss.p);
     HIPCHK(c, hipGetLastError());
     if ((rc = backward(c, s, accumulate))) return rc;
     if (loss) HIPCHK(c, hipMemcpyAsync(loss, s->loss.p, sizeof(double), hipMemcpyDeviceToHost, c->stream));
