@@ -3,6 +3,8 @@
 // Maxwell elasticity and Drucker-Prager (plast = 1) phases, shared by the
 // grid update and the tangent (Newton) coefficients.
 #pragma once
+#include <cmath>
+
 #include "mdg_internal.h"
 
 namespace rheo {
@@ -12,11 +14,61 @@ struct rheo_ctl {
     double dt, R, zeroC, min_eta, max_eta, eta_tol, Tiimin, scale_E, scale_eta, T_peierls, d_min;
 };
 
-// The creep laws active at one (node, phase) and their coefficients: strain
-// rate C T^n of each viscous law at deviatoric stress invariant T.
+// One phase as the kernels read it: the caller's record and the factors of
+// its laws that no node changes, worked out once per call on the host (the
+// kernels took four of their pow per node and phase for them).
+struct rheo_phase {
+    mdg_phase_prop m;
+    double A_pwl, f_pwl, A_lin, f_lin, A_gbs, f_gbs;   // A^(-1/n), f^(-r/n)
+    double sin_fric, cos_fric, sin_dil;
+    int    k_pwl, k_lin;      // the stress exponent where it is 1, 2 or 3, else 0
+    int    p_free, pad;       // no law's prefactor depends on the pressure
+};
+inline rheo_phase make_phase(const mdg_phase_prop &m) {
+    auto k = [](double n) { return n == 1.0 ? 1 : (n == 2.0 ? 2 : (n == 3.0 ? 3 : 0)); };
+    rheo_phase r{};
+    r.m = m;
+    r.A_pwl = std::pow(m.A_pwl, -1.0 / m.n_pwl);
+    r.f_pwl = std::pow(m.f_pwl, -m.r_pwl / m.n_pwl);
+    r.A_lin = std::pow(m.A_lin, -1.0 / m.n_lin);
+    r.f_lin = std::pow(m.f_lin, -m.r_lin / m.n_lin);
+    r.A_gbs = std::pow(m.A_gbs, -1.0 / m.n_gbs);
+    r.f_gbs = std::pow(m.f_gbs, -m.r_gbs / m.n_gbs);
+    r.sin_fric = std::sin(m.fric);
+    r.cos_fric = std::cos(m.fric);
+    r.sin_dil = std::sin(m.dil);
+    r.k_pwl = k(m.n_pwl);
+    r.k_lin = k(m.n_lin);
+    r.p_free = (!m.pwlv || m.V_pwl == 0.0) && (!m.linv || m.V_lin == 0.0) && (!m.gbsv || m.V_gbs == 0.0);
+    return r;
+}
+
+// The library's pow as a call: with its dozen copies inlined k_tangent_grid<true>
+// has 11500 instructions, past the 64 KB instruction cache, and 118 spilled
+// scalars; as calls 4500 and 60.
+__device__ __noinline__ double pow_call(double x, double y) { return pow(x, y); }
+// x^n with k the small whole value of n, or 0: products in place of the
+// library's pow (about 20 instructions instead of 200, within 1.5 ulp).
+__device__ __forceinline__ double pow_k(double x, double n, int k) {
+    if (k == 0) return pow_call(x, n);
+    double p = x;
+    if (k > 1) p *= x;
+    if (k > 2) p *= x;
+    return p;
+}
+// x^e where e may be zero (laws without that factor): exactly 1, as pow gives
+__device__ __forceinline__ double pow_or_1(double x, double e) { return e == 0.0 ? 1.0 : pow_call(x, e); }
+// exp(e) where e is zero (no melt): exactly 1
+__device__ __forceinline__ double exp_or_1(double e) { return e == 0.0 ? 1.0 : exp(e); }
+
+// The creep laws active at one (node, phase) and their coefficients, which
+// depend on temperature, pressure, grain size and melt but not on the strain
+// rate: strain rate C T^n of each viscous law at deviatoric stress invariant T.
 struct creep_laws {
-    bool   elastic, constant, dislocation, peierls, diffusion;
+    bool   elastic, constant, dislocation, peierls, diffusion, gbs;
+    int    k_pwl, k_lin;
     double eta_el, eta_cst, C_pwl, n_pwl, C_exp, nST, C_lin, n_lin, dm_lin;
+    double B_pwl, B_lin, B_gbs, B_exp;
 };
 
 // LocalIterationViscoElastic (RheologyDensity.c:152-197): Newton iterations on
@@ -24,22 +76,26 @@ struct creep_laws {
 // T = 2 eta_ve E.  The grain-boundary-sliding term of the reference is
 // C_gbs T^n_gbs with C_gbs never set (zero), so it is absent here.  Returns
 // false when the reference would exit (20 iterations, res > tol).
-__device__ inline bool local_ve(const creep_laws &L, double Eii, double &eta, double &Eii_pwl,
-                                double &Eii_exp, double &Eii_lin) {
-    const double tol = 1.0e-11;
-    for (int it = 0; it < 20; it++) {
+// The loops here end for the wave as a whole, lanes that are done masked out:
+// with a break per lane inside the tangent's loop over perturbations, hipcc 7.2
+// gave lanes that left in different trips wrong viscosities.
+__device__ __forceinline__ bool local_ve(const creep_laws &L, double Eii, double &eta, double &Eii_pwl,
+                                         double &Eii_exp, double &Eii_lin) {
+    constexpr double tol = 1.0e-11, stop = tol / 100;
+    double res = INFINITY;
+    for (int it = 0; it < 20 && __any(!(res < stop)); it++) {
+        if (res < stop) continue;
         const double Tii = 2.0 * eta * Eii;
         const double e_cst = L.constant ? Tii / 2.0 / L.eta_cst : 0.0;
-        const double e_pwl = L.dislocation ? L.C_pwl * pow(Tii, L.n_pwl) : 0.0;
-        const double e_exp = L.peierls ? L.C_exp * pow(Tii, L.nST) : 0.0;
-        const double e_lin = L.diffusion ? L.C_lin * pow(Tii, L.n_lin) * L.dm_lin : 0.0;
+        const double e_pwl = L.dislocation ? L.C_pwl * pow_k(Tii, L.n_pwl, L.k_pwl) : 0.0;
+        const double e_exp = L.peierls ? L.C_exp * pow_call(Tii, L.nST) : 0.0;
+        const double e_lin = L.diffusion ? L.C_lin * pow_k(Tii, L.n_lin, L.k_lin) * L.dm_lin : 0.0;
         Eii_pwl = e_pwl;
         Eii_exp = e_exp;
         Eii_lin = e_lin;
         const double r = Eii - (L.elastic ? 1.0 : 0.0) * Tii / (2.0 * L.eta_el) - (e_pwl + e_exp + e_lin + e_cst);
-        const double res = fabs(r / Eii);
-        if (res < tol / 100) return true;
-        if (it == 19 && res > tol) return false;
+        res = fabs(r / Eii);
+        if (res < stop) continue;
         double dfdeta = 0.0;
         if (L.elastic) dfdeta += -Eii / L.eta_el;
         if (L.peierls) dfdeta += -e_exp * L.nST / eta;
@@ -48,86 +104,105 @@ __device__ inline bool local_ve(const creep_laws &L, double Eii, double &eta, do
         if (L.constant) dfdeta += -Eii / L.eta_cst;
         eta -= r / dfdeta;
     }
-    return true;
+    return !(res > tol);
 }
 
 // Failure codes of viscosity_concise, or-ed into the caller's flag.
 constexpr int FAIL_LOCAL_ITER = 1;     // local iterations failed (reference exits, :174-177)
 constexpr int FAIL_GRAIN_SIZE = 2;     // d < d_min with m_lin > 0 (reference exits, :506-509)
 
-// ViscosityConcise (RheologyDensity.c:385-1080) for one (node, phase) with
-// grain size d and melt fraction phi: returns the dissipative viscosity;
-// etaVE, Pcorr, Eii_pl by reference.  EXT = false compiles the diffusion,
+// The strain-rate independent part of ViscosityConcise (RheologyDensity.c:
+// 457-523) for one (node, phase).  EXT = false compiles the diffusion,
 // GBS and Peierls laws and the power law's d, f, phi factors out (the
 // caller launches it when no phase uses them: the factors are then exactly
 // 1 and the laws absent, so the results are the same bits), which keeps
 // the register count, and the occupancy, of the constant + power-law case.
 template <bool EXT>
-__device__ inline double viscosity_concise(const mdg_phase_prop &m, const rheo_ctl &md, double G, double T,
-                                           double P, double d, double phi, double Exx, double Ezz, double Exz,
-                                           double fric, double C, double dil, double pref_mult, double &etaVE,
-                                           double &Pcorr, double &Eii_pl, int &fail) {
+__device__ __forceinline__ creep_laws laws_at(const rheo_phase &ph, const rheo_ctl &md, double G, double T, double P, double d,
+                                              double phi, double pref_mult, int &fail) {
+    const mdg_phase_prop &m = ph.m;
+    creep_laws L = {};
     const double dt = (md.step == 0) ? 1e100 : md.dt;
-    bool elastic = md.elastic != 0, plastic = (m.plast == 1);
-    if (md.step == 0) { elastic = false; plastic = false; }          // :483
-    const bool constant = m.cstv != 0, dislocation = m.pwlv != 0;
-    const bool peierls = EXT && m.expv != 0 && T < md.T_peierls;      // :474, before the T floor
-    const bool diffusion = EXT && m.linv != 0, gbs = EXT && m.gbsv != 0;
-    double K = 1.0 / m.beta;
+    L.elastic = md.elastic != 0 && md.step != 0;                       // :483
+    L.constant = m.cstv != 0;
+    L.dislocation = m.pwlv != 0;
+    L.peierls = EXT && m.expv != 0 && T < md.T_peierls;               // :474, before the T floor
+    L.diffusion = EXT && m.linv != 0;
+    L.gbs = EXT && m.gbsv != 0;
+    L.eta_el = (L.elastic ? G : 1e1) * dt;                            // :493
+    L.eta_cst = L.constant ? m.eta0 : 0.0;
+    L.k_pwl = ph.k_pwl;
+    L.k_lin = ph.k_lin;
+    L.n_pwl = m.n_pwl;
+    L.n_lin = m.n_lin;
+    if (T < md.zeroC) T = md.zeroC;
+    if (L.dislocation) {                                               // :501-504
+        L.B_pwl = m.pref_pwl * pref_mult * m.F_pwl * ph.A_pwl * exp((m.Q_pwl + P * m.V_pwl) / md.R / m.n_pwl / T);
+        if (EXT)
+            L.B_pwl = L.B_pwl * pow_or_1(d, m.m_pwl / m.n_pwl) * ph.f_pwl * exp_or_1(-m.a_pwl * phi / m.n_pwl);
+        L.C_pwl = L.k_pwl ? 1.0 / pow_k(2.0 * L.B_pwl, m.n_pwl, L.k_pwl) : pow_call(2.0 * L.B_pwl, -m.n_pwl);
+    }
+    L.dm_lin = 1.0;
+    if (L.diffusion) {                                                 // :505-512, d enters below
+        if (m.m_lin > 0.0 && d < md.d_min) fail |= FAIL_GRAIN_SIZE;
+        L.B_lin = m.F_lin * ph.A_lin * exp((m.Q_lin + P * m.V_lin) / md.R / m.n_lin / T) * ph.f_lin *
+                  exp_or_1(-m.a_lin * phi / m.n_lin);
+        L.C_lin = L.k_lin ? 1.0 / pow_k(2.0 * L.B_lin, m.n_lin, L.k_lin) : pow_call(2.0 * L.B_lin, -m.n_lin);
+        L.dm_lin = pow_or_1(d, -m.m_lin);
+    }
+    if (L.gbs)                                                         // :513-515
+        L.B_gbs = m.F_gbs * ph.A_gbs * exp((m.Q_gbs + P * m.V_gbs) / md.R / m.n_gbs / T) *
+                  pow_or_1(d, m.m_gbs / m.n_gbs) * ph.f_gbs * exp_or_1(-m.a_gbs * phi / m.n_gbs);
+    L.nST = m.n_exp;
+    if (L.peierls) {                                                   // :516-523
+        const double g = m.G_exp;
+        const double ST = m.Q_exp / md.R / T * 2.0 * g * (1 - g);
+        const double Arr = exp(-m.Q_exp / md.R / T * ((1.0 - g) * (1.0 - g)));
+        L.nST = ST + m.n_exp;
+        const double F_exp = pow_call(pow_call(2.0, 1.0 - ST - m.n_exp) / pow_call(sqrt(3.0), ST + m.n_exp + 1.0), 1.0 / L.nST);
+        L.B_exp = F_exp * (pow_call(g * m.S_exp, ST / L.nST) / pow_call(m.E_exp * Arr, 1.0 / L.nST));
+        L.C_exp = pow_call(2.0 * L.B_exp, -L.nST);
+    }
+    return L;
+}
+
+// ViscosityConcise (RheologyDensity.c:385-1080) for one (node, phase) with
+// the laws of laws_at: returns the dissipative viscosity; etaVE, Pcorr,
+// Eii_pl and the visco-elastic viscosity before plasticity by reference.
+// WARM starts the visco-elastic iterations from eta_ve.  fr holds sin and cos
+// of the friction angle and sin of the dilation angle.
+struct friction {
+    double sin_fric, cos_fric, sin_dil;
+};
+template <bool EXT>
+__device__ __forceinline__ double viscosity_concise(const rheo_phase &ph, const creep_laws &L, const rheo_ctl &md, double P,
+                                                    double d, double Exx, double Ezz, double Exz, const friction &fr,
+                                                    double C, double &etaVE, double &Pcorr, double &Eii_pl,
+                                                    int &fail) {
+    const mdg_phase_prop &m = ph.m;
+    const double dt = (md.step == 0) ? 1e100 : md.dt;
+    const bool plastic = m.plast == 1 && md.step != 0;                // :483
+    const double K = L.elastic ? 1.0 / m.beta : 1e10;                  // :493
+    const double sin_fric = fr.sin_fric, sin_dil = L.elastic ? fr.sin_dil : 0.0;
     const double Eyy = -(Exx + Ezz);
     double Eii = sqrt(0.5 * (Exx * Exx + Ezz * Ezz + Eyy * Eyy) + Exz * Exz);   // :457-459
     if (Eii * md.scale_E < 1e-30) Eii = 1e-30 / md.scale_E;
     Pcorr = P;
-    if (!elastic) { G = 1e1; dil = 0.0; K = 1e10; }                   // :493
-    if (T < md.zeroC) T = md.zeroC;
-    double B_pwl = 0.0, C_pwl = 0.0;
-    if (dislocation) {                                                 // :501-504
-        B_pwl = m.pref_pwl * pref_mult * m.F_pwl * pow(m.A_pwl, -1.0 / m.n_pwl) *
-                exp((m.Q_pwl + P * m.V_pwl) / md.R / m.n_pwl / T);
-        if (EXT)
-            B_pwl = B_pwl * pow(d, m.m_pwl / m.n_pwl) * pow(m.f_pwl, -m.r_pwl / m.n_pwl) *
-                    exp(-m.a_pwl * phi / m.n_pwl);
-        C_pwl = pow(2.0 * B_pwl, -m.n_pwl);
-    }
-    double B_lin = 0.0, C_lin = 0.0;
-    if (diffusion) {                                                   // :505-512, d enters below
-        if (m.m_lin > 0.0 && d < md.d_min) fail |= FAIL_GRAIN_SIZE;
-        B_lin = m.F_lin * pow(m.A_lin, -1.0 / m.n_lin) * exp((m.Q_lin + P * m.V_lin) / md.R / m.n_lin / T) *
-                pow(m.f_lin, -m.r_lin / m.n_lin) * exp(-m.a_lin * phi / m.n_lin);
-        C_lin = pow(2.0 * B_lin, -m.n_lin);
-    }
-    double B_gbs = 0.0;
-    if (gbs)                                                           // :513-515
-        B_gbs = m.F_gbs * pow(m.A_gbs, -1.0 / m.n_gbs) * exp((m.Q_gbs + P * m.V_gbs) / md.R / m.n_gbs / T) *
-                pow(d, m.m_gbs / m.n_gbs) * pow(m.f_gbs, -m.r_gbs / m.n_gbs) * exp(-m.a_gbs * phi / m.n_gbs);
-    double ST = 0.0, B_exp = 0.0, C_exp = 0.0;
-    if (peierls) {                                                     // :516-523
-        const double g = m.G_exp;
-        ST = m.Q_exp / md.R / T * 2.0 * g * (1 - g);
-        const double Arr = exp(-m.Q_exp / md.R / T * pow(1.0 - g, 2.0));
-        const double F_exp = pow(pow(2.0, 1.0 - ST - m.n_exp) / pow(sqrt(3.0), ST + m.n_exp + 1.0),
-                                 1.0 / (ST + m.n_exp));
-        B_exp = F_exp * (pow(g * m.S_exp, ST / (ST + m.n_exp)) / pow(m.E_exp * Arr, 1.0 / (ST + m.n_exp)));
-        C_exp = pow(2.0 * B_exp, -(ST + m.n_exp));
-    }
-    const double sin_fric = sin(fric), cos_fric = cos(fric), sin_dil = sin(dil);
     double Tyield = 0.0;
     if (plastic) {                                                     // :530-539
-        Tyield = C * cos_fric + P * sin_fric;
+        Tyield = C * fr.cos_fric + P * sin_fric;
         if (m.Slim < Tyield) Tyield = m.Slim;
     }
-    const double eta_el = G * dt;
-    const double eta_cst = constant ? m.eta0 : 0.0;
-    double eta_up = 1.0e100 / md.scale_eta;                            // :585-592
-    if (constant) eta_up = fmin(eta_up, eta_cst);
-    if (dislocation) eta_up = fmin(eta_up, B_pwl * pow(Eii, 1.0 / m.n_pwl - 1.0));
-    if (elastic) eta_up = fmin(eta_up, eta_el);
-    if (peierls) eta_up = fmin(eta_up, B_exp * pow(Eii, 1.0 / (ST + m.n_exp) - 1.0));
-    if (diffusion) eta_up = fmin(eta_up, B_lin * pow(Eii, 1.0 / m.n_lin - 1.0) * pow(d, m.m_lin / m.n_lin));
-    if (gbs) eta_up = fmin(eta_up, B_gbs * pow(Eii, 1.0 / m.n_gbs - 1.0));
-    double eta_ve = eta_up, Eii_pwl = 0.0, Eii_exp = 0.0, Eii_lin = 0.0;
-    const creep_laws L = {elastic, constant, dislocation, peierls, diffusion, eta_el, eta_cst, C_pwl, m.n_pwl,
-                          C_exp, ST + m.n_exp, C_lin, m.n_lin, diffusion ? pow(d, -m.m_lin) : 1.0};
+    double eta_up = 1.0e100 / md.scale_eta;                        // :585-592
+    if (L.constant) eta_up = fmin(eta_up, L.eta_cst);
+    if (L.dislocation) eta_up = fmin(eta_up, L.B_pwl * pow_call(Eii, 1.0 / m.n_pwl - 1.0));
+    if (L.elastic) eta_up = fmin(eta_up, L.eta_el);
+    if (L.peierls) eta_up = fmin(eta_up, L.B_exp * pow_call(Eii, 1.0 / L.nST - 1.0));
+    if (L.diffusion)
+        eta_up = fmin(eta_up, L.B_lin * pow_or_1(Eii, 1.0 / m.n_lin - 1.0) * pow_or_1(d, m.m_lin / m.n_lin));
+    if (L.gbs) eta_up = fmin(eta_up, L.B_gbs * pow_call(Eii, 1.0 / m.n_gbs - 1.0));
+    double eta_ve = eta_up;
+    double Eii_pwl = 0.0, Eii_exp = 0.0, Eii_lin = 0.0;
     if (!local_ve(L, Eii, eta_ve, Eii_pwl, Eii_exp, Eii_lin)) fail |= FAIL_LOCAL_ITER;
     double Tii = 2.0 * eta_ve * Eii;
     bool is_pl = false;
@@ -138,18 +213,20 @@ __device__ inline double viscosity_concise(const mdg_phase_prop &m, const rheo_c
             is_pl = true;
             const double F0 = F_trial, tol = md.eta_tol;
             const double Kdt_ss = K * dt * sin_fric * sin_dil;
-            double eta_vp = m.eta_vp * pow(Eii, 1.0 / m.n_vp - 1);
+            double eta_vp = m.eta_vp * pow_or_1(Eii, 1.0 / m.n_vp - 1);
             gdot = F_trial / (eta_ve + eta_vp + Kdt_ss);
             double Pc = P, Tiic = Tii;
-            for (int it = 0; it < 20; it++) {
+            bool done = false;
+            for (int it = 0; it < 20 && __any(!done); it++) {
+                if (done) continue;
                 Pc = P + K * dt * (gdot * sin_dil);
-                eta_vp = m.eta_vp * pow(fabs(gdot), 1.0 / m.n_vp - 1.0);
+                eta_vp = m.eta_vp * pow_or_1(fabs(gdot), 1.0 / m.n_vp - 1.0);
                 Tyield = Tyield + gdot * eta_vp;    // accumulates, as in the reference
                 Tiic = Tii - eta_ve * gdot;
                 F_trial = Tiic - Tyield;
                 const double res = fabs(F_trial);
-                if (res < tol || res / F0 < tol) break;
-                gdot -= F_trial / (-eta_ve - eta_vp / m.n_vp - Kdt_ss);
+                done = res < tol || res / F0 < tol;
+                if (!done) gdot -= F_trial / (-eta_ve - eta_vp / m.n_vp - Kdt_ss);
             }
             if (Tiic < 0.0) {                                          // :694-701
                 gdot = (Tii - md.Tiimin) / eta_ve;
@@ -166,16 +243,40 @@ __device__ inline double viscosity_concise(const mdg_phase_prop &m, const rheo_c
     // dissipative viscosity (:987-1032): each law's viscosity at its own
     // strain-rate share; diffusion creep at the phase's reference grain size
     double inv = 0.0;
-    if (peierls) inv += 1.0 / (B_exp * pow(Eii_exp, 1.0 / (ST + m.n_exp) - 1.0));
-    if (dislocation) inv += 1.0 / (B_pwl * pow(Eii_pwl, 1.0 / m.n_pwl - 1.0));
-    if (diffusion) inv += 1.0 / (B_lin * pow(Eii_lin, 1.0 / m.n_lin - 1.0) * pow(m.gs_ref, m.m_lin / m.n_lin));
-    if (constant) inv += 1.0 / eta_cst;
+    if (L.peierls) inv += 1.0 / (L.B_exp * pow_call(Eii_exp, 1.0 / L.nST - 1.0));
+    if (L.dislocation) inv += 1.0 / (L.B_pwl * pow_call(Eii_pwl, 1.0 / m.n_pwl - 1.0));
+    if (L.diffusion)
+        inv += 1.0 / (L.B_lin * pow_or_1(Eii_lin, 1.0 / m.n_lin - 1.0) * pow_or_1(m.gs_ref, m.m_lin / m.n_lin));
+    if (L.constant) inv += 1.0 / L.eta_cst;
     if (is_pl) inv += 1.0 / (Tii / gdot);
     double eta = 1.0 / inv;
     etaVE = fmax(fmin(etaVE, md.max_eta), md.min_eta);                 // :1058-1073
     if (eta > md.max_eta) eta = md.max_eta;
     if (eta < md.min_eta) eta = md.min_eta;
     return eta;
+}
+
+// Friction terms of a node: the phase's own, or those of the node's angles.
+__device__ __forceinline__ friction friction_at(const rheo_phase &ph, const mdg_rheo_nodes &f, int i) {
+    friction r{ph.sin_fric, ph.cos_fric, ph.sin_dil};
+    if (f.fric) {
+        r.sin_fric = sin(f.fric[i]);
+        r.cos_fric = cos(f.fric[i]);
+    }
+    if (f.dil) r.sin_dil = sin(f.dil[i]);
+    return r;
+}
+
+// The phase table of a call on the device (a buffer kept with the context).
+struct phase_buf : dbuf<rheo_phase> {
+    std::vector<rheo_phase> h;    // lives until the copy has run
+};
+inline int upload_phases(mdg_ctx *c, const mdg_phase_prop *phases, int nph, phase_buf &buf) {
+    buf.h.resize(nph);
+    for (int p = 0; p < nph; p++) buf.h[p] = make_phase(phases[p]);
+    HIPCHK(c, buf.reserve(nph));
+    HIPCHK(c, hipMemcpyAsync(buf.p, buf.h.data(), nph * sizeof(rheo_phase), hipMemcpyHostToDevice, c->stream));
+    return MDG_OK;
 }
 
 // Whether any phase needs the EXT instantiation of viscosity_concise.
