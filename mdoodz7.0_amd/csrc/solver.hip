@@ -806,49 +806,53 @@ __global__ void k_rtab(axis_map m, int nf, int nc, int RT, int *__restrict__ f0,
 template <typename T, int RT>
 __device__ inline double restrict_node(const comp_maps &m, const rtab &t, const sgrid &gf, const T *__restrict__ rf,
                                        int K, int L) {
-    const int kx = t.fx[K], lz = t.fz[L];
+    const int kx = t.fx[K], lz = t.fz[L], nx = (m.comp == 0) ? gf.Nx : gf.Nx + 1, nz = (m.comp == 0) ? gf.Nz + 1 : gf.Nz;
     double wxs[RT];
+    const double *wzs = t.wz + (size_t)L * RT;
 #pragma unroll
     for (int q = 0; q < RT; q++) wxs[q] = t.wx[(size_t)K * RT + q];
+    // the whole window is read (clamped to the grid, where the weights are
+    // zero; faces that are not free hold zero residuals), so that no load
+    // waits for a weight
     double s = 0.0;
-#pragma unroll
+#pragma unroll RT <= RT2 ? RT : 1
     for (int p = 0; p < RT; p++) {
-        const double wz = t.wz[(size_t)L * RT + p];
-        if (wz == 0.0) continue;
-        const int l = lz + p;
+        const T *row = rf + (size_t)min(lz + p, nz - 1) * nx;
+        double r = 0.0;
 #pragma unroll
-        for (int q = 0; q < RT; q++) {
-            if (wxs[q] == 0.0) continue;
-            const int k = kx + q;
-            const bool fr = (m.comp == 0) ? vx_free(gf, k, l) : vz_free(gf, k, l);
-            if (fr) s += wxs[q] * wz * (double)rf[k + l * m.nxf];
-        }
+        for (int q = 0; q < RT; q++) r += wxs[q] * (double)row[min(kx + q, nx - 1)];
+        s += wzs[p] * r;
     }
     return s;
 }
 
-// b_c = P^T r_f, with ghost contributions folded back like P maps them.
+// b_c = P^T r_f at coarse unknown i, with ghost contributions folded back like
+// P maps them.
+template <typename T, int RT>
+__device__ __forceinline__ T restrict_at(const comp_maps &mu, const comp_maps &mv, const rtab &tu, const rtab &tv,
+                                         const sgrid &gf, const sgrid &gc, const T *__restrict__ rf, int i) {
+    const int nuc = nvx(gc), nuf = nvx(gf);
+    if (i < nuc) {
+        const int K = i % gc.Nx, L = i / gc.Nx;
+        if (!vx_free(gc, K, L)) return T(0);
+        double s = restrict_node<T, RT>(mu, tu, gf, rf, K, L);
+        if (L == 1) s += (mu.ghost_lo == 1 ? 1.0 : -1.0) * restrict_node<T, RT>(mu, tu, gf, rf, K, 0);
+        if (L == gc.Nz - 1) s += (mu.ghost_hi == 1 ? 1.0 : -1.0) * restrict_node<T, RT>(mu, tu, gf, rf, K, gc.Nz);
+        return (T)s;
+    }
+    const int j = i - nuc, K = j % (gc.Nx + 1), L = j / (gc.Nx + 1);
+    if (!vz_free(gc, K, L)) return T(0);
+    const T *r = rf + nuf;
+    double s = restrict_node<T, RT>(mv, tv, gf, r, K, L);
+    if (K == 1) s += (mv.ghost_lo == 1 ? 1.0 : -1.0) * restrict_node<T, RT>(mv, tv, gf, r, 0, L);
+    if (K == gc.Nx - 1) s += (mv.ghost_hi == 1 ? 1.0 : -1.0) * restrict_node<T, RT>(mv, tv, gf, r, gc.Nx, L);
+    return (T)s;
+}
 template <typename T, int RT>
 __global__ void k_restrict(sgrid gf, sgrid gc, comp_maps mu, comp_maps mv, rtab tu, rtab tv, const T *__restrict__ rf,
                            T *__restrict__ bc) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nuc = nvx(gc), nvc = nvz(gc), nuf = nvx(gf);
-    if (i < nuc) {
-        const int K = i % gc.Nx, L = i / gc.Nx;
-        if (!vx_free(gc, K, L)) { bc[i] = T(0); return; }
-        double s = restrict_node<T, RT>(mu, tu, gf, rf, K, L);
-        if (L == 1) s += (mu.ghost_lo == 1 ? 1.0 : -1.0) * restrict_node<T, RT>(mu, tu, gf, rf, K, 0);
-        if (L == gc.Nz - 1) s += (mu.ghost_hi == 1 ? 1.0 : -1.0) * restrict_node<T, RT>(mu, tu, gf, rf, K, gc.Nz);
-        bc[i] = (T)s;
-    } else if (i < nuc + nvc) {
-        const int j = i - nuc, K = j % (gc.Nx + 1), L = j / (gc.Nx + 1);
-        if (!vz_free(gc, K, L)) { bc[i] = T(0); return; }
-        const T *r = rf + nuf;
-        double s = restrict_node<T, RT>(mv, tv, gf, r, K, L);
-        if (K == 1) s += (mv.ghost_lo == 1 ? 1.0 : -1.0) * restrict_node<T, RT>(mv, tv, gf, r, 0, L);
-        if (K == gc.Nx - 1) s += (mv.ghost_hi == 1 ? 1.0 : -1.0) * restrict_node<T, RT>(mv, tv, gf, r, gc.Nx, L);
-        bc[i] = (T)s;
-    }
+    if (i < nvx(gc) + nvz(gc)) bc[i] = restrict_at<T, RT>(mu, mv, tu, tv, gf, gc, rf, i);
 }
 
 // Coarse viscosity: geometric mean of the fine values whose positions fall
@@ -912,6 +916,207 @@ __global__ void __launch_bounds__(256) k_dense_solve(int n, const int *__restric
         for (int j = 0; j < n; j++) s += Ainv[(size_t)i * n + j] * (double)sb[j];
         x[idx[i]] = (T)s;
     }
+}
+
+// ------------------------------------------- small levels in one workgroup
+// The part of the V-cycle on the levels of at most SM_POS positions, down to
+// the dense coarsest solve and back, in one launch: smoothing calls, residuals
+// and transfers of those levels are all launch latency as kernels of their
+// own (one of the smoothing calls, 12-16 steps through global memory in one
+// workgroup, took 22-33 us, and there are two per level and V-cycle).  One
+// thread owns position (k, l), i.e. Vx(k, l) and Vz(k, l), with its two rows
+// in nine coefficients each in registers; the iterates alternate between two
+// LDS buffers (one barrier per step), the viscosities sit in LDS from the
+// start.  Same steps as k_cheb_block and the level kernels, in FP64 at either
+// precision of the levels: the barriers and latencies are the same, and an
+// FP32 hierarchy at the limit of its precision (a closed box with a viscosity
+// jump of 1e6) gains iterations.
+// Bound: LDS reads (ten neighbours per position and step) and the barriers,
+// about 0.4 us a step on 26^2.  The levels below 47^2 of a 383^2 hierarchy take
+// 44 us per V-cycle in it where their kernels took 110 us; the solve of the
+// 101^2 inclusion went from 75.4 to 55.4 ms, of 383^2 ellipses (FP64, patches)
+// from 400 to 364 ms, of 767^2 (mixed) from 734 to 659 ms.  The limit of 1024
+// positions is one per thread; 47^2 in here would cost its 24 steps 3 x 0.4 us
+// and the LDS of FP64 lines, about what its own launches cost.
+#define SM_POS 1024
+#define SM_THREADS 1024
+template <typename T>
+struct sm_level {
+    sgrid g;
+    stc<double> cf;
+    comp_maps mu, mv;          // transfer to the next coarser level
+    rtab tu, tv;
+    const T *en, *es;
+    const double *ab;          // 1/theta, then (a, c) of each further step
+    int nu, n, npos, deg, rt;
+    int oab;                   // offset of a copy of ab in the LDS doubles
+    int x0, x1, b, oen, oes;   // offsets into the LDS values
+};
+#define SM_RED 1024            // LDS doubles of the dense solve's partial sums
+struct sm_coarse {
+    int nfree, ndbl;           // unknowns; LDS doubles in front of the values
+    const int *idx;
+    const double *Ainv;
+};
+
+// deg smoothing steps on one level: x in X0 (all zero when `zero`), the result
+// left in X0, X1 the other buffer.
+template <typename T>
+__device__ __forceinline__ void sm_smooth(const sm_level<T> &L, double gamma, bool zero, const double *ab, double *X0, double *X1,
+                                          const double *B, const double *en, const double *es) {
+    const sgrid g = L.g;
+    const int t = threadIdx.x, Nx = g.Nx, NxV = Nx + 1;
+    const int l = t / Nx, k = t - l * Nx, iu = t, iv = L.nu + k + l * NxV;
+    const bool own = t < L.npos, fu = own && vx_free(g, k, l), fv = own && l < g.Nz && vz_free(g, k, l);
+    row9<double> ru = {}, rv = {};
+    double bu = 0.0, bv = 0.0, du = 0.0, dv = 0.0, xu = 0.0, xv = 0.0;
+    if (fu) {
+        ru = vx_row9<double>(g, L.cf, k, l, en, es, gamma);
+        bu = B[iu];
+        xu = X0[iu];
+        du = 1.0 / vx_diag9(ru, L.cf);
+    }
+    if (fv) {
+        rv = vz_row9<double>(g, L.cf, k, l, en, es, gamma);
+        bv = B[iv];
+        xv = X0[iv];
+        dv = 1.0 / vz_diag9(rv, L.cf);
+    }
+    double pu = xu, pv = xv, *cur = X0, *nxt = X1;
+    for (int s = 0; s < L.deg; s++) {
+        const double a = s ? ab[2 * s - 1] : 0.0, cc = s ? ab[2 * s] : ab[0];
+        double yu = xu, yv = xv, qu = bu, qv = bv;
+        if (!(zero && s == 0)) {
+            const double *u = cur, *v = cur + L.nu;
+            if (fu) {
+                const double vsw = v[iv - L.nu - NxV], vse = v[iv - L.nu - NxV + 1], vnw = v[iv - L.nu], vne = v[iv - L.nu + 1];
+                qu -= vx_apply9(ru, L.cf, xu, u[iu - 1], u[iu + 1], u[iu - Nx], u[iu + Nx], vsw, vse, vnw, vne);
+            }
+            if (fv) {
+                const int j = iv - L.nu;
+                qv -= vz_apply9(rv, L.cf, xv, v[j - 1], v[j + 1], v[j - NxV], v[j + NxV], u[iu - 1], u[iu], u[iu - 1 + Nx], u[iu + Nx]);
+            }
+        }
+        if (fu) yu += cc * (qu * du) + a * (xu - pu);
+        if (fv) yv += cc * (qv * dv) + a * (xv - pv);
+        pu = xu; pv = xv;
+        xu = yu; xv = yv;
+        if (fu) nxt[iu] = xu;
+        if (fv) nxt[iv] = xv;
+        __syncthreads();
+        double *q = cur; cur = nxt; nxt = q;
+    }
+    if (cur != X0) {
+        if (fu) X0[iu] = xu;
+        if (fv) X0[iv] = xv;
+        __syncthreads();
+    }
+}
+
+// r = b - A x of one level into R (non-free faces zero)
+template <typename T>
+__device__ __forceinline__ void sm_residual(const sm_level<T> &L, double gamma, const double *X, const double *B, const double *en,
+                                            const double *es, double *R) {
+    const sgrid g = L.g;
+    const int t = threadIdx.x, Nx = g.Nx, NxV = Nx + 1, l = t / Nx, k = t - l * Nx;
+    if (t < L.npos) {
+        const double *u = X, *v = X + L.nu;
+        const int j = k + l * NxV;
+        double r = 0.0;
+        if (vx_free(g, k, l)) {
+            const row9<double> q = vx_row9<double>(g, L.cf, k, l, en, es, gamma);
+            r = B[t] - vx_apply9(q, L.cf, u[t], u[t - 1], u[t + 1], u[t - Nx], u[t + Nx], v[j - NxV], v[j - NxV + 1], v[j], v[j + 1]);
+        }
+        R[t] = r;
+        if (l < g.Nz) {
+            r = 0.0;
+            if (vz_free(g, k, l)) {
+                const row9<double> q = vz_row9<double>(g, L.cf, k, l, en, es, gamma);
+                r = B[L.nu + j] - vz_apply9(q, L.cf, v[j], v[j - 1], v[j + 1], v[j - NxV], v[j + NxV], u[t - 1], u[t], u[t - 1 + Nx],
+                                            u[t + Nx]);
+            }
+            R[L.nu + j] = r;
+            if (k == Nx - 1) R[L.nu + j + 1] = 0.0;
+        }
+    }
+    __syncthreads();
+}
+
+template <typename T, int RT>
+__device__ __forceinline__ void sm_restrict(const sm_level<T> &F, const sm_level<T> &C, const double *rf, double *bc) {
+    const sgrid gf = F.g, gc = C.g;
+    for (int i = threadIdx.x; i < C.n; i += SM_THREADS) bc[i] = restrict_at<double, RT>(F.mu, F.mv, F.tu, F.tv, gf, gc, rf, i);
+    __syncthreads();
+}
+
+template <typename T>
+__global__ void __launch_bounds__(SM_THREADS) k_small_cycle(int nlev, const sm_level<T> *__restrict__ lev, sm_coarse co,
+                                                            double gamma, const T *__restrict__ b, T *__restrict__ x) {
+    extern __shared__ double sm_raw[];
+    double *const sm = sm_raw + co.ndbl;
+    const int t = threadIdx.x;
+    // right-hand side of the top level, zero starts, viscosities of every level
+    for (int i = 0; i < nlev; i++) {
+        const sm_level<T> &L = lev[i];
+        for (int q = t; q < L.n; q += SM_THREADS) {
+            sm[L.x0 + q] = 0.0;
+            sm[L.x1 + q] = 0.0;
+            if (i == 0) sm[L.b + q] = b[q];
+        }
+        if (i + 1 == nlev) break;
+        const int nc = ncell(L.g), nv = L.g.Nx * L.g.Nz;
+        for (int q = t; q < nc; q += SM_THREADS) sm[L.oen + q] = L.en[q];
+        for (int q = t; q < nv; q += SM_THREADS) sm[L.oes + q] = L.es[q];
+        for (int q = t; q < 2 * L.deg - 1; q += SM_THREADS) sm_raw[L.oab + q] = L.ab[q];
+    }
+    __syncthreads();
+    for (int i = 0; i + 1 < nlev; i++) {
+        const sm_level<T> &L = lev[i], &C = lev[i + 1];
+        sm_smooth<T>(L, gamma, true, sm_raw + L.oab, sm + L.x0, sm + L.x1, sm + L.b, sm + L.oen, sm + L.oes);
+        sm_residual<T>(L, gamma, sm + L.x0, sm + L.b, sm + L.oen, sm + L.oes, sm + L.x1);
+        if (L.rt == RT2) sm_restrict<T, RT2>(L, C, sm + L.x1, sm + C.b);
+        else sm_restrict<T, RT4>(L, C, sm + L.x1, sm + C.b);
+        // x1 held the residual: its walls and ghosts are zeros again, its free
+        // faces are written before they are read
+    }
+    {
+        // x[idx[i]] = sum_j Ainv[j][i] b[idx[j]] (Ainv is symmetric): 128 rows
+        // by 8 shares of the columns at a time, the shares added in order
+        const sm_level<T> &L = lev[nlev - 1];
+        double *red = sm_raw;                  // SM_RED doubles
+        const int col = t & 127, part = t >> 7;
+        for (int i0 = 0; i0 < co.nfree; i0 += 128) {
+            const int i = i0 + col;
+            double s = 0.0;
+            if (i < co.nfree)
+                for (int j = part; j < co.nfree; j += 8)
+                    s += co.Ainv[(size_t)j * co.nfree + i] * sm[L.b + co.idx[j]];
+            __syncthreads();
+            red[part * 128 + col] = s;
+            __syncthreads();
+            if (part == 0 && i < co.nfree) {
+                double r = 0.0;
+                for (int q = 0; q < 8; q++) r += red[q * 128 + col];
+                sm[L.x0 + co.idx[i]] = r;
+            }
+        }
+        __syncthreads();
+    }
+    for (int i = nlev - 2; i >= 0; i--) {
+        const sm_level<T> &L = lev[i], &C = lev[i + 1];
+        const sgrid g = L.g, gc = C.g;
+        double *xf = sm + L.x0;
+        const double *xc = sm + C.x0;
+        const int l = t / g.Nx, k = t - l * g.Nx;
+        if (t < L.npos) {
+            if (vx_free(g, k, l)) xf[t] += prolong_at<double>(L.mu, gc, xc, k, l);
+            if (l < g.Nz && vz_free(g, k, l)) xf[L.nu + k + l * (g.Nx + 1)] += prolong_at<double>(L.mv, gc, xc + C.nu, k, l);
+        }
+        __syncthreads();
+        sm_smooth<T>(L, gamma, false, sm_raw + L.oab, sm + L.x0, sm + L.x1, sm + L.b, sm + L.oen, sm + L.oes);
+    }
+    const sm_level<T> &L = lev[0];
+    for (int q = t; q < L.n; q += SM_THREADS) x[q] = (T)sm[L.x0 + q];
 }
 
 // ------------------------------------------------------- outer-level kernels
@@ -1305,6 +1510,11 @@ struct mg_hier {
     bool patch = false;                     // vertex-patch Schwarz preconditioning in the smoother
     int deg_coarse = 0;                     // smoothing degree below the finest level
     ktimer *tm = nullptr;                   // times the fine-level smoother steps (graphs = 2)
+    int small_from = -1;                    // levels from here on run in k_small_cycle (-1: none)
+    size_t small_lds = 0;
+    dbuf<sm_level<T>> small;
+    dbuf<double> small_ab;
+    sm_coarse small_co{};
     hipGraph_t graph = nullptr;             // one CG iteration (V-cycle included)
     hipGraphExec_t exec = nullptr;
     // pressure Poisson CG (BFBt): vectors, scalars and graph
@@ -1328,7 +1538,7 @@ struct mg_hier {
         for (auto &l : L) l.release();
         L.clear();
         cg_x.release(); cg_r.release(); cg_z.release(); cg_p.release(); cg_q.release();
-        scal.release(); part.release();
+        scal.release(); part.release(); small.release(); small_ab.release();
         pc_x.release(); pc_r.release(); pc_p.release(); pc_q.release(); bf_t.release();
         pscal.release(); ppart.release();
         if (h_scal) (void)hipHostFree(h_scal);
@@ -1423,6 +1633,78 @@ static void host_gauss_jordan_inverse(std::vector<double> &A, int n, bool *ok) {
 
 template <typename T>
 static int build_poisson(mdg_ctx *c, solver_state *s, mg_hier<T> &H);
+
+// Chebyshev coefficients of deg smoothing steps on [lmax / div, lmax]: 1/theta,
+// then (a, c) of each further step.
+static void cheb_table(double lmax, double div, int deg, std::vector<double> &ab) {
+    const double lmin = lmax / div, theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin), sigma = theta / delta;
+    double rho = 1.0 / sigma;
+    ab.push_back(1.0 / theta);
+    for (int k = 0; k < deg - 1; k++) {
+        const double rho_new = 1.0 / (2.0 * sigma - rho);
+        ab.push_back(rho_new * rho);
+        ab.push_back(2.0 * rho_new / delta);
+        rho = rho_new;
+    }
+}
+
+// The levels that k_small_cycle takes: the longest tail of the hierarchy whose
+// levels have at most SM_POS positions and fit the LDS together.
+#define SM_LDS_MAX (150 * 1024)
+template <typename T>
+static int plan_small(mdg_ctx *c, mg_hier<T> &H, const mdg_solver_opts *o) {
+    H.small_from = -1;
+    const int nl = (int)H.L.size();
+    if (!H.fused || nl < 2) return MDG_OK;
+    auto deg_of = [&](int i) { return i > 0 && H.deg_coarse > 0 ? H.deg_coarse : o->cheb_degree; };
+    size_t dbl = SM_RED, val = 0;
+    int from = nl;
+    for (int i = nl - 1; i >= 0; i--) {
+        const mg_level<T> &l = H.L[i];
+        const size_t d = dbl + (i + 1 < nl ? 2 * (size_t)deg_of(i) : 0);
+        const size_t v = val + 3 * (size_t)l.n + (i + 1 < nl ? (size_t)ncell(l.g) + (size_t)l.g.Nx * l.g.Nz : 0);
+        if (l.g.Nx * (l.g.Nz + 1) > SM_POS || l.n > CHEB_BLOCK_MAX || (d + v) * 8 > SM_LDS_MAX) break;
+        dbl = d;
+        val = v;
+        from = i;
+    }
+    if (from > nl - 2) return MDG_OK;
+    std::vector<sm_level<T>> h(nl - from);
+    std::vector<double> ab;
+    int od = SM_RED, ov = 0;
+    std::vector<size_t> oab(nl - from, 0);
+    for (int i = from; i < nl; i++) {
+        const mg_level<T> &l = H.L[i];
+        sm_level<T> &d = h[i - from];
+        d = sm_level<T>{};
+        d.g = l.g;
+        d.cf = make_stc<double>(l.g);
+        d.mu = l.mu; d.mv = l.mv; d.tu = l.tu; d.tv = l.tv;
+        d.en = l.en.p; d.es = l.es.p;
+        d.nu = l.nu; d.n = l.n; d.npos = l.g.Nx * (l.g.Nz + 1); d.deg = deg_of(i); d.rt = l.rt;
+        d.x0 = ov; d.x1 = ov + l.n; d.b = ov + 2 * l.n;
+        ov += 3 * l.n;
+        if (i + 1 == nl) break;
+        d.oen = ov; d.oes = ov + ncell(l.g);
+        ov += ncell(l.g) + l.g.Nx * l.g.Nz;
+        d.oab = od;
+        od += 2 * d.deg;
+        oab[i - from] = ab.size();
+        cheb_table(l.lmax, l.cheb_div, d.deg, ab);
+    }
+    HIPCHK(c, H.small_ab.reserve(ab.size()));
+    HIPCHK(c, H.small.reserve(h.size()));
+    for (size_t q = 0; q + 1 < h.size(); q++) h[q].ab = H.small_ab.p + oab[q];
+    HIPCHK(c, hipMemcpyAsync(H.small_ab.p, ab.data(), ab.size() * 8, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(H.small.p, h.data(), h.size() * sizeof(sm_level<T>), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));   // ab and h are local
+    const mg_level<T> &cl = H.L.back();
+    H.small_co = sm_coarse{cl.nfree, od, cl.idx.p, cl.Ainv.p};
+    H.small_lds = ((size_t)od + ov) * 8;
+    HIPCHK(c, hipFuncSetAttribute((const void *)k_small_cycle<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)H.small_lds));
+    H.small_from = from;
+    return MDG_OK;
+}
 
 template <typename T>
 static int build_hierarchy(mdg_ctx *c, solver_state *s, mg_hier<T> &H, const mdg_solver_opts *o) {
@@ -1557,6 +1839,10 @@ static int build_hierarchy(mdg_ctx *c, solver_state *s, mg_hier<T> &H, const mdg
     HIPCHK(c, cl.Ainv.reserve(A.size()));
     HIPCHK(c, hipMemcpyAsync(cl.Ainv.p, A.data(), A.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));   // A is a local host vector
+    {
+        int rc = plan_small(c, H, o);
+        if (rc) return rc;
+    }
     if (o->schur == 1) {
         int rc = build_poisson(c, s, H);
         if (rc) return rc;
@@ -1880,6 +2166,11 @@ template <typename T>
 static void vcycle(mdg_ctx *c, mg_hier<T> &H, size_t i, double gamma, int deg, int cycle) {
     mg_level<T> &lv = H.L[i];
     if (i > 0 && H.deg_coarse > 0) deg = H.deg_coarse;
+    if ((int)i == H.small_from && !(i == 0 && H.tm)) {
+        hipLaunchKernelGGL(k_small_cycle<T>, dim3(1), dim3(SM_THREADS), H.small_lds, c->stream, (int)H.L.size() - H.small_from,
+                           (const sm_level<T> *)H.small.p, H.small_co, gamma, lv.rhs(), lv.x.p);
+        return;
+    }
     if (i + 1 == H.L.size()) {
         hipLaunchKernelGGL(k_fill<T>, dim3(nblk(lv.n)), dim3(256), 0, c->stream, lv.n, lv.x.p, T(0));
         hipLaunchKernelGGL(k_dense_solve<T>, dim3(1), dim3(256), 0, c->stream, lv.nfree, lv.idx.p, lv.Ainv.p, lv.rhs(), lv.x.p);

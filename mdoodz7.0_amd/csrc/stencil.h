@@ -184,6 +184,75 @@ __device__ inline T apply_vz_rcp(const sgrid &g, const stc<T> &cf, int k, int l,
     return y * cf.dV;
 }
 
+// The same two rows for kernels that apply a row many times: five coefficients
+// of the own component, the two of the shear stresses' cross terms and the two
+// penalties (all times dV).  The penalty acts on the divergences themselves, as
+// in apply_*_rcp: multiplied out into nine coefficients of single velocities it
+// would lose the digits that cancel in a divergence, gamma times over, in FP32.
+// A face that is not free gets zeros.
+template <typename T>
+struct row9 {
+    T c, w, e, s, n, a, b, p0, p1;
+};
+template <typename T>
+__device__ inline row9<T> vx_row9(const sgrid &g, const stc<T> &cf, int k, int l, const T *__restrict__ en,
+                                  const T *__restrict__ es, T gamma) {
+    const int Nx = g.Nx, Ncx = Nx - 1;
+    const T enW = en[(k - 1) + (l - 1) * Ncx], enE = en[k + (l - 1) * Ncx];
+    const T D33S = es[k + (l - 1) * Nx], D33N = es[k + l * Nx];
+    const bool gS = (l == 1), gN = (l == g.Nz - 1);
+    const T fS = ghost_factor<T>(g.ghostS, gS), fN = ghost_factor<T>(g.ghostN, gN);
+    const T x2 = cf.idx2 * cf.dV, z2 = cf.idz2 * cf.dV, xz = cf.idxz * cf.dV, gx = gamma * cf.idx * cf.dV;
+    row9<T> r;
+    r.c = T(2) * (enE + enW) * x2 + (D33N * fN + D33S * fS) * z2;
+    r.w = -T(2) * enW * x2;
+    r.e = -T(2) * enE * x2;
+    r.s = gS ? T(0) : -D33S * z2;
+    r.n = gN ? T(0) : -D33N * z2;
+    r.a = D33S * xz;
+    r.b = D33N * xz;
+    r.p0 = gx * (g.pen_const ? T(1) : enW);
+    r.p1 = gx * (g.pen_const ? T(1) : enE);
+    return r;
+}
+template <typename T>
+__device__ inline row9<T> vz_row9(const sgrid &g, const stc<T> &cf, int k, int l, const T *__restrict__ en,
+                                  const T *__restrict__ es, T gamma) {
+    const int Nx = g.Nx, Ncx = Nx - 1;
+    const T enS = en[(k - 1) + (l - 1) * Ncx], enN = en[(k - 1) + l * Ncx];
+    const T D33W = es[(k - 1) + l * Nx], D33E = es[k + l * Nx];
+    const bool gW = (k == 1), gE = (k == Nx - 1);
+    const T fW = ghost_factor<T>(g.ghostW, gW), fE = ghost_factor<T>(g.ghostE, gE);
+    const T x2 = cf.idx2 * cf.dV, z2 = cf.idz2 * cf.dV, xz = cf.idxz * cf.dV, gz = gamma * cf.idz * cf.dV;
+    row9<T> r;
+    r.c = (D33E * fE + D33W * fW) * x2 + T(2) * (enN + enS) * z2;
+    r.w = gW ? T(0) : -D33W * x2;
+    r.e = gE ? T(0) : -D33E * x2;
+    r.s = -T(2) * enS * z2;
+    r.n = -T(2) * enN * z2;
+    r.a = D33W * xz;
+    r.b = D33E * xz;
+    r.p0 = gz * (g.pen_const ? T(1) : enS);
+    r.p1 = gz * (g.pen_const ? T(1) : enN);
+    return r;
+}
+// The rows applied: own component at the face and its W, E, S, N neighbours,
+// then the other component's four around it.
+template <typename T>
+__device__ __forceinline__ T vx_apply9(const row9<T> &r, const stc<T> &cf, T c, T w, T e, T s, T n, T sw, T se, T nw, T ne) {
+    const T divW = (c - w) * cf.idx + (nw - sw) * cf.idz, divE = (e - c) * cf.idx + (ne - se) * cf.idz;
+    return r.c * c + r.w * w + r.e * e + r.s * s + r.n * n + r.a * (se - sw) + r.b * (nw - ne) + (r.p0 * divW - r.p1 * divE);
+}
+template <typename T>
+__device__ __forceinline__ T vz_apply9(const row9<T> &r, const stc<T> &cf, T c, T w, T e, T s, T n, T sw, T se, T nw, T ne) {
+    const T divS = (se - sw) * cf.idx + (c - s) * cf.idz, divN = (ne - nw) * cf.idx + (n - c) * cf.idz;
+    return r.c * c + r.w * w + r.e * e + r.s * s + r.n * n + r.a * (nw - sw) + r.b * (se - ne) + (r.p0 * divS - r.p1 * divN);
+}
+template <typename T>
+__device__ __forceinline__ T vx_diag9(const row9<T> &r, const stc<T> &cf) { return r.c + (r.p0 + r.p1) * cf.idx; }
+template <typename T>
+__device__ __forceinline__ T vz_diag9(const row9<T> &r, const stc<T> &cf) { return r.c + (r.p0 + r.p1) * cf.idz; }
+
 // Diagonal of A_gamma (Jacobi scaling of the smoothers)
 template <typename T>
 __device__ inline T diag_vx(const sgrid &g, int k, int l, const T *__restrict__ en,
