@@ -918,6 +918,163 @@ __global__ void __launch_bounds__(256) k_dense_solve(int n, const int *__restric
     }
 }
 
+// ------------------------------------- several smoothing steps in one launch
+// On levels whose tiles do not fill the chip a smoothing step is latency: one
+// launch, one round trip for its operands, the phases of a patch solve. This
+// kernel runs S steps of the Chebyshev recurrence (patch-preconditioned, or
+// Jacobi) on a region of 32 x 32 positions in LDS, one position per thread:
+// the region's halo of 2S positions (S for Jacobi: the reach of a step is
+// two, or one) is recomputed by the neighbouring regions, so no step needs
+// another workgroup. A thread keeps its two rows as nine coefficients each,
+// its vertex patch's inverse (read from the level's table), x_k, x_{k-1} and
+// b in registers; the neighbours' x, the residuals and the patch solutions
+// go through LDS, three barriers a step. The level's other kernels fold in:
+// a zero start needs no fill, the residual after the last step comes from the
+// same region (one more position of halo), and the start of the second
+// smoothing call adds the coarse correction while it reads x.
+// Bound: three barriers and the LDS round trips of a step (0.9 us in FP64, 0.5
+// in FP32) after a start of 5 us; multi_steps has the times per step.  The
+// 101^2 solve went from 51.2 to 42.9 ms with it, of 383^2 (FP64, patches) from
+// 327 to 176 ms, of 767^2 (mixed) from 860 to 459 ms.
+#define CM_R 32            // region side
+#define CM_W (CM_R + 2)    // LDS row, one cell of padding on each side
+#define CM_MAX 8           // steps a launch at most
+struct cm_steps {
+    int n, halo, tx, nbx, ntiles;
+    double a[CM_MAX], c[CM_MAX];
+};
+enum { CM_ZERO = 0, CM_X = 1, CM_PROLONG = 2, CM_CONT = 3 };   // start: x = 0, x, x + P x_c, (x_k, x_{k-1})
+template <typename T>
+struct cm_io {
+    const T *x, *xp, *b, *en, *es, *pinv, *xc;   // xc: the coarser level's correction (CM_PROLONG)
+    T *xo, *xpo, *r;                             // x_{k+n}; x_{k+n-1} and r = b - A x where wanted
+};
+template <typename T, bool PATCH, int START>
+__global__ void __launch_bounds__(CM_R *CM_R) k_cheb_multi(sgrid g, stc<T> cf, T gamma, cm_steps st, cm_io<T> io, sgrid gc,
+                                                           comp_maps mu, comp_maps mv) {
+    constexpr int NL = CM_W * CM_W;
+    __shared__ T xs[PATCH ? 1 : 2][NL], vs[PATCH ? 1 : 2][NL];      // x of Vx and Vz (two copies for Jacobi)
+    __shared__ T rs[PATCH ? 2 * NL : 1], ys[PATCH ? 2 * NL : 1];   // residuals, patch solutions y_1 and y_3
+    const int t = threadIdx.x, ix = t & (CM_R - 1), iz = t / CM_R, p = (iz + 1) * CM_W + ix + 1;
+    const int tile = xcd_tile(blockIdx.x, st.ntiles), tz = tile / st.nbx;
+    const int k = (tile - tz * st.nbx) * st.tx - st.halo + ix, l = tz * st.tx - st.halo + iz;
+    const int nu = nvx(g), Nx = g.Nx, NxV = Nx + 1, iu = k + l * Nx, iv = nu + k + l * NxV;
+    const bool fu = vx_free(g, k, l), fv = vz_free(g, k, l);
+    row9<T> ru = {}, rv = {};
+    T bu = T(0), bv = T(0), xu = T(0), xv = T(0), pu = T(0), pv = T(0);
+    if (fu) {
+        ru = vx_row9<T>(g, cf, k, l, io.en, io.es, gamma);
+        bu = io.b[iu];
+        if (START != CM_ZERO) xu = io.x[iu];
+        if (START == CM_CONT) pu = io.xp[iu];
+        if (START == CM_PROLONG) xu += prolong_at<T>(mu, gc, io.xc, k, l);
+    }
+    if (fv) {
+        rv = vz_row9<T>(g, cf, k, l, io.en, io.es, gamma);
+        bv = io.b[iv];
+        if (START != CM_ZERO) xv = io.x[iv];
+        if (START == CM_CONT) pv = io.xp[iv];
+        if (START == CM_PROLONG) xv += prolong_at<T>(mv, gc, io.xc + nvx(gc), k, l);
+    }
+    if (START != CM_CONT) {
+        pu = xu;
+        pv = xv;
+    }
+    T M[10] = {};
+    T du = T(0), dv = T(0);
+    if (PATCH) {
+        if (k >= 0 && l >= 0 && k < Nx && l < g.Nz) {
+            const T *m = io.pinv + k + l * Nx;
+            const int NV = Nx * g.Nz;
+#pragma unroll
+            for (int q = 0; q < 10; q++) M[q] = m[(size_t)q * NV];
+        }
+    } else {
+        if (fu) du = T(1) / vx_diag9(ru, cf);
+        if (fv) dv = T(1) / vz_diag9(rv, cf);
+    }
+    for (int q = t; q < NL; q += CM_R * CM_R) {
+        xs[0][q] = T(0);
+        vs[0][q] = T(0);
+        if constexpr (PATCH) {
+            rs[q] = T(0); rs[NL + q] = T(0); ys[q] = T(0); ys[NL + q] = T(0);
+        } else {
+            xs[1][q] = T(0);
+            vs[1][q] = T(0);
+        }
+    }
+    __syncthreads();
+    xs[0][p] = xu;
+    vs[0][p] = xv;
+    __syncthreads();
+    // residual of the thread's two rows from LDS copy `c` of x
+    auto residual = [&](int c, T &qu, T &qv) {
+        const T *u = xs[c] + p, *v = vs[c] + p;
+        qu = bu;
+        qv = bv;
+        if (fu)
+            qu -= vx_apply9(ru, cf, xu, u[-1], u[1], u[-CM_W], u[CM_W], v[-CM_W], v[1 - CM_W], v[0], v[1]);
+        if (fv)
+            qv -= vz_apply9(rv, cf, xv, v[-1], v[1], v[-CM_W], v[CM_W], u[-1], u[0], u[CM_W - 1], u[CM_W]);
+    };
+    int cur = 0;
+    for (int s = 0; s < st.n; s++) {
+        const T a = (T)st.a[s], cc = (T)st.c[s];
+        T qu, qv, zu, zv;
+        if (START == CM_ZERO && s == 0) {
+            qu = bu;
+            qv = bv;
+        } else {
+            residual(cur, qu, qv);
+        }
+        if (PATCH) {
+            rs[p] = qu;
+            rs[NL + p] = qv;
+            __syncthreads();
+            // faces xS = Vx(k, l), xN = Vx(k, l+1), zW = Vz(k, l), zE = Vz(k+1, l) of vertex (k, l)
+            const T r1 = rs[p + CM_W], r3 = rs[NL + p + 1];
+            const T y1 = M[1] * qu + M[4] * r1 + M[5] * qv + M[6] * r3;
+            const T y3 = M[3] * qu + M[6] * r1 + M[8] * qv + M[9] * r3;
+            ys[p] = y1;
+            ys[NL + p] = y3;
+            const T y0 = M[0] * qu + M[1] * r1 + M[2] * qv + M[3] * r3;
+            const T y2 = M[2] * qu + M[5] * r1 + M[7] * qv + M[8] * r3;
+            __syncthreads();
+            zu = y0 + ys[p - CM_W];            // patch (k, l) as xS, patch (k, l-1) as xN
+            zv = y2 + ys[NL + p - 1];          // patch (k, l) as zW, patch (k-1, l) as zE
+        } else {
+            zu = qu * du;
+            zv = qv * dv;
+            cur ^= 1;
+        }
+        T yu = xu, yv = xv;
+        if (fu) yu += cc * zu + a * (xu - pu);
+        if (fv) yv += cc * zv + a * (xv - pv);
+        pu = xu; pv = xv;
+        xu = yu; xv = yv;
+        xs[cur][p] = xu;
+        vs[cur][p] = xv;
+        __syncthreads();
+    }
+    const int h = st.halo;
+    if (ix < h || ix >= h + st.tx || iz < h || iz >= h + st.tx || k >= Nx || l > g.Nz) return;
+    T qu = T(0), qv = T(0);
+    if (io.r) residual(cur, qu, qv);
+    io.xo[iu] = xu;
+    if (io.xpo) io.xpo[iu] = pu;
+    if (io.r) io.r[iu] = qu;
+    if (l < g.Nz) {
+        io.xo[iv] = xv;
+        if (io.xpo) io.xpo[iv] = pv;
+        if (io.r) io.r[iv] = qv;
+        if (k == Nx - 1) {                     // the never-free Vz column Nx
+            io.xo[iv + 1] = T(0);
+            if (io.xpo) io.xpo[iv + 1] = T(0);
+            if (io.r) io.r[iv + 1] = T(0);
+        }
+    }
+}
+
 // ------------------------------------------- small levels in one workgroup
 // The part of the V-cycle on the levels of at most SM_POS positions, down to
 // the dense coarsest solve and back, in one launch: smoothing calls, residuals
@@ -1471,7 +1628,9 @@ struct mg_level {
     sgrid g;
     int nu = 0, nv = 0, n = 0;
     dbuf<T> en, es, dinv, x, b, r, d;
-    dbuf<T> pinv;          // vertex-patch inverses (smoother 2; smoother 3's eigenvalue estimate)
+    dbuf<T> pinv;          // vertex-patch inverses (smoother 2; smoother 3's eigenvalue estimate, k_cheb_multi)
+    int multi = 0;         // smoothing steps per launch of k_cheb_multi (0: one launch per step)
+    dbuf<T> mx;            // its iterates between launches: two pairs (x_k, x_{k-1})
     bool patch = false;    // smoothed with vertex patches (smoother 2, 3 on the finest patch_levels levels)
     double lmax = 1.0;
     double cheb_div = 30.0;  // smoothed range [lmax / cheb_div, lmax]
@@ -1491,7 +1650,7 @@ struct mg_level {
     rtab tu{}, tv{};
     int rt = RT2;          // restriction window (RT2 or RT4)
     void release() {
-        rt_f.release(); rt_w.release();
+        rt_f.release(); rt_w.release(); mx.release();
         en.release(); es.release(); dinv.release(); x.release(); b.release(); r.release();
         d.release(); idx.release(); Ainv.release(); pinv.release();
         px.release(); pb.release(); pr.release(); pd.release(); pdinv.release(); pAinv.release();
@@ -1646,6 +1805,25 @@ static void cheb_table(double lmax, double div, int deg, std::vector<double> &ab
         ab.push_back(2.0 * rho_new / delta);
         rho = rho_new;
     }
+}
+
+// Steps per launch of k_cheb_multi on a level (0: k_pcheb or k_cheb3, one launch
+// per step).  More steps share one launch's latency but widen the recomputed
+// halo.  Kernel time per patch step in us, k_pcheb against 2, 3, 4 a launch:
+//   FP64   383^2   9.2 | 7.2  5.4  6.5     FP32   767^2  14.3 | 8.0  6.9  8.3
+//          191^2   6.5 | 3.8  2.9  2.4            383^2   7.2 | 3.7  2.8  3.2
+//           95^2   5.9 | 3.8  2.8  2.3            191^2   6.1 | 2.7  2.1  1.7
+// (6 a launch on levels up to 95^2 take another 8% off the 383^2 solve.)
+// Jacobi, FP64, whole solves in ms, k_cheb3 against 2, 3, 4, 5, 6 a launch:
+// 101^2 52 | 53 48 44 45 43, 255^2 133 | 124 108 91 92 84, 511^2 263 | 242 209
+// 176 177 163.  An FP32 Jacobi hierarchy keeps single steps: it is there that
+// a viscosity jump of 1e6 leaves CG at the limit of FP32, and the solve's
+// iterations depend on the last bits.
+template <typename T>
+static int multi_steps(const sgrid &g, bool patch) {
+    const long n = (long)g.Nx * (g.Nz + 1);
+    if (patch) return n <= 12000 ? 6 : (n <= 40000 ? 4 : 3);
+    return sizeof(T) == 8 ? 6 : 0;
 }
 
 // The levels that k_small_cycle takes: the longest tail of the hierarchy whose
@@ -1842,6 +2020,12 @@ static int build_hierarchy(mdg_ctx *c, solver_state *s, mg_hier<T> &H, const mdg
     {
         int rc = plan_small(c, H, o);
         if (rc) return rc;
+    }
+    for (int i = 0; i + 1 < (int)H.L.size(); i++) {
+        mg_level<T> &lv = H.L[i];
+        const int deg = i > 0 && H.deg_coarse > 0 ? H.deg_coarse : o->cheb_degree;
+        lv.multi = H.fused && deg >= 2 && (H.small_from < 0 || i < H.small_from) ? multi_steps<T>(lv.g, lv.patch) : 0;
+        if (lv.multi) HIPCHK(c, lv.mx.reserve(4 * (size_t)lv.n));
     }
     if (o->schur == 1) {
         int rc = build_poisson(c, s, H);
@@ -2160,6 +2344,39 @@ static void chebyshev(mdg_ctx *c, mg_level<T> &lv, double gamma, int deg, bool z
     hipLaunchKernelGGL(k_axpby<T>, dim3(nblk(n)), dim3(256), 0, c->stream, n, T(1), lv.d.p, T(1), lv.x.p);
 }
 
+// A smoothing call in launches of lv.multi steps: from zero with the residual
+// left in lv.r (`down`), or from lv.x plus the coarser level's correction.
+template <typename T, bool PATCH>
+static void cheb_multi(mdg_ctx *c, mg_level<T> &lv, const mg_level<T> &cl, double gamma, int deg, bool down) {
+    std::vector<double> ab;
+    cheb_table(lv.lmax, lv.cheb_div, deg, ab);
+    const int nl = std::max(2, (deg + lv.multi - 1) / lv.multi);   // the call ends in lv.x, which its first launch reads
+    const T *x = lv.x.p, *xp = nullptr;
+    for (int i = 0, s0 = 0; i < nl; i++) {
+        const bool last = i + 1 == nl;
+        cm_steps st{};
+        st.n = (deg * (i + 1)) / nl - s0;
+        st.halo = st.n * (PATCH ? 2 : 1) + (last && down ? 1 : 0);
+        st.tx = CM_R - 2 * st.halo;
+        st.nbx = (lv.g.Nx + st.tx - 1) / st.tx;
+        st.ntiles = st.nbx * ((lv.g.Nz + 1 + st.tx - 1) / st.tx);
+        for (int q = 0; q < st.n; q++) {
+            const int s = s0 + q;
+            st.a[q] = s ? ab[2 * s - 1] : 0.0;
+            st.c[q] = s ? ab[2 * s] : ab[0];
+        }
+        s0 += st.n;
+        T *out = lv.mx.p + (size_t)(i & 1) * 2 * lv.n;
+        cm_io<T> io{x, xp, lv.rhs(), lv.en.p, lv.es.p, lv.pinv.p, cl.x.p, last ? lv.x.p : out, last ? nullptr : out + lv.n,
+                    last && down ? lv.r.p : nullptr};
+        auto kern = i ? k_cheb_multi<T, PATCH, CM_CONT> : (down ? k_cheb_multi<T, PATCH, CM_ZERO> : k_cheb_multi<T, PATCH, CM_PROLONG>);
+        hipLaunchKernelGGL(kern, dim3(st.ntiles), dim3(CM_R * CM_R), 0, c->stream, lv.g, make_stc<T>(lv.g), (T)gamma, st, io, cl.g,
+                           lv.mu, lv.mv);
+        x = out;
+        xp = out + lv.n;
+    }
+}
+
 // solves approximately A_g x = b on level i (b, x in lv.b, lv.x); cycle = 1
 // gives a V-cycle, 2 a W-cycle.
 template <typename T>
@@ -2178,17 +2395,31 @@ static void vcycle(mdg_ctx *c, mg_hier<T> &H, size_t i, double gamma, int deg, i
     }
     mg_level<T> &cl = H.L[i + 1];
     ktimer *tm = (i == 0) ? H.tm : nullptr;
-    chebyshev(c, lv, gamma, deg, true, H.fused, tm, lv.patch);
-    const int reps = (i + 2 == H.L.size()) ? 1 : cycle;
-    for (int rep = 0; rep < reps; rep++) {
-        hipLaunchKernelGGL(k_vel_residual<T>, dim3(nblk(lv.n)), dim3(256), 0, c->stream, lv.g, (T)gamma, lv.x.p, lv.rhs(),
-                           lv.en.p, lv.es.p, lv.r.p);
+    auto restrict_r = [&]() {
         if (lv.rt == RT2)
             hipLaunchKernelGGL((k_restrict<T, RT2>), dim3(nblk(cl.n)), dim3(256), 0, c->stream, lv.g, cl.g, lv.mu, lv.mv, lv.tu,
                                lv.tv, (const T *)lv.r.p, cl.b.p);
         else
             hipLaunchKernelGGL((k_restrict<T, RT4>), dim3(nblk(cl.n)), dim3(256), 0, c->stream, lv.g, cl.g, lv.mu, lv.mv, lv.tu,
                                lv.tv, (const T *)lv.r.p, cl.b.p);
+    };
+    if (lv.multi && !tm) {
+        auto smooth = [&](bool down) {
+            if (lv.patch) cheb_multi<T, true>(c, lv, cl, gamma, deg, down);
+            else cheb_multi<T, false>(c, lv, cl, gamma, deg, down);
+        };
+        smooth(true);
+        restrict_r();
+        vcycle(c, H, i + 1, gamma, deg, cycle);
+        smooth(false);
+        return;
+    }
+    chebyshev(c, lv, gamma, deg, true, H.fused, tm, lv.patch);
+    const int reps = (i + 2 == H.L.size()) ? 1 : cycle;
+    for (int rep = 0; rep < reps; rep++) {
+        hipLaunchKernelGGL(k_vel_residual<T>, dim3(nblk(lv.n)), dim3(256), 0, c->stream, lv.g, (T)gamma, lv.x.p, lv.rhs(),
+                           lv.en.p, lv.es.p, lv.r.p);
+        restrict_r();
         vcycle(c, H, i + 1, gamma, deg, cycle);
         hipLaunchKernelGGL(k_prolong<T>, dim3(nblk(lv.n)), dim3(256), 0, c->stream, lv.g, cl.g, lv.mu, lv.mv, cl.x.p, lv.x.p);
     }
