@@ -16,6 +16,8 @@
 #define P2G_MAXPH 32
 #define P2G_MAXTAB 1024
 #define P2G_TILE 256     // nodes per block of the row-tiled kernels
+#define P2G_FILL 512     // blocks of k_p2g_tile below which it takes one node row per block
+#define P2G_LTAB 64      // phase tables up to this long are averaged once per block, in LDS
 
 struct p2g_fld {
     const double      *src;   // per-phase table (flag 0) or sorted per-marker (flag 1)
@@ -67,12 +69,32 @@ __device__ __forceinline__ void p2g_visit(const p2g_geo &g, const unsigned *__re
     }
 }
 
+__device__ __forceinline__ double avg_val(int avg, double v) {
+    if (avg == 1) v = 1.0 / v;
+    if (avg == 2) v = p2g_log(v);
+    return v;
+}
 __device__ __forceinline__ double mark_val(const p2g_fld &f, int p, unsigned i) {
     // a phase outside the table reads as NaN instead of out of bounds
-    double v = (f.flag == 0) ? ((p < f.n_src) ? f.src[p] : __builtin_nan("")) : f.src[i];
-    if (f.avg == 1) v = 1.0 / v;
-    if (f.avg == 2) v = p2g_log(v);
-    return v;
+    const double v = (f.flag == 0) ? (((unsigned)p < (unsigned)f.n_src) ? f.src[p] : __builtin_nan("")) : f.src[i];
+    return avg_val(f.avg, v);
+}
+// The row-tiled kernels work a phase table's averaging (1/v, log v) out once
+// per entry and block instead of once per marker: 37.7M markers, 3 vertex
+// fields 609 -> 459 us, 4 centre fields 380 -> 275 us (k_p2g_tile).
+template <int NF>
+__device__ __forceinline__ void load_tables(const p2g_set &fs, double (*ltab)[P2G_LTAB]) {
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+        const p2g_fld &F = fs.f[f];
+        if (F.flag == 0 && F.n_src <= P2G_LTAB)
+            for (int p = threadIdx.x; p < F.n_src; p += P2G_TILE) ltab[f][p] = avg_val(F.avg, F.src[p]);
+    }
+}
+__device__ __forceinline__ double tab_val(const p2g_fld &F, const double *ltab, int p, double v) {
+    if (F.flag != 0) return avg_val(F.avg, v);
+    if (F.n_src > P2G_LTAB) return mark_val(F, p, 0u);
+    return ((unsigned)p < (unsigned)F.n_src) ? ltab[p] : __builtin_nan("");
 }
 
 template <int NF>
@@ -116,16 +138,28 @@ __global__ void __launch_bounds__(256) k_p2g(p2g_geo g, p2g_set fs, const unsign
 // neighbour cells and sums the markers whose home is one of its 3 x 3
 // neighbours, with the reference's weight expression (|X[home] + o dx - x|
 // for a neighbour at offset o).  Fixed order: bit-reproducible.
+// Bound: the visits' FP64 and LDS reads, 9 markers' worth per marker; so the
+// nodes' coordinates sit in LDS and a home is kept as its two offsets from
+// the block (no division or global load per visit).  637 x 301 vertices, 1.7M
+// markers: 3 vertex fields 381 -> 197 us, 4 centre fields 267 -> 147 us, phase
+// fractions 212 (general path) -> 111 us.
+// PHASE: sums the weights of each phase (P2Mastah with prop = 1) instead.
 template <int NF> struct tile9_cap { static constexpr int v = (NF <= 2) ? 1024 : 640; };
+struct p2g_perc {
+    double *p[P2G_MAXPH];
+};
 
-template <int NF>
+template <int NF, bool PHASE>
 __global__ void __launch_bounds__(P2G_TILE)
 k_p2g9_tile(p2g_geo g, p2g_set fs, const unsigned *__restrict__ qoff, const unsigned *__restrict__ keys,
             const double *__restrict__ mx, const double *__restrict__ mz, const int *__restrict__ mph,
-            int nbx, int nblocks) {
+            int nbx, int nblocks, int nph, const signed char *ntype, p2g_perc perc) {
     constexpr int CAP = tile9_cap<NF>::v;
-    __shared__ double lx[CAP], lz[CAP], lv[NF][CAP];
-    __shared__ int lh[CAP];
+    __shared__ double lx[CAP], lz[CAP], lv[PHASE ? 1 : NF][PHASE ? 1 : CAP], ltab[NF][P2G_LTAB];
+    __shared__ double lX[P2G_TILE + 2], lZ[3];   // columns k0 - 1 .. k0 + 256, rows l - 1 .. l + 1
+    __shared__ short lk[CAP], lp[PHASE ? CAP : 1];
+    __shared__ signed char ll[CAP];
+    extern __shared__ double acc[];              // PHASE: nph x P2G_TILE
     const int b = blockIdx.x, xcd = b & 7, per = nblocks >> 3, rem = nblocks & 7;
     const int tile = xcd * per + min(xcd, rem) + (b >> 3);
     const int l = tile / nbx, k0 = (tile - l * nbx) * P2G_TILE;
@@ -141,6 +175,13 @@ k_p2g9_tile(p2g_geo g, p2g_set fs, const unsigned *__restrict__ qoff, const unsi
     const int cz0 = max(zc ? l - 1 + g.ax.zoff : l - 2, 0);
     const int cz1 = min(zc ? l + 1 + g.ax.zoff : l + 1, g.Ncz - 1);
     const int node = own ? l * g.nx + k : -1;
+    if constexpr (PHASE) {
+        for (int p = 0; p < nph; p++) acc[p * P2G_TILE + t] = 0.0;
+    } else {
+        load_tables<NF>(fs, ltab);
+    }
+    for (int q = t; q < P2G_TILE + 2; q += P2G_TILE) lX[q] = g.X[min(max(k0 - 1 + q, 0), g.nx - 1)];
+    if (t < 3) lZ[t] = g.Z[min(max(l - 1 + t, 0), g.nz - 1)];
     double W = 0.0, BW[NF];
 #pragma unroll
     for (int f = 0; f < NF; f++) BW[f] = 0.0;
@@ -154,38 +195,53 @@ k_p2g9_tile(p2g_geo g, p2g_set fs, const unsigned *__restrict__ qoff, const unsi
         }
         for (unsigned cs = S; cs < E; cs += CAP) {
             const unsigned ce = min(E, cs + (unsigned)CAP);
-            __syncthreads();   // previous chunk consumed
+            __syncthreads();   // previous chunk consumed (tables and coordinates there)
             for (unsigned j = cs + t; j < ce; j += P2G_TILE) {
                 const unsigned q = j - cs;
                 lx[q] = mx[j];
                 lz[q] = mz[j];
                 const unsigned key = keys[j], cell = key >> 2, qd = key & 3u;
-                const int cx = (int)(cell % (unsigned)g.Ncx), czm = (int)(cell / (unsigned)g.Ncx);
-                const int hk = xc ? cx - g.ax.xoff : cx + (int)(qd & 1u);
-                const int hl = zc ? czm - g.ax.zoff : czm + (int)(qd >> 1);
-                lh[q] = hk + hl * g.nx;
+                const int cx = (int)(cell - (unsigned)cz * (unsigned)g.Ncx);   // the chunk's markers lie in cell row cz
+                lk[q] = (short)((xc ? cx - g.ax.xoff : cx + (int)(qd & 1u)) - k0);
+                ll[q] = (signed char)((zc ? cz - g.ax.zoff : cz + (int)(qd >> 1)) - l);
                 const int p = mph[j];
+                if constexpr (PHASE) {
+                    lp[q] = (short)((p >= 0 && p < nph) ? p : -1);
+                } else {
 #pragma unroll
-                for (int f = 0; f < NF; f++) lv[f][q] = mark_val(fs.f[f], p, j);
+                    for (int f = 0; f < NF; f++) lv[f][q] = tab_val(fs.f[f], ltab[f], p, fs.f[f].flag ? fs.f[f].src[j] : 0.0);
+                }
             }
             __syncthreads();
             const unsigned a = max(ts, cs), e = min(te, ce);
             for (unsigned i = a; i < e; i++) {
                 const unsigned q = i - cs;
-                const int h = lh[q], hl = h / g.nx, hk = h - hl * g.nx;
-                const int ox = k - hk, oz = l - hl;
+                const int hk = lk[q], ox = t - hk, oz = -(int)ll[q];
                 if (ox < -1 || ox > 1 || oz < -1 || oz > 1) continue;
-                const double x = lx[q], z = lz[q];
-                const double dxm = (ox == 0) ? fabs(g.X[hk] - x) : fabs(g.X[hk] + ox * g.dx - x);
-                const double dzm = (oz == 0) ? fabs(g.Z[hl] - z) : fabs(g.Z[hl] + oz * g.dz - z);
+                const double x = lx[q], z = lz[q], X = lX[hk + 1], Z = lZ[1 - oz];
+                const double dxm = (ox == 0) ? fabs(X - x) : fabs(X + ox * g.dx - x);
+                const double dzm = (oz == 0) ? fabs(Z - z) : fabs(Z + oz * g.dz - z);
                 const double w = (1.0 - dxm * g.ix_itp) * (1.0 - dzm * g.iz_itp);
                 W += w;
+                if constexpr (PHASE) {
+                    const int p = lp[q];
+                    if (p >= 0) acc[p * P2G_TILE + t] += w;
+                } else {
 #pragma unroll
-                for (int f = 0; f < NF; f++) BW[f] += lv[f][q] * w;
+                    for (int f = 0; f < NF; f++) BW[f] += lv[f][q] * w;
+                }
             }
         }
     }
     if (!own) return;
+    if constexpr (PHASE) {
+        const bool skip = fabs(W) < 1e-30 || (ntype && (ntype[node] == 30 || ntype[node] == 31));
+        for (int p = 0; p < nph; p++) {
+            const double v = acc[p * P2G_TILE + t];
+            perc.p[p][node] = skip ? v : v / W;
+        }
+        return;
+    }
 #pragma unroll
     for (int f = 0; f < NF; f++) {
         const p2g_fld &F = fs.f[f];
@@ -243,7 +299,7 @@ k_p2g_tile(p2g_geo g, p2g_set fs, const unsigned *__restrict__ qoff, const doubl
            int need_phase, int nbx, int nblocks, int *__restrict__ stray) {
     constexpr int CAP = tile_cap<NF>::v;
     __shared__ double lw[CAP];
-    __shared__ double lwv[NF][CAP];
+    __shared__ double lwv[NF][CAP], ltab[NF][P2G_LTAB];
     __shared__ int lhome[PRE ? 1 : CAP];   // homes are checked when the weights are cached
     // XCD-aware order: hardware block b runs on XCD b % 8; XCD x gets the
     // contiguous logical tiles [start(x), start(x) + count(x)).
@@ -288,12 +344,13 @@ k_p2g_tile(p2g_geo g, p2g_set fs, const unsigned *__restrict__ qoff, const doubl
         for (int f = 0; f < NF; f++) BW[r][f] = 0.0;
     }
     bool bad = false;
+    load_tables<NF>(fs, ltab);
     for (int cz = cz0; cz <= cz1 && cx0 <= cx1; cz++) {
         const unsigned S = qoff[4u * (unsigned)(cx0 + cz * g.Ncx)];
         const unsigned E = qoff[4u * (unsigned)(cx1 + cz * g.Ncx) + 4u];
         for (unsigned cs = S; cs < E; cs += CAP) {
             const unsigned ce = min(E, cs + (unsigned)CAP);
-            __syncthreads();   // previous chunk fully consumed
+            __syncthreads();   // previous chunk fully consumed (tables there)
             // Every thread first issues all loads of its (up to PER) markers so
             // that the whole chunk is in flight at once, then computes.
             constexpr int PER = CAP / P2G_TILE;
@@ -337,12 +394,7 @@ k_p2g_tile(p2g_geo g, p2g_set fs, const unsigned *__restrict__ qoff, const doubl
                 lw[q] = w;
 #pragma unroll
                 for (int f = 0; f < NF; f++) {
-                    const p2g_fld &F = fs.f[f];
-                    const int p = ps[m];
-                    double v = (F.flag == 0) ? ((p < F.n_src) ? F.src[p] : __builtin_nan("")) : vs[f][m];
-                    if (F.avg == 1) v = 1.0 / v;
-                    if (F.avg == 2) v = p2g_log(v);
-                    lwv[f][q] = v * w;
+                    lwv[f][q] = tab_val(fs.f[f], ltab[f], ps[m], vs[f][m]) * w;
                 }
             }
             __syncthreads();
@@ -383,13 +435,13 @@ k_p2g_tile(p2g_geo g, p2g_set fs, const unsigned *__restrict__ qoff, const doubl
     }
 }
 
-// Phase fractions (P2Mastah with prop = 1): per-thread phase accumulators in LDS.
+// Phase fractions (P2Mastah with prop = 1) of the general path: per-thread
+// phase accumulators in LDS, markers read one by one.
 __global__ void __launch_bounds__(128) k_p2g_phase(p2g_geo g, int nph, const signed char *ntype,
                                                    const unsigned *__restrict__ qoff,
                                                    const double *__restrict__ mx,
                                                    const double *__restrict__ mz,
-                                                   const int *__restrict__ mph,
-                                                   double *__restrict__ perc,
+                                                   const int *__restrict__ mph, p2g_perc perc,
                                                    int *__restrict__ stray) {
     __shared__ double acc[P2G_MAXPH * 128];
     const int t = threadIdx.x;
@@ -403,11 +455,86 @@ __global__ void __launch_bounds__(128) k_p2g_phase(p2g_geo g, int nph, const sig
         const int p = mph[i];
         if (p >= 0 && p < nph) acc[p * 128 + t] += w;
     });
-    const size_t nn = (size_t)g.nx * g.nz;
     const bool skip = fabs(W) < 1e-30 || (ntype && (ntype[node] == 30 || ntype[node] == 31));
     for (int p = 0; p < nph; p++) {
         const double a = acc[p * 128 + t];
-        perc[p * nn + node] = skip ? a : a / W;
+        perc.p[p][node] = skip ? a : a / W;
+    }
+}
+
+// Phase fractions of the 1-cell stencil from cached weights, row-tiled like
+// k_p2g_tile: the cell rows of P2G_TILE nodes of one row go through LDS as
+// (weight, phase) with coalesced loads, 12 B per marker, where the general
+// path reads every marker's position, scattered, and works its weight out
+// again.  Same sums in the same order.  37.7M markers, 9 phases: 485 -> 179 us;
+// 160k markers: 13.4 -> 7.8 us.
+#define PH_CAP 1024
+__global__ void __launch_bounds__(P2G_TILE)
+k_p2g_phase_tile(p2g_geo g, int nph, const signed char *ntype, const unsigned *__restrict__ qoff,
+                 const double *__restrict__ mw, const int *__restrict__ mph, int nbx, int nblocks, p2g_perc perc) {
+    __shared__ double lw[PH_CAP];
+    __shared__ short lp[PH_CAP];
+    extern __shared__ double acc[];              // nph x P2G_TILE
+    const int b = blockIdx.x, xcd = b & 7, per = nblocks >> 3, rem = nblocks & 7;
+    const int tile = xcd * per + min(xcd, rem) + (b >> 3);
+    const int l = tile / nbx, k0 = (tile - l * nbx) * P2G_TILE;
+    const int kend = min(k0 + P2G_TILE, g.nx);
+    const int t = threadIdx.x, k = k0 + t;
+    const bool own = k < kend;
+    unsigned rs[4] = {0u, 0u, 0u, 0u}, re[4] = {0u, 0u, 0u, 0u};
+    int nr = 0;
+    if (own)
+        for_node_ranges(qoff, g.Ncx, g.Ncz, g.ax, k, l, [&](unsigned s0, unsigned e0) {
+            if (nr < 4) {
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (q == nr) { rs[q] = s0; re[q] = e0; }
+                nr++;
+            }
+        });
+    const bool xc = (g.ax.xkind == CELL_AXIS), zc = (g.ax.zkind == CELL_AXIS);
+    const int cx0 = max(xc ? k0 + g.ax.xoff : k0 - 1, 0), cx1 = min(xc ? kend - 1 + g.ax.xoff : kend - 1, g.Ncx - 1);
+    const int cz0 = max(zc ? l + g.ax.zoff : l - 1, 0), cz1 = min(zc ? l + g.ax.zoff : l, g.Ncz - 1);
+    for (int p = 0; p < nph; p++) acc[p * P2G_TILE + t] = 0.0;
+    double W = 0.0;
+    for (int cz = cz0; cz <= cz1 && cx0 <= cx1; cz++) {
+        const unsigned S = qoff[4u * (unsigned)(cx0 + cz * g.Ncx)];
+        const unsigned E = qoff[4u * (unsigned)(cx1 + cz * g.Ncx) + 4u];
+        for (unsigned cs = S; cs < E; cs += PH_CAP) {
+            const unsigned ce = min(E, cs + (unsigned)PH_CAP);
+            __syncthreads();   // previous chunk consumed
+            double ws[PH_CAP / P2G_TILE];
+            int ps[PH_CAP / P2G_TILE];
+#pragma unroll
+            for (int m = 0; m < PH_CAP / P2G_TILE; m++) {
+                const unsigned j = cs + t + (unsigned)m * P2G_TILE;
+                ws[m] = (j < ce) ? mw[j] : 0.0;
+                ps[m] = (j < ce) ? mph[j] : -1;
+            }
+#pragma unroll
+            for (int m = 0; m < PH_CAP / P2G_TILE; m++) {
+                lw[t + m * P2G_TILE] = ws[m];
+                lp[t + m * P2G_TILE] = (short)((ps[m] >= 0 && ps[m] < nph) ? ps[m] : -1);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const unsigned a = max(rs[q], cs), e = min(re[q], ce);
+                for (unsigned i = a; i < e; i++) {
+                    const double w = lw[i - cs];
+                    const int p = lp[i - cs];
+                    W += w;
+                    if (p >= 0) acc[p * P2G_TILE + t] += w;
+                }
+            }
+        }
+    }
+    if (!own) return;
+    const int node = l * g.nx + k;
+    const bool skip = fabs(W) < 1e-30 || (ntype && (ntype[node] == 30 || ntype[node] == 31));
+    for (int p = 0; p < nph; p++) {
+        const double v = acc[p * P2G_TILE + t];
+        perc.p[p][node] = skip ? v : v / W;
     }
 }
 
@@ -472,8 +599,12 @@ static int launch_fields(mdg_ctx *c, p2g_geo g, const p2g_set &s, int nf) {
         int need_phase = 0;
         for (int f = 0; f < nf; f++) need_phase |= (s.f[f].flag == 0);
         // node rows on cell edges in z draw from two cell rows: 4 rows a block
-        const int rows = (g.ax.zkind == VERT_AXIS) ? 4 : 1;
-        const int nbx = (g.nx + P2G_TILE - 1) / P2G_TILE, nb = nbx * ((g.nz + rows - 1) / rows);
+        // where that leaves two blocks for every CU (101^2, 3 fields: 26 blocks
+        // 70 us, 101 blocks 17 us; 2047^2 fills the chip either way, and 4
+        // rows read a cell row 1.25 times instead of twice)
+        const int nbx = (g.nx + P2G_TILE - 1) / P2G_TILE;
+        const int rows = (g.ax.zkind == VERT_AXIS && (long)nbx * g.nz >= 4 * P2G_FILL) ? 4 : 1;
+        const int nb = nbx * ((g.nz + rows - 1) / rows);
         dim3 grid(nb), block(P2G_TILE);
         const bool pre = (c->mw_state[g.set] == 1);
         const double *mw = c->mw[g.set].p;
@@ -495,8 +626,9 @@ static int launch_fields(mdg_ctx *c, p2g_geo g, const p2g_set &s, int nf) {
     if (g.R == 1 && g.S == 1 && c->mw_state[g.set] == 1) {
         // 9-cell stencil on exact homes: row tiles
         const int nbx = (g.nx + P2G_TILE - 1) / P2G_TILE, nb = nbx * g.nz;
-#define T9(NF) hipLaunchKernelGGL(k_p2g9_tile<NF>, dim3(nb), dim3(P2G_TILE), 0, c->stream, g, s, c->qoff.p, \
-                                  (const unsigned *)c->keys2.p, c->mx.p, c->mz.p, c->mphase.p, nbx, nb)
+#define T9(NF) hipLaunchKernelGGL((k_p2g9_tile<NF, false>), dim3(nb), dim3(P2G_TILE), 0, c->stream, g, s, c->qoff.p, \
+                                  (const unsigned *)c->keys2.p, c->mx.p, c->mz.p, c->mphase.p, nbx, nb, 0, \
+                                  (const signed char *)nullptr, p2g_perc{})
         switch (nf) {
         case 1: T9(1); break;
         case 2: T9(2); break;
@@ -659,19 +791,41 @@ extern "C" int mdg_p2mastah(mdg_ctx *c, const double *mat_prop, int n_mat_prop, 
             nt = c->ntype_tmp.p;
         }
     }
+    // fractions go straight to device arrays, through node_tmp to host ones
+    p2g_perc perc = {};
+    for (int p = 0; p < nb_phases; p++) {
+        if (!phase_perc[p]) return mdg_fail(c, MDG_ERR_ARG, "phase_perc[%d] is null", p);
+        perc.p[p] = mdg_is_device_ptr(phase_perc[p]) ? phase_perc[p] : c->node_tmp.p + p * nn;
+    }
+    // Row tiles need exact homes.  The 1-cell ones read cached weights, which
+    // are worked out here only where they cost less than they save at once
+    // (37.7M markers: weights 240 us and tiles 179 us against 484 us; below a
+    // million markers the extra launch and its check weigh more).
+    if (c->n_markers >= (1 << 20) && (rc = ensure_weights(c, g))) return rc;
     rc = run_checked(c, g, [&](p2g_geo &gg) {
-        hipLaunchKernelGGL(k_p2g_phase, dim3(mdg_grid1d((long)nn, 128)), dim3(128), 0, c->stream, gg,
-                           nb_phases, nt, c->qoff.p, c->mx.p, c->mz.p, c->mphase.p, c->node_tmp.p,
-                           c->flag_dev.p);
+        const int nbx = (gg.nx + P2G_TILE - 1) / P2G_TILE, nb = nbx * gg.nz;
+        const size_t lds = (size_t)nb_phases * P2G_TILE * sizeof(double);
+        const bool exact = c->mw_state[gg.set] == 1 && gg.S == gg.R;
+        if (exact && lds > 40 * 1024)   // many phases: past the 64 KB a launch gets by default
+            HIPCHK(c, hipFuncSetAttribute(gg.R == 0 ? (const void *)k_p2g_phase_tile : (const void *)k_p2g9_tile<1, true>,
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        if (exact && gg.R == 0)
+            hipLaunchKernelGGL(k_p2g_phase_tile, dim3(nb), dim3(P2G_TILE), lds, c->stream, gg, nb_phases, nt, c->qoff.p,
+                               (const double *)c->mw[gg.set].p, c->mphase.p, nbx, nb, perc);
+        else if (exact)
+            hipLaunchKernelGGL((k_p2g9_tile<1, true>), dim3(nb), dim3(P2G_TILE), lds, c->stream, gg, p2g_set{}, c->qoff.p,
+                               (const unsigned *)c->keys2.p, c->mx.p, c->mz.p, c->mphase.p, nbx, nb, nb_phases, nt, perc);
+        else
+            hipLaunchKernelGGL(k_p2g_phase, dim3(mdg_grid1d((long)nn, 128)), dim3(128), 0, c->stream, gg,
+                               nb_phases, nt, c->qoff.p, c->mx.p, c->mz.p, c->mphase.p, perc,
+                               c->flag_dev.p);
         HIPCHK(c, hipGetLastError());
         return MDG_OK;
     });
     if (rc) return rc;
-    for (int p = 0; p < nb_phases; p++) {
-        if (!phase_perc[p]) return mdg_fail(c, MDG_ERR_ARG, "phase_perc[%d] is null", p);
-        HIPCHK(c, hipMemcpyAsync(phase_perc[p], c->node_tmp.p + p * nn, nn * sizeof(double),
-                                 hipMemcpyDefault, c->stream));
-    }
+    for (int p = 0; p < nb_phases; p++)
+        if (perc.p[p] != phase_perc[p])
+            HIPCHK(c, hipMemcpyAsync(phase_perc[p], perc.p[p], nn * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return MDG_OK;
 }
