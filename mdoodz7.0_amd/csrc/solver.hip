@@ -119,6 +119,25 @@ __global__ void k_rand_free(int n, const T *__restrict__ dinv, T *__restrict__ x
     x[i] = (dinv[i] != T(0)) ? ((h & 1u) ? T(1) : T(-1)) * (T(0.5) + T((h >> 8) & 255u) / T(512)) : T(0);
 }
 
+// x = d / sqrt(yy): the normalisation of a power iteration, yy on the device
+template <typename T>
+__global__ void k_rescale(int n, const double *__restrict__ yy, const T *__restrict__ d, T *__restrict__ x) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) x[i] = (T)(1.0 / sqrt(*yy)) * d[i];
+}
+// Unit vectors e_idx[j] of length n, one after the other, and the matrix
+// A[i][j] = -r_j[idx[i]] from the residuals r_j = -A e_idx[j]
+template <typename T>
+__global__ void k_unit_cols(int n, int nf, const int *__restrict__ idx, T *__restrict__ e) {
+    const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < (size_t)n * nf) e[q] = ((int)(q % n) == idx[q / n]) ? T(1) : T(0);
+}
+template <typename T>
+__global__ void k_gather_cols(int n, int nf, const int *__restrict__ idx, const T *__restrict__ r, double *__restrict__ A) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < nf * nf) A[q] = -(double)r[(size_t)(q % nf) * n + idx[q / nf]];
+}
+
 template <typename T>
 __global__ void k_copy(int n, const T *__restrict__ a, T *__restrict__ b) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1673,6 +1692,7 @@ struct mg_hier {
     size_t small_lds = 0;
     dbuf<sm_level<T>> small;
     dbuf<double> small_ab;
+    dbuf<T> cols;                           // unit vectors and residuals of the coarsest level's assembly
     sm_coarse small_co{};
     hipGraph_t graph = nullptr;             // one CG iteration (V-cycle included)
     hipGraphExec_t exec = nullptr;
@@ -1697,7 +1717,7 @@ struct mg_hier {
         for (auto &l : L) l.release();
         L.clear();
         cg_x.release(); cg_r.release(); cg_z.release(); cg_p.release(); cg_q.release();
-        scal.release(); part.release(); small.release(); small_ab.release();
+        scal.release(); part.release(); small.release(); small_ab.release(); cols.release();
         pc_x.release(); pc_r.release(); pc_p.release(); pc_q.release(); bf_t.release();
         pscal.release(); ppart.release();
         if (h_scal) (void)hipHostFree(h_scal);
@@ -1740,12 +1760,17 @@ void mdg_solver_release(mdg_ctx *c) {
 
 static int nblk(int n) { return mdg_grid1d(n, 256); }
 
+// dot product into a device double
+template <typename T>
+static void dot_dev(mdg_ctx *c, solver_state *s, int n, const T *a, const T *b, double *out) {
+    const int nb = std::min(1024, mdg_grid1d(n, RB));
+    hipLaunchKernelGGL(k_dot_part<T>, dim3(nb), dim3(RB), 0, c->stream, n, a, b, s->part.p);
+    hipLaunchKernelGGL(k_sum_part, dim3(1), dim3(RB), 0, c->stream, nb, s->part.p, out);
+}
 // dot product into a host double (synchronising)
 template <typename T>
 static int dot_host(mdg_ctx *c, solver_state *s, int n, const T *a, const T *b, double *out) {
-    const int nb = std::min(1024, mdg_grid1d(n, RB));
-    hipLaunchKernelGGL(k_dot_part<T>, dim3(nb), dim3(RB), 0, c->stream, n, a, b, s->part.p);
-    hipLaunchKernelGGL(k_sum_part, dim3(1), dim3(RB), 0, c->stream, nb, s->part.p, s->scal.p);
+    dot_dev<T>(c, s, n, a, b, s->scal.p);
     HIPCHK(c, hipMemcpyAsync(out, s->scal.p, 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return MDG_OK;
@@ -1965,12 +1990,14 @@ static int build_hierarchy(mdg_ctx *c, solver_state *s, mg_hier<T> &H, const mdg
         ncx = ncx2;
         ncz = ncz2;
     }
-    // Chebyshev bounds: power iteration on Dinv*A_g per level
+    // Chebyshev bounds: power iteration on Dinv*A_g per level, normalised on
+    // the device; the last step's two norms come to the host once per level
+    // (read back in every step they were half of a small solve's set-up)
     for (size_t li = 0; li + 1 < H.L.size(); li++) {
         mg_level<T> &lv = H.L[li];
         hipLaunchKernelGGL(k_rand_free<T>, dim3(nblk(lv.n)), dim3(256), 0, c->stream, lv.n, (const T *)lv.dinv.p, lv.x.p);
-        double lam = 1.0;
-        for (int it = 0; it < 30; it++) {
+        const int nit = 30;
+        for (int it = 0; it < nit; it++) {
             hipLaunchKernelGGL(k_vel_residual<T>, dim3(nblk(lv.n)), dim3(256), 0, c->stream, lv.g, (T)gamma, lv.x.p,
                                (const T *)nullptr, lv.en.p, lv.es.p, lv.r.p);     // r = -A x
             if (lv.patch)
@@ -1978,18 +2005,19 @@ static int build_hierarchy(mdg_ctx *c, solver_state *s, mg_hier<T> &H, const mdg
                                    (const T *)lv.pinv.p, (const T *)lv.r.p, lv.d.p);
             else
                 hipLaunchKernelGGL(k_scale_dinv<T>, dim3(nblk(lv.n)), dim3(256), 0, c->stream, lv.n, T(-1), lv.dinv.p, lv.r.p, lv.d.p);
-            double yy, xx;
-            int rc;
-            if ((rc = dot_host<T>(c, s, lv.n, lv.d.p, lv.d.p, &yy)) || (rc = dot_host<T>(c, s, lv.n, lv.x.p, lv.x.p, &xx))) return rc;
-            lam = sqrt(yy / xx);
-            const T sc = (T)(1.0 / sqrt(yy));
-            hipLaunchKernelGGL(k_axpby<T>, dim3(nblk(lv.n)), dim3(256), 0, c->stream, lv.n, sc, lv.d.p, T(0), lv.x.p);
+            dot_dev<T>(c, s, lv.n, lv.d.p, lv.d.p, s->scal.p);
+            if (it + 1 == nit) dot_dev<T>(c, s, lv.n, lv.x.p, lv.x.p, s->scal.p + 1);
+            hipLaunchKernelGGL(k_rescale<T>, dim3(nblk(lv.n)), dim3(256), 0, c->stream, lv.n, (const double *)s->scal.p,
+                               (const T *)lv.d.p, lv.x.p);
         }
-        lv.lmax = 1.2 * lam;   // power iteration approaches lambda_max from below
+        double nrm[2];
+        HIPCHK(c, hipMemcpyAsync(nrm, s->scal.p, 16, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        lv.lmax = 1.2 * sqrt(nrm[0] / nrm[1]);   // power iteration approaches lambda_max from below
         lv.cheb_div = o->cheb_range > 0.0 ? o->cheb_range : 30.0;
     }
     // coarsest: dense inverse of A_g on its free unknowns, assembled by
-    // applying the operator to unit vectors on the device
+    // applying the operator to all unit vectors on the device, read back once
     mg_level<T> &cl = H.L.back();
     std::vector<int> idx;
     for (int i = 0; i < cl.nu; i++) if (vx_free(cl.g, i % cl.g.Nx, i / cl.g.Nx)) idx.push_back(i);
@@ -2000,21 +2028,24 @@ static int build_hierarchy(mdg_ctx *c, solver_state *s, mg_hier<T> &H, const mdg
     HIPCHK(c, cl.idx.reserve(nf));
     HIPCHK(c, hipMemcpyAsync(cl.idx.p, idx.data(), nf * 4, hipMemcpyHostToDevice, c->stream));
     std::vector<double> A((size_t)nf * nf);
-    std::vector<T> col(cl.n), e(cl.n);
-    for (int j = 0; j < nf; j++) {
-        std::fill(e.begin(), e.end(), T(0));
-        e[idx[j]] = T(1);
-        HIPCHK(c, hipMemcpyAsync(cl.x.p, e.data(), cl.n * sizeof(T), hipMemcpyHostToDevice, c->stream));
-        hipLaunchKernelGGL(k_vel_residual<T>, dim3(nblk(cl.n)), dim3(256), 0, c->stream, cl.g, (T)gamma, cl.x.p,
-                           (const T *)nullptr, cl.en.p, cl.es.p, cl.r.p);
-        HIPCHK(c, hipMemcpyAsync(col.data(), cl.r.p, cl.n * sizeof(T), hipMemcpyDeviceToHost, c->stream));
+    const size_t ncol = (size_t)nf * cl.n;
+    HIPCHK(c, H.cols.reserve(2 * ncol));
+    HIPCHK(c, cl.Ainv.reserve(A.size()));
+    if (nf > 0) {
+        hipLaunchKernelGGL(k_unit_cols<T>, dim3(mdg_grid1d((long)ncol, 256)), dim3(256), 0, c->stream, cl.n, nf,
+                           (const int *)cl.idx.p, H.cols.p);
+        for (int j = 0; j < nf; j++)
+            hipLaunchKernelGGL(k_vel_residual<T>, dim3(nblk(cl.n)), dim3(256), 0, c->stream, cl.g, (T)gamma,
+                               H.cols.p + (size_t)j * cl.n, (const T *)nullptr, cl.en.p, cl.es.p, H.cols.p + ncol + (size_t)j * cl.n);
+        hipLaunchKernelGGL(k_gather_cols<T>, dim3(mdg_grid1d((long)nf * nf, 256)), dim3(256), 0, c->stream, cl.n, nf,
+                           (const int *)cl.idx.p, (const T *)(H.cols.p + ncol), cl.Ainv.p);
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, hipMemcpyAsync(A.data(), cl.Ainv.p, A.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
-        for (int i = 0; i < nf; i++) A[(size_t)i * nf + j] = -(double)col[idx[i]];
     }
     bool ok;
     host_gauss_jordan_inverse(A, nf, &ok);
     if (!ok) return mdg_fail(c, MDG_ERR_NOT_SPD, "singular coarsest operator");
-    HIPCHK(c, cl.Ainv.reserve(A.size()));
     HIPCHK(c, hipMemcpyAsync(cl.Ainv.p, A.data(), A.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));   // A is a local host vector
     {
