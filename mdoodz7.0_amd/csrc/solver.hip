@@ -1839,6 +1839,9 @@ static void cheb_table(double lmax, double div, int deg, std::vector<double> &ab
 //          191^2   6.5 | 3.8  2.9  2.4            383^2   7.2 | 3.7  2.8  3.2
 //           95^2   5.9 | 3.8  2.8  2.3            191^2   6.1 | 2.7  2.1  1.7
 // (6 a launch on levels up to 95^2 take another 8% off the 383^2 solve.)
+// FP64 levels of more than 2M positions keep k_pcheb, whose large tiles stream
+// them: 2047^2 solve 3.96 ms per CG iteration against 4.83 with 3 a launch, while
+// the 1023^2 solve is 9% faster with them (FP32: 2.44 against 3.2 at 2047^2).
 // Jacobi, FP64, whole solves in ms, k_cheb3 against 2, 3, 4, 5, 6 a launch:
 // 101^2 52 | 53 48 44 45 43, 255^2 133 | 124 108 91 92 84, 511^2 263 | 242 209
 // 176 177 163.  An FP32 Jacobi hierarchy keeps single steps: it is there that
@@ -1847,7 +1850,7 @@ static void cheb_table(double lmax, double div, int deg, std::vector<double> &ab
 template <typename T>
 static int multi_steps(const sgrid &g, bool patch) {
     const long n = (long)g.Nx * (g.Nz + 1);
-    if (patch) return n <= 12000 ? 6 : (n <= 40000 ? 4 : 3);
+    if (patch) return n <= 12000 ? 6 : (n <= 40000 ? 4 : (sizeof(T) == 4 || n <= 2000000 ? 3 : 0));
     return sizeof(T) == 8 ? 6 : 0;
 }
 
