@@ -81,7 +81,7 @@ extern "C" void mdg_destroy(mdg_ctx *c) {
     c->BCu_t.release(); c->BCv_t.release(); c->BCp_t.release(); c->BCg_t.release();
     c->BCu_v.release(); c->BCv_v.release();
     c->mx.release(); c->mz.release(); c->mphase.release(); c->perm.release();
-    c->qoff.release(); c->keys.release(); c->keys2.release(); c->idx.release();
+    c->qoff.release(); c->keys.release(); c->keys2.release();
     for (auto &b : c->mw) b.release();
     c->sort_tmp.release(); c->field_tmp.release(); c->node_tmp.release();
     c->table_tmp.release(); c->ntype_tmp.release(); c->flag_dev.release();

@@ -66,7 +66,6 @@ struct mdg_ctx {
     int               mw_state[4] = {0, 0, 0, 0};
     double            weights_ms = 0.0;
     dbuf<unsigned>    keys, keys2;   // sort scratch
-    dbuf<int>         idx;           // sort scratch
     dbuf<unsigned char> sort_tmp;
     // P2G scratch
     dbuf<double>      field_tmp;     // per-marker field in sorted order
