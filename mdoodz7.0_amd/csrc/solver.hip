@@ -1026,15 +1026,18 @@ __global__ void __launch_bounds__(CM_R *CM_R) k_cheb_multi(sgrid g, stc<T> cf, T
     xs[0][p] = xu;
     vs[0][p] = xv;
     __syncthreads();
-    // residual of the thread's two rows from LDS copy `c` of x
+    // residual of the thread's two rows from LDS copy `c` of x; the two rows
+    // share six of their sixteen neighbours (its own two faces among them),
+    // and LDS reads are what a step's threads queue for (16 reads -> 10: launches
+    // of the 383^2 FP64 hierarchy 14.0 -> 13.1 us on average)
     auto residual = [&](int c, T &qu, T &qv) {
         const T *u = xs[c] + p, *v = vs[c] + p;
+        const T uw = u[-1], ue = u[1], us = u[-CM_W], un = u[CM_W], unw = u[CM_W - 1];
+        const T vw = v[-1], ve = v[1], vso = v[-CM_W], vn = v[CM_W], vse = v[1 - CM_W];
         qu = bu;
         qv = bv;
-        if (fu)
-            qu -= vx_apply9(ru, cf, xu, u[-1], u[1], u[-CM_W], u[CM_W], v[-CM_W], v[1 - CM_W], v[0], v[1]);
-        if (fv)
-            qv -= vz_apply9(rv, cf, xv, v[-1], v[1], v[-CM_W], v[CM_W], u[-1], u[0], u[CM_W - 1], u[CM_W]);
+        if (fu) qu -= vx_apply9(ru, cf, xu, uw, ue, us, un, vso, vse, xv, ve);
+        if (fv) qv -= vz_apply9(rv, cf, xv, vw, ve, vso, vn, uw, xu, unw, un);
     };
     int cur = 0;
     for (int s = 0; s < st.n; s++) {
@@ -1109,7 +1112,7 @@ __global__ void __launch_bounds__(CM_R *CM_R) k_cheb_multi(sgrid g, stc<T> cf, T
 // jump of 1e6) gains iterations.
 // Bound: LDS reads (ten neighbours per position and step) and the barriers,
 // about 0.4 us a step on 26^2.  The levels below 47^2 of a 383^2 hierarchy take
-// 44 us per V-cycle in it where their kernels took 110 us; the solve of the
+// 46 us per V-cycle in it where their kernels took 110 us; the solve of the
 // 101^2 inclusion went from 75.4 to 55.4 ms, of 383^2 ellipses (FP64, patches)
 // from 400 to 364 ms, of 767^2 (mixed) from 734 to 659 ms.  The limit of 1024
 // positions is one per thread; 47^2 in here would cost its 24 steps 3 x 0.4 us
@@ -1163,14 +1166,16 @@ __device__ __forceinline__ void sm_smooth(const sm_level<T> &L, double gamma, bo
         const double a = s ? ab[2 * s - 1] : 0.0, cc = s ? ab[2 * s] : ab[0];
         double yu = xu, yv = xv, qu = bu, qv = bv;
         if (!(zero && s == 0)) {
-            const double *u = cur, *v = cur + L.nu;
-            if (fu) {
-                const double vsw = v[iv - L.nu - NxV], vse = v[iv - L.nu - NxV + 1], vnw = v[iv - L.nu], vne = v[iv - L.nu + 1];
-                qu -= vx_apply9(ru, L.cf, xu, u[iu - 1], u[iu + 1], u[iu - Nx], u[iu + Nx], vsw, vse, vnw, vne);
-            }
-            if (fv) {
-                const int j = iv - L.nu;
-                qv -= vz_apply9(rv, L.cf, xv, v[j - 1], v[j + 1], v[j - NxV], v[j + NxV], u[iu - 1], u[iu], u[iu - 1 + Nx], u[iu + Nx]);
+            // ten neighbours for the two rows (LDS reads bound a step; with 16 the
+            // kernel took 47.9 us on a 383^2 hierarchy, now 45.7): faces
+            // next to a free one, so inside the level's arrays, but for v's
+            // row Nz, read past its end (into the next array) and not used
+            if (fu || fv) {
+                const double *u = cur + iu, *v = cur + iv;
+                const double uw = u[-1], ue = u[1], us = u[-Nx], un = u[Nx], unw = u[Nx - 1];
+                const double vw = v[-1], ve = v[1], vso = v[-NxV], vn = v[NxV], vse = v[1 - NxV];
+                if (fu) qu -= vx_apply9(ru, L.cf, xu, uw, ue, us, un, vso, vse, xv, ve);
+                if (fv) qv -= vz_apply9(rv, L.cf, xv, vw, ve, vso, vn, uw, xu, unw, un);
             }
         }
         if (fu) yu += cc * (qu * du) + a * (xu - pu);
