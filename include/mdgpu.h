@@ -328,7 +328,8 @@ typedef struct {
                               around each cell (0)                              */
     double poisson_tol;    /* BFBt pressure-Poisson CG tolerance (1e-3)        */
     int    poisson_max_its;/* (30)                                             */
-    int    smoother;       /* 0 fused three-term Chebyshev kernels, 1 the
+    int    smoother;       /* 0 fused three-term Chebyshev kernels (one or
+                              several steps per launch), 1 the
                               residual/update two-kernel form, 2 the two-kernel
                               form preconditioned by vertex-patch additive
                               Schwarz (exact solves on the four faces around
@@ -336,7 +337,9 @@ typedef struct {
                               modes the penalty term leaves to the smoother)
                               instead of the diagonal, 3 the same patch
                               preconditioning fused into one kernel per step
-                              with the patch systems solved in the kernel (0) */
+                              with the patch systems solved in the kernel, or
+                              several steps per launch with the stored patch
+                              inverses (0)                                    */
     int    cheb_degree_coarse; /* smoothing degree on every level below the
                               finest (16)                                      */
     double cheb_range;     /* the Chebyshev smoother targets eigenvalues of
@@ -347,7 +350,8 @@ typedef struct {
                               HIP graph, 1 launch its kernels one by one (for
                               profilers that do not trace graph nodes), 2 as 1
                               with HIP events around every fine-level
-                              smoother step (smoother_ms below) (0)           */
+                              smoother step, launched one by one
+                              (smoother_ms below) (0)                         */
     /* outputs */
     int    its, inner_its, poisson_its, levels, status;
     double rel_res, time_ms;

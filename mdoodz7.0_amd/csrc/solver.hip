@@ -24,7 +24,8 @@
 // tolerance; an FP32 preconditioner only needs to be a good approximate
 // inverse, and the FP64 CG around it keeps its attainable accuracy.
 // Smoothing uses the three-term Chebyshev recurrence on the iterates, one
-// fused stencil kernel per step (k_cheb3).
+// fused stencil kernel per step (k_cheb3, k_pcheb) or several steps per launch
+// (k_cheb_multi); the smallest levels run in one workgroup (k_small_cycle).
 #include <cmath>
 #include <memory>
 #include <type_traits>
