@@ -76,16 +76,16 @@ k_tangent_grid(rheo_ctl md, const rheo_phase *__restrict__ phases, int n,
     double e = 0.0, der[4] = {0.0, 0.0, 0.0, 0.0};
     for (int p = 0; p < md.nph; p++) {
         const double w = f.perc[(size_t)p * n + i];
-        if (!(fabs(w) > 1e-13)) continue;
+        const bool on = fabs(w) > 1e-13;
+        if (!__any(on)) continue;
         const rheo_phase &m = sph[p];
         const friction fr = friction_at(m, f, i);
         const double co = f.C ? f.C[i] : m.m.C;
-        creep_laws L = laws_at<EXT>(m, md, G, T, P, dg, phi, pref, bad);
+        creep_laws L = laws_at<EXT>(m, md, on, G, T, P, dg, phi, pref, bad);
         double eb, Pc, Epl;
-        viscosity_concise<EXT>(m, L, md, P, dg, Exx, Ezz, Exz, fr, co, eb, Pc, Epl, bad);
-        if (md.average == 0) e += w * eb;
-        else if (md.average == 1) e += w / eb;
-        else e += w * log(eb);
+        viscosity_concise<EXT>(m, L, md, on, P, dg, Exx, Ezz, Exz, fr, co, eb, Pc, Epl, bad);
+        const double a = (md.average == 0) ? w * eb : (md.average == 1) ? w / eb : w * log(eb);
+        e = on ? e + a : e;
         double ep = 0.0;
         const int ns = (m.p_free && !(m.m.plast == 1 && md.step != 0)) ? 6 : 8;
 #pragma unroll 1
@@ -93,9 +93,9 @@ k_tangent_grid(rheo_ctl md, const rheo_phase *__restrict__ phases, int n,
             const int q = s >> 1;
             const double h = (q == 0) ? px : (q == 1) ? pz : (q == 2) ? pg : pp, dl = (s & 1) ? -h : h;
             const double Pq = P + (q == 3 ? dl : 0.0);
-            if (q == 3 && !m.p_free) L = laws_at<EXT>(m, md, G, T, Pq, dg, phi, pref, bad);
+            if (q == 3 && !m.p_free) L = laws_at<EXT>(m, md, on, G, T, Pq, dg, phi, pref, bad);
             double es;
-            viscosity_concise<EXT>(m, L, md, Pq, dg, Exx + (q == 0 ? dl : 0.0), Ezz + (q == 1 ? dl : 0.0),
+            viscosity_concise<EXT>(m, L, md, on, Pq, dg, Exx + (q == 0 ? dl : 0.0), Ezz + (q == 1 ? dl : 0.0),
                                    Exz + (q == 2 ? dl : 0.0), fr, co, es, Pc, Epl, bad);
             if (!(s & 1)) {
                 ep = es;
@@ -104,12 +104,13 @@ k_tangent_grid(rheo_ctl md, const rheo_phase *__restrict__ phases, int n,
             double v = w * (ep - es) / ((q == 2) ? 4.0 * h : 2.0 * h);
             if (md.average == 1) v /= eb * eb;
             else if (md.average == 2) v /= eb;
+            v = on ? v : 0.0;
             der[0] += (q == 0) ? v : 0.0;
             der[1] += (q == 1) ? v : 0.0;
             der[2] += (q == 2) ? v : 0.0;
             der[3] += (q == 3) ? v : 0.0;
         }
-        if (ns == 6) der[3] += w * 0.0 / (2.0 * pp);
+        if (ns == 6) der[3] += on ? w * 0.0 / (2.0 * pp) : 0.0;
     }
     if (md.average == 1) e = 1.0 / e;
     else if (md.average == 2) e = exp(e);

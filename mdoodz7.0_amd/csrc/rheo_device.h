@@ -43,6 +43,17 @@ inline rheo_phase make_phase(const mdg_phase_prop &m) {
     return r;
 }
 
+// Control flow in the evaluation is the wave's: a branch or loop is entered by
+// all lanes when one of them needs it, and the lanes that do not keep their
+// values through selects (`on`: the node has the phase; `run`: its iteration
+// goes on).  A branch per lane is not safe here.  hipcc 7.2 keeps a test that
+// is the same for all lanes (whether the phase has a law) as a mask of the
+// lanes active where it is first compared.  With a break per lane in local_ve
+// that was inside the loop, the tangent's evaluations at perturbed states read
+// the mask again, and where the base state's longest lanes had finished there
+// the others took a law that the phase does not have (a viscosity of zero).
+// Made by all lanes, a compare leaves no partial mask.
+
 // The library's pow as a call: with its dozen copies inlined k_tangent_grid<true>
 // has 11500 instructions, past the 64 KB instruction cache, and 118 spilled
 // scalars; as calls 4500 and 60.
@@ -58,8 +69,8 @@ __device__ __forceinline__ double pow_k(double x, double n, int k) {
 }
 // x^e where e may be zero (laws without that factor): exactly 1, as pow gives
 __device__ __forceinline__ double pow_or_1(double x, double e) { return e == 0.0 ? 1.0 : pow_call(x, e); }
-// exp(e) where e is zero (no melt): exactly 1
-__device__ __forceinline__ double exp_or_1(double e) { return e == 0.0 ? 1.0 : exp(e); }
+// exp(e) where e is zero (no melt): exactly 1, as exp gives
+__device__ __forceinline__ double exp_or_1(double e) { return __any(e != 0.0) ? exp(e) : 1.0; }
 
 // The creep laws active at one (node, phase) and their coefficients, which
 // depend on temperature, pressure, grain size and melt but not on the strain
@@ -76,35 +87,36 @@ struct creep_laws {
 // T = 2 eta_ve E.  The grain-boundary-sliding term of the reference is
 // C_gbs T^n_gbs with C_gbs never set (zero), so it is absent here.  Returns
 // false when the reference would exit (20 iterations, res > tol).
-// The loops here end for the wave as a whole, lanes that are done masked out:
-// with a break per lane inside the tangent's loop over perturbations, hipcc 7.2
-// gave lanes that left in different trips wrong viscosities.
-__device__ __forceinline__ bool local_ve(const creep_laws &L, double Eii, double &eta, double &Eii_pwl,
+__device__ __forceinline__ bool local_ve(const creep_laws &L, bool on, double Eii, double &eta, double &Eii_pwl,
                                          double &Eii_exp, double &Eii_lin) {
     constexpr double tol = 1.0e-11, stop = tol / 100;
     double res = INFINITY;
-    for (int it = 0; it < 20 && __any(!(res < stop)); it++) {
-        if (res < stop) continue;
+    bool run = on;
+    for (int it = 0; it < 20; it++) {
         const double Tii = 2.0 * eta * Eii;
         const double e_cst = L.constant ? Tii / 2.0 / L.eta_cst : 0.0;
         const double e_pwl = L.dislocation ? L.C_pwl * pow_k(Tii, L.n_pwl, L.k_pwl) : 0.0;
-        const double e_exp = L.peierls ? L.C_exp * pow_call(Tii, L.nST) : 0.0;
+        const double t_exp = __any(L.peierls) ? L.C_exp * pow_call(Tii, L.nST) : 0.0;
+        const double e_exp = L.peierls ? t_exp : 0.0;
         const double e_lin = L.diffusion ? L.C_lin * pow_k(Tii, L.n_lin, L.k_lin) * L.dm_lin : 0.0;
-        Eii_pwl = e_pwl;
-        Eii_exp = e_exp;
-        Eii_lin = e_lin;
+        Eii_pwl = run ? e_pwl : Eii_pwl;
+        Eii_exp = run ? e_exp : Eii_exp;
+        Eii_lin = run ? e_lin : Eii_lin;
         const double r = Eii - (L.elastic ? 1.0 : 0.0) * Tii / (2.0 * L.eta_el) - (e_pwl + e_exp + e_lin + e_cst);
-        res = fabs(r / Eii);
-        if (res < stop) continue;
+        res = run ? fabs(r / Eii) : res;
+        run = run && !(res < stop);
+        if (!__any(run)) break;
         double dfdeta = 0.0;
         if (L.elastic) dfdeta += -Eii / L.eta_el;
-        if (L.peierls) dfdeta += -e_exp * L.nST / eta;
+        const double d_exp = __any(L.peierls) ? dfdeta + -e_exp * L.nST / eta : 0.0;
+        dfdeta = L.peierls ? d_exp : dfdeta;
         if (L.diffusion) dfdeta += -e_lin * L.n_lin / eta;
         if (L.dislocation) dfdeta += -e_pwl * L.n_pwl / eta;
         if (L.constant) dfdeta += -Eii / L.eta_cst;
-        eta -= r / dfdeta;
+        const double next = eta - r / dfdeta;
+        eta = run ? next : eta;
     }
-    return !(res > tol);
+    return !on || !(res > tol);
 }
 
 // Failure codes of viscosity_concise, or-ed into the caller's flag.
@@ -118,8 +130,8 @@ constexpr int FAIL_GRAIN_SIZE = 2;     // d < d_min with m_lin > 0 (reference ex
 // 1 and the laws absent, so the results are the same bits), which keeps
 // the register count, and the occupancy, of the constant + power-law case.
 template <bool EXT>
-__device__ __forceinline__ creep_laws laws_at(const rheo_phase &ph, const rheo_ctl &md, double G, double T, double P, double d,
-                                              double phi, double pref_mult, int &fail) {
+__device__ __forceinline__ creep_laws laws_at(const rheo_phase &ph, const rheo_ctl &md, bool on, double G, double T, double P,
+                                              double d, double phi, double pref_mult, int &fail) {
     const mdg_phase_prop &m = ph.m;
     creep_laws L = {};
     const double dt = (md.step == 0) ? 1e100 : md.dt;
@@ -135,7 +147,7 @@ __device__ __forceinline__ creep_laws laws_at(const rheo_phase &ph, const rheo_c
     L.k_lin = ph.k_lin;
     L.n_pwl = m.n_pwl;
     L.n_lin = m.n_lin;
-    if (T < md.zeroC) T = md.zeroC;
+    T = T < md.zeroC ? md.zeroC : T;
     if (L.dislocation) {                                               // :501-504
         L.B_pwl = m.pref_pwl * pref_mult * m.F_pwl * ph.A_pwl * exp((m.Q_pwl + P * m.V_pwl) / md.R / m.n_pwl / T);
         if (EXT)
@@ -144,7 +156,7 @@ __device__ __forceinline__ creep_laws laws_at(const rheo_phase &ph, const rheo_c
     }
     L.dm_lin = 1.0;
     if (L.diffusion) {                                                 // :505-512, d enters below
-        if (m.m_lin > 0.0 && d < md.d_min) fail |= FAIL_GRAIN_SIZE;
+        fail |= (on && m.m_lin > 0.0 && d < md.d_min) ? FAIL_GRAIN_SIZE : 0;
         L.B_lin = m.F_lin * ph.A_lin * exp((m.Q_lin + P * m.V_lin) / md.R / m.n_lin / T) * ph.f_lin *
                   exp_or_1(-m.a_lin * phi / m.n_lin);
         L.C_lin = L.k_lin ? 1.0 / pow_k(2.0 * L.B_lin, m.n_lin, L.k_lin) : pow_call(2.0 * L.B_lin, -m.n_lin);
@@ -154,7 +166,7 @@ __device__ __forceinline__ creep_laws laws_at(const rheo_phase &ph, const rheo_c
         L.B_gbs = m.F_gbs * ph.A_gbs * exp((m.Q_gbs + P * m.V_gbs) / md.R / m.n_gbs / T) *
                   pow_or_1(d, m.m_gbs / m.n_gbs) * ph.f_gbs * exp_or_1(-m.a_gbs * phi / m.n_gbs);
     L.nST = m.n_exp;
-    if (L.peierls) {                                                   // :516-523
+    if (__any(L.peierls)) {                                            // :516-523
         const double g = m.G_exp;
         const double ST = m.Q_exp / md.R / T * 2.0 * g * (1 - g);
         const double Arr = exp(-m.Q_exp / md.R / T * ((1.0 - g) * (1.0 - g)));
@@ -167,16 +179,15 @@ __device__ __forceinline__ creep_laws laws_at(const rheo_phase &ph, const rheo_c
 }
 
 // ViscosityConcise (RheologyDensity.c:385-1080) for one (node, phase) with
-// the laws of laws_at: returns the dissipative viscosity; etaVE, Pcorr,
-// Eii_pl and the visco-elastic viscosity before plasticity by reference.
-// WARM starts the visco-elastic iterations from eta_ve.  fr holds sin and cos
-// of the friction angle and sin of the dilation angle.
+// the laws of laws_at: returns the dissipative viscosity; etaVE, Pcorr and
+// Eii_pl by reference.  fr holds sin and cos of the friction angle and sin of
+// the dilation angle.
 struct friction {
     double sin_fric, cos_fric, sin_dil;
 };
 template <bool EXT>
-__device__ __forceinline__ double viscosity_concise(const rheo_phase &ph, const creep_laws &L, const rheo_ctl &md, double P,
-                                                    double d, double Exx, double Ezz, double Exz, const friction &fr,
+__device__ __forceinline__ double viscosity_concise(const rheo_phase &ph, const creep_laws &L, const rheo_ctl &md, bool on,
+                                                    double P, double d, double Exx, double Ezz, double Exz, const friction &fr,
                                                     double C, double &etaVE, double &Pcorr, double &Eii_pl,
                                                     int &fail) {
     const mdg_phase_prop &m = ph.m;
@@ -186,56 +197,57 @@ __device__ __forceinline__ double viscosity_concise(const rheo_phase &ph, const 
     const double sin_fric = fr.sin_fric, sin_dil = L.elastic ? fr.sin_dil : 0.0;
     const double Eyy = -(Exx + Ezz);
     double Eii = sqrt(0.5 * (Exx * Exx + Ezz * Ezz + Eyy * Eyy) + Exz * Exz);   // :457-459
-    if (Eii * md.scale_E < 1e-30) Eii = 1e-30 / md.scale_E;
+    Eii = Eii * md.scale_E < 1e-30 ? 1e-30 / md.scale_E : Eii;
     Pcorr = P;
     double Tyield = 0.0;
     if (plastic) {                                                     // :530-539
         Tyield = C * fr.cos_fric + P * sin_fric;
-        if (m.Slim < Tyield) Tyield = m.Slim;
+        Tyield = m.Slim < Tyield ? m.Slim : Tyield;
     }
     double eta_up = 1.0e100 / md.scale_eta;                        // :585-592
     if (L.constant) eta_up = fmin(eta_up, L.eta_cst);
     if (L.dislocation) eta_up = fmin(eta_up, L.B_pwl * pow_call(Eii, 1.0 / m.n_pwl - 1.0));
     if (L.elastic) eta_up = fmin(eta_up, L.eta_el);
-    if (L.peierls) eta_up = fmin(eta_up, L.B_exp * pow_call(Eii, 1.0 / L.nST - 1.0));
+    if (__any(L.peierls)) {
+        const double up = fmin(eta_up, L.B_exp * pow_call(Eii, 1.0 / L.nST - 1.0));
+        eta_up = L.peierls ? up : eta_up;
+    }
     if (L.diffusion)
         eta_up = fmin(eta_up, L.B_lin * pow_or_1(Eii, 1.0 / m.n_lin - 1.0) * pow_or_1(d, m.m_lin / m.n_lin));
     if (L.gbs) eta_up = fmin(eta_up, L.B_gbs * pow_call(Eii, 1.0 / m.n_gbs - 1.0));
     double eta_ve = eta_up;
     double Eii_pwl = 0.0, Eii_exp = 0.0, Eii_lin = 0.0;
-    if (!local_ve(L, Eii, eta_ve, Eii_pwl, Eii_exp, Eii_lin)) fail |= FAIL_LOCAL_ITER;
+    fail |= local_ve(L, on, Eii, eta_ve, Eii_pwl, Eii_exp, Eii_lin) ? 0 : FAIL_LOCAL_ITER;
     double Tii = 2.0 * eta_ve * Eii;
     bool is_pl = false;
     double eta_vep = eta_ve, gdot = 0.0;
     if (plastic) {                                                     // :655-707
-        double F_trial = Tii - Tyield;
-        if (F_trial > 1e-17) {
-            is_pl = true;
-            const double F0 = F_trial, tol = md.eta_tol;
+        const double F0 = Tii - Tyield, tol = md.eta_tol;
+        is_pl = on && F0 > 1e-17;
+        if (__any(is_pl)) {
             const double Kdt_ss = K * dt * sin_fric * sin_dil;
-            double eta_vp = m.eta_vp * pow_or_1(Eii, 1.0 / m.n_vp - 1);
-            gdot = F_trial / (eta_ve + eta_vp + Kdt_ss);
+            double g = F0 / (eta_ve + m.eta_vp * pow_or_1(Eii, 1.0 / m.n_vp - 1) + Kdt_ss);
             double Pc = P, Tiic = Tii;
-            bool done = false;
-            for (int it = 0; it < 20 && __any(!done); it++) {
-                if (done) continue;
-                Pc = P + K * dt * (gdot * sin_dil);
-                eta_vp = m.eta_vp * pow_or_1(fabs(gdot), 1.0 / m.n_vp - 1.0);
-                Tyield = Tyield + gdot * eta_vp;    // accumulates, as in the reference
-                Tiic = Tii - eta_ve * gdot;
-                F_trial = Tiic - Tyield;
-                const double res = fabs(F_trial);
-                done = res < tol || res / F0 < tol;
-                if (!done) gdot -= F_trial / (-eta_ve - eta_vp / m.n_vp - Kdt_ss);
+            bool run = is_pl;
+            for (int it = 0; it < 20; it++) {
+                const double eta_vp = m.eta_vp * pow_or_1(fabs(g), 1.0 / m.n_vp - 1.0);
+                Pc = run ? P + K * dt * (g * sin_dil) : Pc;
+                Tyield = run ? Tyield + g * eta_vp : Tyield;    // accumulates, as in the reference
+                Tiic = run ? Tii - eta_ve * g : Tiic;
+                const double F_trial = Tiic - Tyield, res = fabs(F_trial);
+                run = run && !(res < tol || res / F0 < tol);
+                if (!__any(run)) break;
+                const double next = g - F_trial / (-eta_ve - eta_vp / m.n_vp - Kdt_ss);
+                g = run ? next : g;
             }
-            if (Tiic < 0.0) {                                          // :694-701
-                gdot = (Tii - md.Tiimin) / eta_ve;
-                Tiic = md.Tiimin;
-                Pc = P;
-            }
-            Pcorr = Pc;
+            const bool neg = Tiic < 0.0;                               // :694-701
+            g = neg ? (Tii - md.Tiimin) / eta_ve : g;
+            Tiic = neg ? md.Tiimin : Tiic;
+            Pc = neg ? P : Pc;
+            gdot = is_pl ? g : 0.0;
+            Pcorr = is_pl ? Pc : P;
             eta_vep = Tiic / (2.0 * Eii);
-            Tii = Tiic;
+            Tii = is_pl ? Tiic : Tii;
         }
     }
     etaVE = is_pl ? eta_vep : eta_ve;                                  // :962-970
@@ -243,16 +255,22 @@ __device__ __forceinline__ double viscosity_concise(const rheo_phase &ph, const 
     // dissipative viscosity (:987-1032): each law's viscosity at its own
     // strain-rate share; diffusion creep at the phase's reference grain size
     double inv = 0.0;
-    if (L.peierls) inv += 1.0 / (L.B_exp * pow_call(Eii_exp, 1.0 / L.nST - 1.0));
+    if (__any(L.peierls)) {
+        const double i_exp = 1.0 / (L.B_exp * pow_call(Eii_exp, 1.0 / L.nST - 1.0));
+        inv = L.peierls ? i_exp : inv;
+    }
     if (L.dislocation) inv += 1.0 / (L.B_pwl * pow_call(Eii_pwl, 1.0 / m.n_pwl - 1.0));
     if (L.diffusion)
         inv += 1.0 / (L.B_lin * pow_or_1(Eii_lin, 1.0 / m.n_lin - 1.0) * pow_or_1(m.gs_ref, m.m_lin / m.n_lin));
     if (L.constant) inv += 1.0 / L.eta_cst;
-    if (is_pl) inv += 1.0 / (Tii / gdot);
+    if (__any(is_pl)) {
+        const double i_pl = inv + 1.0 / (Tii / gdot);
+        inv = is_pl ? i_pl : inv;
+    }
     double eta = 1.0 / inv;
     etaVE = fmax(fmin(etaVE, md.max_eta), md.min_eta);                 // :1058-1073
-    if (eta > md.max_eta) eta = md.max_eta;
-    if (eta < md.min_eta) eta = md.min_eta;
+    eta = eta > md.max_eta ? md.max_eta : eta;
+    eta = eta < md.min_eta ? md.min_eta : eta;
     return eta;
 }
 

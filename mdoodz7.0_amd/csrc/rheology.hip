@@ -59,17 +59,20 @@ k_viscosity_grid(rheo_ctl md, const rheo_phase *__restrict__ phases, int n,
     int bad = 0;
     for (int p = 0; p < md.nph; p++) {
         const double w = f.perc[(size_t)p * n + i];
-        if (!(fabs(w) > 1e-13)) continue;                              // :1212-1215
+        const bool on = fabs(w) > 1e-13;                               // :1212-1215
+        if (!__any(on)) continue;
         const rheo_phase &m = sph[p];
-        double etaVE, Pcorr, Eii_pl;
-        const creep_laws L = laws_at<EXT>(m, md, G, T, P, dg, phi, pref, bad);
-        const double eta = viscosity_concise<EXT>(m, L, md, P, dg, Exx, Ezz, Exz, friction_at(m, f, i),
-                                                         f.C ? f.C[i] : m.m.C, etaVE, Pcorr, Eii_pl, bad);
-        if (md.average == 0) { e += w * etaVE; ep += w * eta; }
-        else if (md.average == 1) { e += w / etaVE; ep += w / eta; }
-        else { e += w * log(etaVE); ep += w * log(eta); }
-        pc += w * Pcorr;
-        epl += w * Eii_pl;
+        double etaVE, Pcorr, Eii_pl, a, b;
+        const creep_laws L = laws_at<EXT>(m, md, on, G, T, P, dg, phi, pref, bad);
+        const double eta = viscosity_concise<EXT>(m, L, md, on, P, dg, Exx, Ezz, Exz, friction_at(m, f, i),
+                                                  f.C ? f.C[i] : m.m.C, etaVE, Pcorr, Eii_pl, bad);
+        if (md.average == 0) { a = w * etaVE; b = w * eta; }
+        else if (md.average == 1) { a = w / etaVE; b = w / eta; }
+        else { a = w * log(etaVE); b = w * log(eta); }
+        e = on ? e + a : e;
+        ep = on ? ep + b : ep;
+        pc = on ? pc + w * Pcorr : pc;
+        epl = on ? epl + w * Eii_pl : epl;
     }
     if (md.average == 1) { e = 1.0 / e; ep = 1.0 / ep; }
     else if (md.average == 2) { e = exp(e); ep = exp(ep); }
