@@ -800,11 +800,14 @@ extern "C" int mdg_p2mastah(mdg_ctx *c, const double *mat_prop, int n_mat_prop, 
         if (!phase_perc[p]) return mdg_fail(c, MDG_ERR_ARG, "phase_perc[%d] is null", p);
         perc.p[p] = mdg_is_device_ptr(phase_perc[p]) ? phase_perc[p] : c->node_tmp.p + p * nn;
     }
-    // Row tiles need exact homes.  The 1-cell ones read cached weights, which
-    // are worked out here only where they cost less than they save at once
-    // (37.7M markers: weights 240 us and tiles 179 us against 484 us; below a
-    // million markers the extra launch and its check weigh more).
-    if (c->n_markers >= (1 << 20) && (rc = ensure_weights(c, g))) return rc;
+    // Row tiles need exact homes.  The 9-cell ones sum in another order than the
+    // general path, so the node set's state is always worked out for them: which
+    // kernel runs, and the bits, must not depend on the calls before.  The 1-cell
+    // ones sum in the general path's order and read cached weights, which are
+    // worked out here only where they cost less than they save at once (37.7M
+    // markers: weights 240 us and tiles 179 us against 484 us; below a million
+    // markers the extra launch and its check weigh more).
+    if ((g.R == 1 || c->n_markers >= (1 << 20)) && (rc = ensure_weights(c, g))) return rc;
     rc = run_checked(c, g, [&](p2g_geo &gg) {
         const int nbx = (gg.nx + P2G_TILE - 1) / P2G_TILE, nb = nbx * gg.nz;
         const size_t lds = (size_t)nb_phases * P2G_TILE * sizeof(double);
