@@ -143,6 +143,7 @@ extern "C" int mdg_set_bc(mdg_ctx *c, const signed char *BCu_t, const double *BC
     };
     int rc;
     if ((rc = check(BCu_t, nu, "BCu_t")) || (rc = check(BCv_t, nv, "BCv_t"))) return rc;
+    c->air_nodes = true;   // until the tags below have been looked at, also if a copy is refused
     if ((rc = copy_any(c, c->BCu_t, BCu_t, nu)) || (rc = copy_any(c, c->BCu_v, BCu_v, nu)) ||
         (rc = copy_any(c, c->BCv_t, BCv_t, nv)) || (rc = copy_any(c, c->BCv_v, BCv_v, nv)) ||
         (rc = copy_any(c, c->BCp_t, BCp_t, np)) || (rc = copy_any(c, c->BCg_t, BCg_t, ng)))

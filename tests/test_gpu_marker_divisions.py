@@ -76,3 +76,16 @@ def test_grid_to_markers(oracle_mod, name, tagged):
     ctx.update_particle_stress(*grids, x, z, ph, *got)
     for a, b in zip(got, ref):
         assert np.array_equal(_bits(a), _bits(b))
+
+
+def test_tags_of_a_refused_set_bc(oracle_mod):
+    """A set_bc that is refused for its last array has replaced the centre tags
+    all the same: the grid -> marker kernels read them."""
+    O = oracle_mod
+    g, ctx, x, z, ph = _box(O, "unit")
+    ctx.set_bc(g.BCu_t, g.BCu_v, g.BCv_t, g.BCv_v, g.BCp_t, g.BCg_t)
+    g.BCp_t[-4 * (g.Nx - 1):] = 30
+    arrays = [np.ascontiguousarray(a) for a in (g.BCu_t, g.BCu_v, g.BCv_t, g.BCv_v, g.BCp_t)]
+    assert ctx._L.mdg_set_bc(ctx.h, *[mdgpu.ptr(a) for a in arrays], None) != 0
+    F = np.random.default_rng(10).standard_normal(g.BCp_t.size)
+    assert np.array_equal(_bits(ctx.g2p_centroids(F, x, z, ph)), _bits(O.g2p_centroids(g, F, x, z, ph)))
