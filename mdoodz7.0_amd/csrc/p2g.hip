@@ -813,8 +813,10 @@ extern "C" int mdg_p2mastah(mdg_ctx *c, const double *mat_prop, int n_mat_prop, 
         const size_t lds = (size_t)nb_phases * P2G_TILE * sizeof(double);
         const bool exact = c->mw_state[gg.set] == 1 && gg.S == gg.R;
         if (exact && lds > 40 * 1024)   // many phases: past the 64 KB a launch gets by default
+            // (the attribute is the process's: the most phases' size, not this call's)
             HIPCHK(c, hipFuncSetAttribute(gg.R == 0 ? (const void *)k_p2g_phase_tile : (const void *)k_p2g9_tile<1, true>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          P2G_MAXPH * P2G_TILE * (int)sizeof(double)));
         if (exact && gg.R == 0)
             hipLaunchKernelGGL(k_p2g_phase_tile, dim3(nb), dim3(P2G_TILE), lds, c->stream, gg, nb_phases, nt, c->qoff.p,
                                (const double *)c->mw[gg.set].p, c->mphase.p, nbx, nb, perc);

@@ -1913,7 +1913,8 @@ static int plan_small(mdg_ctx *c, mg_hier<T> &H, const mdg_solver_opts *o) {
     const mg_level<T> &cl = H.L.back();
     H.small_co = sm_coarse{cl.nfree, od, cl.idx.p, cl.Ainv.p};
     H.small_lds = ((size_t)od + ov) * 8;
-    HIPCHK(c, hipFuncSetAttribute((const void *)k_small_cycle<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)H.small_lds));
+    // the attribute is the process's: one value for all, whatever this hierarchy needs
+    HIPCHK(c, hipFuncSetAttribute((const void *)k_small_cycle<T>, hipFuncAttributeMaxDynamicSharedMemorySize, SM_LDS_MAX));
     H.small_from = from;
     return MDG_OK;
 }
