@@ -90,7 +90,7 @@ struct creep_laws {
 __device__ __forceinline__ bool local_ve(const creep_laws &L, bool on, double Eii, double &eta, double &Eii_pwl,
                                          double &Eii_exp, double &Eii_lin) {
     constexpr double tol = 1.0e-11, stop = tol / 100;
-    double res = INFINITY;
+    double res = 0.0;
     bool run = on;
     for (int it = 0; it < 20; it++) {
         const double Tii = 2.0 * eta * Eii;
@@ -103,7 +103,7 @@ __device__ __forceinline__ bool local_ve(const creep_laws &L, bool on, double Ei
         Eii_exp = run ? e_exp : Eii_exp;
         Eii_lin = run ? e_lin : Eii_lin;
         const double r = Eii - (L.elastic ? 1.0 : 0.0) * Tii / (2.0 * L.eta_el) - (e_pwl + e_exp + e_lin + e_cst);
-        res = run ? fabs(r / Eii) : res;
+        res = fabs(r / Eii);
         run = run && !(res < stop);
         if (!__any(run)) break;
         double dfdeta = 0.0;
@@ -116,7 +116,7 @@ __device__ __forceinline__ bool local_ve(const creep_laws &L, bool on, double Ei
         const double next = eta - r / dfdeta;
         eta = run ? next : eta;
     }
-    return !on || !(res > tol);
+    return !run || !(res > tol);
 }
 
 // Failure codes of viscosity_concise, or-ed into the caller's flag.

@@ -9,8 +9,10 @@
 // bounded by FP64 issue rather than by its ~20 doubles of traffic per node:
 // factors that no node changes come with the phase table, exponents 1, 2 and 3
 // are products, and factors that are exactly 1 are not raised to a power.
-// 62 -> 34 us at 1023 x 255 centres with dislocation, diffusion and Peierls
-// creep, 145 -> 79 us at 1023^2 with two visco-elasto-plastic phases.
+// 62 -> 36 us at 1023 x 255 centres with dislocation, diffusion and Peierls
+// creep, 145 -> 81 us at 1023^2 with two visco-elasto-plastic phases.  The launch
+// bounds ask for three waves per SIMD (the creep kernel's 171 registers would
+// leave two: 40 us).
 #include "mdg_internal.h"
 
 #include "rheo_device.h"
@@ -25,7 +27,7 @@ using rheo::viscosity_concise;
 namespace {
 
 template <bool EXT>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 3)
 k_viscosity_grid(rheo_ctl md, const rheo_phase *__restrict__ phases, int n,
                  const signed char *__restrict__ tag, int centroid, mdg_rheo_nodes f,
                  int *__restrict__ fail) {
