@@ -46,6 +46,7 @@ typedef unsigned short bf16_t;
 namespace {
 
 constexpr int NL = 7;
+constexpr int NG = 8;             // gradient buffers
 constexpr int L_CIN[NL] = {4, 32, 32, 64, 64, 32, 32};
 constexpr int L_COUT[NL] = {32, 32, 64, 64, 32, 32, 3};
 constexpr int L_LEVEL[NL] = {0, 1, 2, 3, 2, 1, 0};
@@ -606,11 +607,11 @@ int ensure_buffers(mdg_ctx *c, pcnet_state *s, int H, int W) {
     }
     HIPCHK(c, s->act.reserve(off));
     HIPCHK(c, hipMemsetAsync(s->act.p, 0, off * sizeof(bf16_t), c->stream));
-    // gradient buffers: 0 dy (lev0, 4), 1 ds0/de0 (lev0, 32), 2 dz (lev0 32), 3 de1 (lev1 32),
-    // 4 dz1 (lev1 32), 5 de2 (lev2 64), 6 dz2 (lev2 64), 7 dz3 (lev3 64), 8 dp (lev0..2 scratch, 64)
-    const int glev[9] = {0, 0, 0, 1, 1, 2, 2, 3, 0}, gc[9] = {4, 32, 32, 32, 32, 64, 64, 64, 64};
+    // gradient buffers: 0 dy (lev0, 4), 1 ds0/de0 (lev0, 32), 2 de1 (lev1 32), 3 dz1 (lev1 32),
+    // 4 de2 (lev2 64), 5 dz2 (lev2 64), 6 dz3 (lev3 64), 7 dp (lev0..2 scratch, 64)
+    const int glev[NG] = {0, 0, 1, 1, 2, 2, 3, 0}, gc[NG] = {4, 32, 32, 32, 64, 64, 64, 64};
     long go = 0;
-    for (int i = 0; i < 9; i++) {
+    for (int i = 0; i < NG; i++) {
         s->goff[i] = go;
         go += (long)(H >> glev[i]) * (W >> glev[i]) * gc[i];
     }
@@ -752,8 +753,8 @@ int forward(mdg_ctx *c, pcnet_state *s) {
 
 int backward(mdg_ctx *c, pcnet_state *s, int accumulate) {
     const int H = s->H, W = s->W;
-    float *dy = Gb(s, 0), *de0 = Gb(s, 1), *de1 = Gb(s, 3), *dz1 = Gb(s, 4);
-    float *de2 = Gb(s, 5), *dz2 = Gb(s, 6), *dz3 = Gb(s, 7), *dp = Gb(s, 8);
+    float *dy = Gb(s, 0), *de0 = Gb(s, 1), *de1 = Gb(s, 2), *dz1 = Gb(s, 3);
+    float *de2 = Gb(s, 4), *dz2 = Gb(s, 5), *dz3 = Gb(s, 6), *dp = Gb(s, 7);
     // layer 6 (level 0): ds0 -> de0
     conv_bwd_weights(c, s, 6, A(s, A_S0), dy, accumulate);
     conv_bwd_data(c, s, 6, dy, de0);
