@@ -389,7 +389,10 @@ typedef struct {
                               as kspgcr counts them (Solvers.c:208-211)       */
     double smoother_ms;    /* graphs = 2: mean duration of the fine-level
                               smoother steps (k_cheb3; k_pcheb with smoother
-                              3) in this solve                                */
+                              3) in this solve; with graphs 0 and 1 the finest
+                              level runs these kernels only in FP64 with
+                              patches beyond 2M positions and in FP32 with
+                              the diagonal, several steps per launch else     */
     int    smoother_launches;
     /* input: smoothers 2 and 3 use vertex patches on the finest patch_levels
      * levels and the diagonal below them (0: every level, the default; the
@@ -626,12 +629,11 @@ int mdg_pcnet_train(mdg_ctx *ctx, int steps, int batch, float lr, unsigned long 
 int mdg_pcnet_train_residual(mdg_ctx *ctx, int steps, int batch, float lr, unsigned long long seed,
                              double *losses);
 
-/* Times the dominant kernel of the solve: the fine-level fused Chebyshev
- * smoother step (FP64) of the last FP64 solve (the vertex-patch step when
- * that solve used smoother 3, the Jacobi step otherwise), averaged over reps
- * launches with HIP events on the context stream.  Returns ms per launch and
- * the algorithmic (compulsory) bytes per launch.  No counterpart in the
- * reference; it feeds the roofline figure of the benchmark. */
+/* Times the single fine-level fused Chebyshev smoother step (FP64) of the last
+ * FP64 solve (the vertex-patch step when that solve used smoother 3, the Jacobi
+ * step otherwise), averaged over reps launches with HIP events on the context
+ * stream.  Returns ms per launch and the algorithmic (compulsory) bytes per
+ * launch.  No counterpart in the reference; it feeds the roofline figure of the benchmark. */
 int mdg_time_smoother(mdg_ctx *ctx, int reps, double *ms_per_launch, double *bytes_per_launch);
 
 /* Time of the last timed call (P2G kernel, G2P and advection kernels,

@@ -953,9 +953,10 @@ __global__ void __launch_bounds__(256) k_dense_solve(int n, const int *__restric
 // same region (one more position of halo), and the start of the second
 // smoothing call adds the coarse correction while it reads x.
 // Bound: three barriers and the LDS round trips of a step (0.9 us in FP64, 0.5
-// in FP32) after a start of 5 us; multi_steps has the times per step.  The
-// 101^2 solve went from 51.2 to 42.9 ms with it, of 383^2 (FP64, patches) from
-// 327 to 176 ms, of 767^2 (mixed) from 860 to 459 ms.
+// in FP32) after a start of 5 us; multi_steps has the times per step.  A CG
+// iteration (V-cycle included, k_small_cycle in place) with one step per launch
+// and with this kernel, on one card: 101^2 0.28 and 0.225 ms, 383^2 (FP64,
+// patches) 0.81 and 0.43, 767^2 (FP32 V-cycle) 1.10 and 0.52.
 #define CM_R 32            // region side
 #define CM_W (CM_R + 2)    // LDS row, one cell of padding on each side
 #define CM_MAX 8           // steps a launch at most
@@ -1113,9 +1114,10 @@ __global__ void __launch_bounds__(CM_R *CM_R) k_cheb_multi(sgrid g, stc<T> cf, T
 // jump of 1e6) gains iterations.
 // Bound: LDS reads (ten neighbours per position and step) and the barriers,
 // about 0.4 us a step on 26^2.  The levels below 47^2 of a 383^2 hierarchy take
-// 46 us per V-cycle in it where their kernels took 110 us; the solve of the
-// 101^2 inclusion went from 75.4 to 55.4 ms, of 383^2 ellipses (FP64, patches)
-// from 400 to 364 ms, of 767^2 (mixed) from 734 to 659 ms.  The limit of 1024
+// 46 us per V-cycle in it where their kernels took 110 us.  A CG iteration
+// (k_cheb_multi in place above these levels) with kernels of their own and with
+// this one, on one card: 101^2 0.265 and 0.225 ms, 383^2 (FP64, patches) 0.465
+// and 0.43, 767^2 (FP32 V-cycle) 0.565 and 0.525.  The limit of 1024
 // positions is one per thread; 47^2 in here would cost its 24 steps 3 x 0.4 us
 // and the LDS of FP64 lines, about what its own launches cost.
 #define SM_POS 1024
@@ -1850,7 +1852,10 @@ static void cheb_table(double lmax, double div, int deg, std::vector<double> &ab
 // the 1023^2 solve is 9% faster with them (FP32: 2.44 against 3.2 at 2047^2).
 // Jacobi, FP64, whole solves in ms, k_cheb3 against 2, 3, 4, 5, 6 a launch:
 // 101^2 52 | 53 48 44 45 43, 255^2 133 | 124 108 91 92 84, 511^2 263 | 242 209
-// 176 177 163.  An FP32 Jacobi hierarchy keeps single steps: it is there that
+// 176 177 163.  Larger ones, by 0, 2, 3, 4, 6 a launch: 1023^2 2332 | 2287 2199
+// 2130 2129, 2047^2 16676 | 16403 14979 14023 14141 (2.56 | 2.60 2.38 2.22 2.24
+// ms per CG iteration): a Jacobi step's halo is half a patch step's, so no size
+// goes back to single steps.  An FP32 Jacobi hierarchy keeps single steps: it is there that
 // a viscosity jump of 1e6 leaves CG at the limit of FP32, and the solve's
 // iterations depend on the last bits.
 template <typename T>
@@ -3139,12 +3144,15 @@ extern "C" int mdg_killer_solver(mdg_ctx *c, mdg_solver_opts *o, const double *D
     return rc;
 }
 
-// Times the dominant kernel of the solve (the fine-level fused Chebyshev
-// smoother step x_{k+1} = x_k + a (x_k - x_{k-1}) + c D^-1 (b - A_g x_k),
+// Times the single fine-level step of the smoother (the fused Chebyshev
+// step x_{k+1} = x_k + a (x_k - x_{k-1}) + c D^-1 (b - A_g x_k),
 // FP64) on the hierarchy of the last FP64 solve, reps launches between HIP
 // events on the context stream.  Returns ms per launch and the algorithmic
 // bytes per launch: x_k, x_{k-1} and b read, x_{k+1} written (8 B each per
-// velocity face), eta_n and eta_s read once (8 B per cell and per vertex).
+// velocity face), eta_n and eta_s read once (8 B per cell and per vertex).  It
+// is the kernel that dominates a solve with patches beyond multi_steps' 2M
+// positions, such as 2047^2; smaller ones and those with the diagonal run
+// k_cheb_multi on the finest level instead.
 extern "C" int mdg_time_smoother(mdg_ctx *c, int reps, double *ms, double *bytes) {
     if (!c || !ms || !bytes || reps < 1) return mdg_fail(c, MDG_ERR_ARG, "bad argument");
     if (!c->solver || c->solver->hd.L.empty()) return mdg_fail(c, MDG_ERR_STATE, "no FP64 solve has run");
